@@ -302,15 +302,20 @@ __global__ __launch_bounds__(64 * TAP_WAVES, 1) void ta_proj_kernel(
 // the workgroup's fp32 bias tile [128 q][64 k], the four rows' K [64 k][32 d] and V^T
 // [32 d][64 k] tiles and their mask entries move global -> LDS by DMA (buffer loads straight to
 // LDS, no VGPR staging) through a 2-deep ring, one barrier per step.  Scores S'^T[key][query]
-// come out of three MFMAs per 32x32 tile:
+// come out of two or three MFMAs per 32x32 tile:
 //     bias^T (fp32, the accumulator's start value, read from LDS in accumulator order)
 //     + K.Q^T (2)  +  [1, mask[key]] . [-m[q], 1]^T (1: two used k-slots)
 // so the bias, the key mask and the reference max cost no VALU and the bias is not rounded;
-// the softmax is exp2, an fp16 pair pack and v_dot2 row sums.  The reference max m[q] is kept
-// as an op_t value (exact as an MFMA operand) and moves lazily: at a head's first tile, while a
-// query has seen no unmasked key, or when a tile's row sum exceeds 2^14 (some P above 2^9).  A P
-// that would overflow op_t fails the same test before it reaches the P.V MFMA, and the tile is
-// then repacked from S' with the new reference.  A wave's two key halves of a step are processed
+// the softmax is exp2, an fp16 pair pack and v_dot2 row sums.  The third MFMA is left out while
+// it would add zeros: the reference of every query of the wave is 0 and the tile lies before the
+// row's first masked or padded key (masks are mostly tails).  The reference m[q] is kept as an
+// op_t value (exact as an MFMA operand).  It starts at 0, which a head's first tile accepts when
+// every lane's row sum is at least LSTEP_MIN, and moves lazily: to the first tile's maximum when
+// 0 is not accepted, while a query has seen no unmasked key, or when a tile's row sum exceeds
+// 2^14 (some P above 2^9).  A P that would overflow op_t fails the same test before it reaches
+// the P.V MFMA, and the tile is then repacked from S' with the new reference.  (Against a third
+// MFMA in every tile and a reference that always moved at the first: N = 1024 1083 -> 1051 us a
+// launch, 4 x N = 256 108 -> 105 us.)  A wave's two key halves of a step are processed
 // one after the other (so a tile's scores always use the reference the previous tile left);
 // four waves per SIMD (about 100 VGPRs each) hide each other's MFMA and LDS latencies.
 // Rows whose valid keys are all masked: the fp32 reference adds -1e9 to every logit,
@@ -330,6 +335,10 @@ constexpr int TS_V = 98304, TV_STAGE = 16384;
 constexpr int TS_MASK = 131072, TM_STAGE = 1024;
 constexpr size_t TA_LDS = (size_t)TS_MASK + 2 * TM_STAGE;
 constexpr float LSTEP_MAX = 16384.f;   // per-lane row sum of one tile that forces a rescale
+// A lane's row sum (16 keys) of a head's first tile from which on 0 serves as the reference: the
+// larger P are then at least 2^-10, far inside op_t's normal range, and what the P below it lose
+// (2^-25 each in fp16) is below the rounding of the larger ones.
+constexpr float LSTEP_MIN = 1.f / 64.f;
 
 // 16-byte chunk swizzles: rows of 8 chunks (V^T) and of 4 chunks (K).  A fragment read takes
 // one chunk from each of 32 consecutive rows; any 16 consecutive rows land in 16 distinct
@@ -455,13 +464,22 @@ __global__ __launch_bounds__(64 * TA_WAVES, 1) void ta_attn_kernel(
   asm volatile("" : "+v"(aK[0]), "+v"(aK[1]), "+v"(aM));
 
   issue(0, h0, 0);   // the first stage's DMA overlaps the scan below
-  // rows whose valid keys are all masked (wave-uniform)
+  // rows whose valid keys are all masked, and the row's first key with a nonzero mask term (masked
+  // or padding; N when there is none): tiles of keys before it need no mask (both wave-uniform)
   bool live_l = false;
+  int dirty_l = N;
   {
     const op_t* mr = mask16 + ((long)b * N + ip) * N;
-    for (int k = lane; k < n_valid; k += 64) live_l |= (float)mr[k] != -INFINITY;
+    for (int k = lane; k < N; k += 64) {
+      const float mv = (float)mr[k];
+      live_l |= k < n_valid && mv != -INFINITY;
+      if (mv != 0.f) dirty_l = min(dirty_l, k);
+    }
   }
   const bool live = __ballot(live_l) != 0;
+#pragma unroll
+  for (int sh = 32; sh >= 1; sh >>= 1) dirty_l = min(dirty_l, __shfl_xor(dirty_l, sh));
+  const int first_dirty = __builtin_amdgcn_readfirstlane(dirty_l);
 
   const uint32_t ONE = half_bits((op_t)1.f);
   const uint32_t lo_half = h ? 0u : ~0u;   // keeps a value in lanes 0-31, zero in 32-63
@@ -480,6 +498,7 @@ __global__ __launch_bounds__(64 * TA_WAVES, 1) void ta_attn_kernel(
   f32x16 o;
   float mh, lsum;
   uint64_t mset;   // lane mask: the queries (lanes) that have a reference maximum
+  bool useref;     // some query's reference is nonzero (wave-uniform)
   auto q_fetch = [&](int hd) PF_INLINE {
     const int jq = min(jq0, N - 32);
     const op_t* qptr = Q + ((((long)b * N + ip) * H + hd) * N + jq + m) * D + 8 * h;
@@ -491,6 +510,7 @@ __global__ __launch_bounds__(64 * TA_WAVES, 1) void ta_attn_kernel(
     lsum = 0.f;
     mh = 0.f;
     mset = 0;
+    useref = false;
     set_fb(0.f);
   };
   // P = exp2(S') packed into the two P.V operands; returns the lane's row sum
@@ -513,14 +533,10 @@ __global__ __launch_bounds__(64 * TA_WAVES, 1) void ta_attn_kernel(
   // against the current reference, one check, and the two P.V MFMAs.  When the check fails (no
   // reference yet -- every head's first tile -- or a tile row sum above LSTEP_MAX) the reference
   // moves to the tile's maximum first; the next tile's scores already use the new reference.
-  auto step2 = [&](auto stg) PF_INLINE {
+  auto step2 = [&](auto stg, int kb0) PF_INLINE {
     constexpr int STG = decltype(stg)::value;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      // every lane reads its key's mask entry (an in-bounds address for all lanes; half 1
-      // discards it) together with the tile's other reads: a read inside an h == 0 branch
-      // would get an LDS wait of its own ahead of them
-      const uint32_t mk = lds_rd16(aM + STG * TM_STAGE + 64 * u);
       f32x16 sc;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
@@ -537,15 +553,24 @@ __global__ __launch_bounds__(64 * TA_WAVES, 1) void ta_attn_kernel(
       __builtin_amdgcn_s_setprio(2);
       sc = mfma32(k0, qf[0], sc);
       sc = mfma32(k1, qf[1], sc);
-      ra[0] = (ONE | mk << 16) & lo_half;
-      asm volatile("" : "+v"(ra));
-      sc = mfma32(as_x8(ra), as_x8(fb), sc);
+      if (useref || kb0 + 32 * u + 32 > first_dirty) {
+        // every lane reads its key's mask entry (an in-bounds address for all lanes; half 1
+        // discards it)
+        ra[0] = (ONE | lds_rd16(aM + STG * TM_STAGE + 64 * u) << 16) & lo_half;
+        asm volatile("" : "+v"(ra));
+        sc = mfma32(as_x8(ra), as_x8(fb), sc);
+      }
       __builtin_amdgcn_s_setprio(0);
       u32x4 pf[2];
       float l = exp_pack(sc, pf);
       // the lane masks come straight from v_cmp (a bool ballot would materialize and re-test
       // each lane's predicate); every lane is active here (a live row's valid query block)
-      if ((__builtin_amdgcn_fcmpf(l, LSTEP_MAX, 2 /* ordered > */) | ~mset) != 0) {
+      uint64_t bad = __builtin_amdgcn_fcmpf(l, LSTEP_MAX, 2 /* ordered > */);
+      if (~mset != 0) {   // a head's first tile (or no unmasked key yet): 0 will do as the reference
+        bad |= ~mset & __builtin_amdgcn_fcmpf(l, LSTEP_MIN, 12 /* unordered or < */);
+        if (bad == 0) mset = ~0ull;
+      }
+      if (bad != 0) {
         float mx = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[r]);
@@ -563,6 +588,7 @@ __global__ __launch_bounds__(64 * TA_WAVES, 1) void ta_attn_kernel(
         l = exp_pack(sc, pf);
         mset |= __builtin_amdgcn_fcmpf(mx, -INFINITY, 14 /* unordered or != */);
         mh = mnew;
+        useref = __builtin_amdgcn_fcmpf(mnew, 0.f, 14 /* unordered or != */) != 0;
         set_fb(mnew);
       }
       lsum += l;
@@ -610,7 +636,7 @@ __global__ __launch_bounds__(64 * TA_WAVES, 1) void ta_attn_kernel(
         qf[1] = qn[1];
       }
       if (kbi == nKB - 1 && hd + 1 < h0 + nh) q_fetch(hd + 1);   // lands by the next step's wait
-      step2(stg);
+      step2(stg, 64 * kbi);
       if (kbi == nKB - 1) finalize(hd);
     }
     if (++kbi == nKB) {
