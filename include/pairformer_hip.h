@@ -91,7 +91,9 @@ typedef struct pf_trimul_args {
    * also the residuals p_in_lo, g_in_lo, g_out_lo (W - W16 in the operand type) and B == 1,
    * the mean correction: each of those rows' offsets also gets W_lo . (norm_in.weight * mu),
    * mu = the mean over positions of the normalized z (estimated from up to 32768 sampled
-   * positions): the part of a 16-bit weight's rounding error that every position shares. */
+   * positions): the part of a 16-bit weight's rounding error that every position shares.  With
+   * p_out_lo given as well, small grids (N <= 256 on 256 CUs) multiply by those residuals too
+   * instead: the whole rounding error, and no statistics pass. */
   const float* in_offsets;
   const void* p_in_lo; const void* g_in_lo; const void* g_out_lo;
 } pf_trimul_args;

@@ -7,8 +7,8 @@ import pytest
 import torch
 
 from oracle import pairformer_ref as ref
-from tt_boltz_amd import ops
-from test_gpu_parity import check
+from tt_boltz_amd import ops, pairformer
+from test_gpu_parity import _inputs, _sub_w, check
 
 pytestmark = pytest.mark.gpu
 
@@ -36,3 +36,44 @@ def test_attention_reference_and_mask_tiles(gpu, shift, first_masked):
     want = ref.triangle_attention_core(q, k, v, bias, mask, D ** -0.5)
     got = ops.triangle_attention(q.to(gpu), k.to(gpu), v.to(gpu), bias.to(gpu), mask.to(gpu))
     check(f"attention shift={shift} first_masked={first_masked}", got, want)
+
+
+# ------------------------------------------------------------------------------ trimul
+@pytest.mark.parametrize("B,N", [(1, 64), (1, 192), (1, 256), (1, 320), (2, 64), (2, 320)])
+@pytest.mark.parametrize("incoming", [False, True])
+@pytest.mark.parametrize("plain", [False, True])
+def test_trimul_direct(gpu, B, N, incoming, plain):
+    """The register-weight kernels with one group of 64 positions per workgroup and with several,
+    on both sides of the line between the residual MFMA and the mean correction (N = 256 / 320),
+    with plain weights, for a batch, and with the three ways of adding the residual."""
+    w = _sub_w(5, "tri_mul_in" if incoming else "tri_mul_out")
+    z = torch.cat([_inputs(N, 5 + b)[1] for b in range(B)])
+    pm = torch.cat([_inputs(N, 5 + b, pad_tail=7, rand_mask=True)[3] for b in range(B)])
+    opt = pairformer.Options(weight_residuals=not plain, mean_correction=not plain)
+    mod = pairformer.TriangleMultiplication(incoming, w, opt)
+    want = ref.triangle_multiplication(z.to(gpu), pm.to(gpu), {k: v.to(gpu) for k, v in w.items()},
+                                       "incoming" if incoming else "outgoing")
+    zd, pd = z.to(gpu), pm.to(gpu).contiguous()
+    update = mod(zd, pd)
+    check("trimul update", update, want)
+    other = torch.ones_like(zd)
+    check("trimul out += update", mod(zd, pd, out=other, accumulate=True) - 1.0, want)
+    inplace = zd.clone()
+    mod(inplace, pd, out=inplace, accumulate=True)
+    # the same update added to z: one fp32 rounding of the sum apart
+    assert (inplace - (zd + update)).abs().max() <= 2.0 ** -22 * (zd.abs().max() + update.abs().max())
+
+
+@pytest.mark.parametrize("B,N", [(1, 64), (2, 128), (3, 128), (1, 192)])
+def test_trimul_c64_direct_line(gpu, B, N):
+    """c_z = 64 on both sides of the line between the direct and the persistent kernels (512 groups
+    of 64 positions on 256 CUs)."""
+    from tt_boltz_amd import synthetic
+    w = ref.sub(synthetic.draw({k: v for k, v in synthetic.layer_shapes(64).items() if k.startswith("tri_mul_out.")},
+                               6), "tri_mul_out")
+    g = torch.Generator().manual_seed(N + B)
+    z = torch.randn((B, N, N, 64), generator=g)
+    pm = (torch.rand((B, N, N), generator=g) > 0.1).float()
+    want = ref.triangle_multiplication(z, pm, w, "outgoing")
+    got = pairformer.TriangleMultiplication(False, w)(z.to(gpu), pm.to(gpu))
+    check(f"trimul c64 B={B} N={N}", got, want)

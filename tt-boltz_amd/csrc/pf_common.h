@@ -311,7 +311,12 @@ constexpr float X_LOAD_SCALE = 256.f;
 PF_DEV float planes_amax(const float* __restrict__ parts, int nparts) {
   const int lane = threadIdx.x & 63;
   float mx = 0.f;
-  for (int i = lane; i < nparts; i += 64) mx = fmaxf(mx, parts[i]);
+  for (int i0 = lane; i0 < nparts; i0 += 256) {   // four loads in flight
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = i0 + 64 * k < nparts ? parts[i0 + 64 * k] : 0.f;
+    mx = fmaxf(fmaxf(mx, fmaxf(v[0], v[1])), fmaxf(v[2], v[3]));
+  }
   return wave_max(mx);
 }
 PF_DEV float x_store_scale(float amax, int K) {

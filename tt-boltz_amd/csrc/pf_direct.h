@@ -1,0 +1,119 @@
+// Device helpers of the "direct" pair kernels.
+//
+// A workgroup (one per CU, 8 waves at c_z = 128) walks groups of 64 consecutive positions.  The
+// output channels are split over its waves, and each wave keeps its own 32-channel blocks of the
+// weights in registers as MFMA fragments for the whole launch; the workgroup normalizes a group's
+// positions into LDS once, fully coalesced, and every wave reads its activation fragments from
+// there.  Against weights resident in LDS with one wave per 32-position tile (the form these
+// kernels replaced: 128 KB staged per workgroup, every tile re-reading all of it, LayerNorms on
+// rows strided over lanes) the set-up falls from ~14 to ~6 us, small grids use four times as many
+// CUs, and LDS reads per output fall to a quarter.  Whole trimul, us: N = 64 49 -> 25, N = 128
+// 56 -> 34, N = 512 230 -> 206, N = 1024 968 -> 839.
+#pragma once
+#include "pf_common.h"
+
+namespace {
+
+constexpr int DP_ROWS = 64;   // positions of a workgroup
+
+// LayerNorm (without beta) of DP_ROWS rows of CC channels by NW waves into LDS rows of CC + 8
+// op_t: wave wid takes 64 / NW rows, 16 lanes a row.  Loads and arithmetic are separate so that
+// a caller can issue its weight loads between them.
+template <int CC, int NW>
+struct DirectLn {
+  static constexpr int RPW = DP_ROWS / NW, IT = RPW / 4, NV = CC / 64;
+  f32x4 x[IT][NV], gm[NV];
+  template <class PairOf>
+  PF_DEV void load(const float* z, PairOf pair_of, int wid, int lane) {
+    const int g = lane >> 4, q = lane & 15;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const float* p = z + pair_of(wid * RPW + 4 * it + g) * CC + 4 * q;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) x[it][v] = *reinterpret_cast<const f32x4*>(p + 64 * v);
+    }
+  }
+  PF_DEV void load_gamma(const float* __restrict__ gamma, int lane) {   // null: none
+    const int q = lane & 15;
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+      gm[v] = gamma ? *reinterpret_cast<const f32x4*>(gamma + 64 * v + 4 * q) : f32x4{1.f, 1.f, 1.f, 1.f};
+  }
+  PF_DEV void store(op_t* dst, float eps, int wid, int lane) const {
+    const int g = lane >> 4, q = lane & 15;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      float s = 0.f;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) s += (x[it][v][0] + x[it][v][1]) + (x[it][v][2] + x[it][v][3]);
+      const float mean = row16_sum(s) * (1.f / CC);
+      float var = 0.f;
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { const float d = x[it][v][e] - mean; var += d * d; }
+      const float rstd = rsqrtf(row16_sum(var) * (1.f / CC) + eps);
+      op_t* row = dst + (wid * RPW + 4 * it + g) * (CC + 8) + 4 * q;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        opx4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (op_t)((x[it][v][e] - mean) * (rstd * gm[v][e]));
+        st_x4(row + 64 * v, o);
+      }
+    }
+  }
+};
+
+// The MFMA fragments of a wave's 32 weight rows (CC op_t each, contiguous at `rows`): loaded as
+// whole 1 KB runs (reading fragments straight from global memory would touch 32 cache lines an
+// instruction and cost twice the L1 time), then turned through the wave's own LDS buffer of
+// [32][CC + 8] op_t.  A wave's LDS accesses complete in order, so the buffer needs no barrier.
+template <int CC>
+struct DirectW {
+  opx8 v[CC / 16];
+  PF_DEV void load(const op_t* __restrict__ rows, int lane) {
+#pragma unroll
+    for (int i = 0; i < CC / 16; ++i) v[i] = ld_x8(rows + 8 * (lane + 64 * i));
+  }
+  PF_DEV void turn(op_t* buf, int lane) {   // -> v[s]: row lane & 31, k-step s
+#pragma unroll
+    for (int i = 0; i < CC / 16; ++i) {
+      const int c = lane + 64 * i;
+      st_x8(buf + (c / (CC / 8)) * (CC + 8) + 8 * (c % (CC / 8)), v[i]);
+    }
+#pragma unroll
+    for (int s = 0; s < CC / 16; ++s) v[s] = ld_x8(buf + (lane & 31) * (CC + 8) + 16 * s + 8 * (lane >> 5));
+  }
+};
+
+// How a direct kernel uses the rounding residuals of its weights: not at all, as a second MFMA per
+// fragment, or through the mean correction (pair_stats_kernel) in the rows' offsets.
+enum DirectLo { DL_NONE = 0, DL_MFMA = 1, DL_MEAN = 2 };
+
+// gm[c] (LDS, 128 floats) = gamma[c] * mu[c] of the statistics partials, by a workgroup of NT threads;
+// `scratch`: NT floats of LDS.  The caller synchronizes before reading gm.
+template <int NT>
+PF_DEV void direct_gmu(const float* __restrict__ stats, const float* __restrict__ gamma, float* gm, float* scratch) {
+  float pv[stats_per<NT>()];
+  stats_load<NT>(stats, pv);
+  const float g = gamma && threadIdx.x < PS_C ? gamma[threadIdx.x] : 1.f;
+  stats_reduce<NT>(pv, gm, scratch);
+  if (threadIdx.x < PS_C) gm[threadIdx.x] *= g;   // written by the same thread
+}
+
+// W row . beta in fp32 from the row's fragments (both lane halves get the sum).
+template <int KS>
+PF_DEV float direct_wbeta(const opx8 (&w)[KS], const float* beta, int h) {
+  float acc = 0.f;
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const f32x4 b0 = *reinterpret_cast<const f32x4*>(beta + 16 * s + 8 * h);
+    const f32x4 b1 = *reinterpret_cast<const f32x4*>(beta + 16 * s + 8 * h + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc += (float)w[s][e] * b0[e] + (float)w[s][4 + e] * b1[e];
+  }
+  return xor32_sum(acc);
+}
+
+}  // namespace

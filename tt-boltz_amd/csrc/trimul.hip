@@ -17,6 +17,7 @@
 //   tm_out      LN_out(X) -> p_out, LN_in(z) -> g_out (recomputed, so no gate tensor
 //               goes through HBM), update = p * sigmoid(g), residual into z.
 #include "pf_common.h"
+#include "pf_direct.h"
 #include "pf_internal.h"
 
 namespace {
@@ -43,8 +44,8 @@ PF_DEV void blk32_store(op_t* lds, int tid, const Blk32& r) {
 }
 
 // ---------------------------------------------------------------------------------
-// Input projection.  Persistent: one workgroup (8 waves, two per SIMD) per CU keeps p_in and
-// g_in ([2 CC][CC] each, op_t as given, so rounded once) resident in LDS, with the LayerNorm's
+// Input projection of large grids at c_z = 64 (the others: tm_proj_direct_kernel).  Persistent:
+// one workgroup (8 waves, two per SIMD) per CU keeps p_in and g_in ([2 CC][CC] each, op_t as given, so rounded once) resident in LDS, with the LayerNorm's
 // beta folded into fp32 offsets W beta added in the epilogue (gamma scales the normalized z
 // before its rounding to op_t).  Every wave walks tiles of 32
 // consecutive positions of one operand-plane row (orow, ocol0 .. ocol0+31) and loads the next
@@ -68,17 +69,13 @@ constexpr size_t tmp_lds() {
          (size_t)TMP_WAVES * 32 * SPITCH * sizeof(op_t) + TMP_WAVES * sizeof(float);
 }
 
-// offb (optional, fp32 [4 CC]): the exact W_p beta, W_g beta (else computed from the op_t
-// weights); with p_lo / g_lo (the weights' residuals) and the stats partials also the mean
-// correction (see pair_stats_kernel).
 template <int CC, bool MASK>
 __global__ __launch_bounds__(64 * TMP_WAVES, 1) void tm_proj_kernel(
     const float* __restrict__ z, const float* __restrict__ mask,
     const float* __restrict__ lnw, const float* __restrict__ lnb,
     const op_t* __restrict__ w_p, const op_t* __restrict__ w_g,
     op_t* __restrict__ opA, op_t* __restrict__ opB, float* __restrict__ amax_parts, int B, int N, int incoming,
-    float eps, const float* __restrict__ offb, const op_t* __restrict__ p_lo, const op_t* __restrict__ g_lo,
-    const float* __restrict__ stats) {
+    float eps) {
   constexpr int LW = CC + 8, KS = CC / 16;
   extern __shared__ __attribute__((aligned(16))) op_t wlds[];
   float* gam = reinterpret_cast<float*>(wlds);
@@ -89,49 +86,28 @@ __global__ __launch_bounds__(64 * TMP_WAVES, 1) void tm_proj_kernel(
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   op_t* stg = lg + 2 * CC * LW + wid * 32 * SPITCH;
   float* wave_amax = reinterpret_cast<float*>(lg + 2 * CC * LW + TMP_WAVES * 32 * SPITCH);
-  float* mu = reinterpret_cast<float*>(lg + 2 * CC * LW);   // the output stages, free until the tile loop
   constexpr int NT = 64 * TMP_WAVES;
   static_assert(4 * CC <= NT, "one offset row per thread");
-  const int orow = tid;   // this thread's offset row (W beta): 0 .. 4 CC - 1
-  opx8 rv[CC / 8];        // the row behind it: the residual (mean correction) or the weight
-  float offb_v = 0.f;
-  // set-up in two batches of global loads (each issued whole before its first use): the weights
-  // and partials, then, while the statistics reduce, the residual rows of the mean correction
-  const bool meanfix = offb && stats;
-  {
+  {   // set-up: every global load issued before its first use
     opx8 vp[stage_per<NT, 2 * CC, CC>()], vg[stage_per<NT, 2 * CC, CC>()];
     stage_load<NT, 2 * CC, CC>(w_p, vp);
     stage_load<NT, 2 * CC, CC>(w_g, vg);
     const float gv = tid < CC ? lnw[tid] : 0.f;
-    float pv[stats_per<NT>()];
-    if (meanfix) stats_load<NT>(stats, pv);
-    if (offb && orow < 4 * CC) offb_v = offb[orow];
     stage_store<NT, 2 * CC, CC>(lp, LW, vp);
     stage_store<NT, 2 * CC, CC>(lg, LW, vg);
     if (tid < CC) gam[tid] = gv;
-    if constexpr (CC == C)
-      if (meanfix && orow < 4 * CC) {
-        const op_t* lo = orow < 2 * CC ? p_lo + orow * CC : g_lo + (orow - 2 * CC) * CC;
-#pragma unroll
-        for (int c = 0; c < CC / 8; ++c) rv[c] = ld_x8(lo + 8 * c);
-      }
-    if (meanfix) stats_reduce<NT>(pv, mu, mu + PS_C);
   }
   __syncthreads();
-  if (orow < 4 * CC) {   // offsets W beta (one row per thread)
+  if (tid < 4 * CC) {   // offsets W beta (one row per thread), from the staged weights (rows 16-byte aligned)
     float acc = 0.f;
-    if (offb) {
-      if constexpr (CC == C) acc = corrected_offset_regs<true>(offb_v, rv, stats != nullptr, gam, mu);
-    } else {   // from the staged weights (rows 16-byte aligned)
-      const op_t* w = orow < 2 * CC ? lp + orow * LW : lg + (orow - 2 * CC) * LW;
+    const op_t* w = tid < 2 * CC ? lp + tid * LW : lg + (tid - 2 * CC) * LW;
 #pragma unroll
-      for (int c = 0; c < CC / 8; ++c) {
-        const opx8 w8 = ld_x8(w + 8 * c);
+    for (int c = 0; c < CC / 8; ++c) {
+      const opx8 w8 = ld_x8(w + 8 * c);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc += (float)w8[e] * lnb[8 * c + e];
-      }
+      for (int e = 0; e < 8; ++e) acc += (float)w8[e] * lnb[8 * c + e];
     }
-    cbias[orow] = orow < 2 * CC ? acc : -LOG2E * acc;
+    cbias[tid] = tid < 2 * CC ? acc : -LOG2E * acc;
   }
   __syncthreads();
   const uint32_t ntiles = (uint32_t)B * N * N / 32;
@@ -223,6 +199,135 @@ __global__ __launch_bounds__(64 * TMP_WAVES, 1) void tm_proj_kernel(
     float mx = wave_amax[0];
 #pragma unroll
     for (int w = 1; w < TMP_WAVES; ++w) mx = fmaxf(mx, wave_amax[w]);
+    amax_parts[blockIdx.x] = mx;
+  }
+}
+
+// Input projection (pf_direct.h): groups of 64 positions of one operand-plane row;
+// wave w owns the output channels 32 w .. 32 w + 31 of [a | b].  LO: the weights come with their
+// residuals.  offb: the exact W beta (else from the op_t weights).
+constexpr int TMDP = 72;   // output stage pitch (elements): 64 positions + 16 B
+template <int CC, bool MASK, int LO>
+__global__ __launch_bounds__(2 * 2 * CC, 1) void tm_proj_direct_kernel(
+    const float* __restrict__ z, const float* __restrict__ mask, const float* __restrict__ lnw,
+    const float* __restrict__ lnb, const op_t* __restrict__ w_p, const op_t* __restrict__ w_g,
+    const op_t* __restrict__ p_lo, const op_t* __restrict__ g_lo, const float* __restrict__ offb,
+    const float* __restrict__ stats,
+    op_t* __restrict__ opA, op_t* __restrict__ opB, float* __restrict__ amax_parts, int ngroups, int N, int incoming,
+    float eps) {
+  constexpr int NW = 2 * CC / 32, KS = CC / 16, LW = CC + 8;
+  __shared__ __attribute__((aligned(16))) op_t sx[2][DP_ROWS * LW];
+  __shared__ __attribute__((aligned(16))) op_t wbuf[NW][32 * (LW > TMDP ? LW : TMDP)];   // weights, then outputs
+  __shared__ __attribute__((aligned(16))) float smask[2][DP_ROWS];
+  __shared__ float wave_amax[NW];
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto group = [&](int g) PF_INLINE -> PosTile { return pos_tile(2u * g, N); };
+  auto pair_of = [&](const PosTile& pt, int c) PF_INLINE -> long {
+    return incoming ? ((long)pt.b * N + pt.c0 + c) * N + pt.r : ((long)pt.b * N + pt.r) * N + pt.c0 + c;
+  };
+  DirectLn<CC, NW> ln;
+  float mv = 1.f;
+  auto fetch = [&](int g) PF_INLINE {
+    const PosTile pt = group(g);
+    ln.load(z, [&](int c) PF_INLINE -> long { return pair_of(pt, c); }, wid, lane);
+    if (MASK && tid < DP_ROWS) mv = mask[pair_of(pt, tid)];
+  };
+  fetch(blockIdx.x);
+  ln.load_gamma(lnw, lane);
+  const int row = 32 * wid + m;
+  DirectW<CC> wp, wg, wpl, wgl;
+  wp.load(w_p + 32 * wid * CC, lane);
+  wg.load(w_g + 32 * wid * CC, lane);
+  if constexpr (LO != DL_NONE) {
+    wpl.load(p_lo + 32 * wid * CC, lane);
+    wgl.load(g_lo + 32 * wid * CC, lane);
+  }
+  float cp = 0.f, cg = 0.f;
+  if (offb) {
+    cp = offb[row];
+    cg = offb[2 * CC + row];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (LO == DL_MEAN) {
+    float* gm = reinterpret_cast<float*>(sx[1]);   // free until the second group
+    direct_gmu<64 * NW>(stats, lnw, gm, gm + PS_C);
+  }
+  ln.store(sx[0], eps, wid, lane);
+  if (MASK && tid < DP_ROWS) smask[0][tid] = mv;
+  op_t* stg = wbuf[wid];
+  wp.turn(stg, lane);
+  wg.turn(stg, lane);
+  if constexpr (LO != DL_NONE) {
+    wpl.turn(stg, lane);
+    wgl.turn(stg, lane);
+  }
+  if constexpr (LO == DL_MEAN) {
+    __syncthreads();
+    const float* gm = reinterpret_cast<const float*>(sx[1]);
+    cp += direct_wbeta<KS>(wpl.v, gm, h);
+    cg += direct_wbeta<KS>(wgl.v, gm, h);
+  }
+  if (!offb) {
+    cp = direct_wbeta<KS>(wp.v, lnb, h);
+    cg = direct_wbeta<KS>(wg.v, lnb, h);
+  }
+  cg *= -LOG2E;
+  float amax = 0.f;
+  int buf = 0;
+  for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x, buf ^= 1) {
+    if (gi != (int)blockIdx.x) {
+      ln.store(sx[buf], eps, wid, lane);
+      if (MASK && tid < DP_ROWS) smask[buf][tid] = mv;
+    }
+    __syncthreads();   // sx[buf] is whole; every wave is done with sx[buf ^ 1]
+    if (gi + (int)gridDim.x < ngroups) fetch(gi + gridDim.x);
+    f32x16 ap[2] = {zero16(), zero16()}, ag[2] = {zero16(), zero16()};
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const opx8 xf = ld_x8(sx[buf] + (32 * t + m) * LW + 16 * s + 8 * h);
+        ap[t] = mfma32(xf, wp.v[s], ap[t]);   // rows = position, cols = output channel
+        ag[t] = mfma32(xf, wg.v[s], ag[t]);
+        if constexpr (LO == DL_MFMA) {
+          ap[t] = mfma32(xf, wpl.v[s], ap[t]);
+          ag[t] = mfma32(xf, wgl.v[s], ag[t]);
+        }
+      }
+    // lane (channel m, half h) holds positions 8g + 4h + e of each tile: stage [channel][position]
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 mr = {1.f, 1.f, 1.f, 1.f};
+        if (MASK) mr = *reinterpret_cast<const f32x4*>(smask[buf] + 32 * t + 8 * g + 4 * h);
+        opx4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 4 * g + e;
+          float u = (ap[t][r] + cp) * rcp_fast(1.f + exp2_fast(fmaf(ag[t][r], -LOG2E, cg)));
+          if (MASK) u *= mr[e];
+          amax = fmaxf(amax, fabsf(u));
+          v[e] = (op_t)u;
+        }
+        st_x4(stg + m * TMDP + 32 * t + 8 * g + 4 * h, v);
+      }
+    const PosTile pt = group(gi);
+    op_t* dst = (wid < CC / 32 ? opA : opB) + (((long)pt.b * CC + 32 * (wid % (CC / 32))) * N + pt.r) * N + pt.c0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {   // eight lanes write a channel's 128 bytes
+      const int ch = 8 * q + (lane >> 3), chunk = lane & 7;
+      st_x8(dst + (long)ch * N * N + 8 * chunk, ld_x8(stg + ch * TMDP + 8 * chunk));
+    }
+  }
+  amax = fabsf((float)(op_t)wave_max(amax));
+  if (lane == 0) wave_amax[wid] = amax;
+  __syncthreads();
+  if (tid == 0) {
+    float mx = wave_amax[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) mx = fmaxf(mx, wave_amax[w]);
     amax_parts[blockIdx.x] = mx;
   }
 }
@@ -495,7 +600,8 @@ __global__ __launch_bounds__(64 * TMD_WAVES, 1) void tm_contract_dma_kernel(
 }
 
 // ---------------------------------------------------------------------------------
-// Output: z[i,j,:] (+)= p_out(LN_out(X[:,i,j])) * sigmoid(g_out(LN_in(z[i,j,:]))).
+// Output of large grids at c_z = 64 (the others: tm_out_direct_kernel):
+// z[i,j,:] (+)= p_out(LN_out(X[:,i,j])) * sigmoid(g_out(LN_in(z[i,j,:]))).
 // Persistent: one workgroup (8 waves) per CU keeps p_out / g_out in LDS (op_t as given, so
 // rounded once) with both LayerNorms' beta folded into fp32 offsets W beta, added to the
 // products (gamma scales the normalized values before their rounding to op_t); each wave walks
@@ -508,106 +614,65 @@ __global__ __launch_bounds__(64 * TMD_WAVES, 1) void tm_contract_dma_kernel(
 // ---------------------------------------------------------------------------------
 constexpr int TMO_WAVES = 8, XSP = 40;   // per-wave X stage: [CC channels][32 pairs + 8]
 // LDS: the offsets W_p beta_out [CC], -log2(e) W_g beta_in [CC] and gamma_out [CC], gamma_in [CC]
-// (fp32, first: small immediate offsets), then W_p, W_g [CC][CC + 4] op_t, (HILO) W_p's residual
-// in the same layout, then the per-wave X stages (HILO: half the channels, filled twice a tile)
-template <int CC, bool HILO = false>
+// (fp32, first: small immediate offsets), then W_p, W_g [CC][CC + 4] op_t, then the per-wave X stages
+template <int CC>
 constexpr size_t tmo_lds() {
-  return 4 * CC * sizeof(float) + (size_t)(HILO ? 3 : 2) * CC * (CC + 4) * sizeof(op_t) +
-         (size_t)TMO_WAVES * (HILO ? CC / 2 : CC) * XSP * sizeof(op_t);
+  return 4 * CC * sizeof(float) + (size_t)2 * CC * (CC + 4) * sizeof(op_t) + (size_t)TMO_WAVES * CC * XSP * sizeof(op_t);
 }
 
 // resid: 0 -> out = update; 1 -> out = z_in + update (out may alias z_in); 2 -> out += update
-// X is read back times x_scale, or, when nparts > 0, divided by the contraction's
-// x_store_scale of the operand maxima in amax_parts (contraction length N).
-// HILO: p_out comes with its rounding residual w_pout_lo = p_out - p_out16 (op_t) and the
-// output projection runs on both (two MFMAs per fragment: weights good to ~2^-22 of their size).
-template <typename XT, int CC, bool HILO = false>
+// X is read back divided by the contraction's x_store_scale of the operand maxima in amax_parts
+// (contraction length N).
+template <typename XT, int CC>
 __global__ __launch_bounds__(64 * TMO_WAVES, 1) void tm_out_kernel(
-    const XT* __restrict__ X, float x_scale, const float* __restrict__ amax_parts, int nparts,
+    const XT* __restrict__ X, const float* __restrict__ amax_parts, int nparts,
     const float* z_in, float* out,
     const float* __restrict__ lni_w, const float* __restrict__ lni_b,
     const float* __restrict__ lno_w, const float* __restrict__ lno_b,
-    const op_t* __restrict__ w_pout, const op_t* __restrict__ w_gout, const op_t* __restrict__ w_pout_lo,
-    int B, int N, int resid, float eps, const float* __restrict__ offb_g, const op_t* __restrict__ gout_lo,
-    const float* __restrict__ stats) {
+    const op_t* __restrict__ w_pout, const op_t* __restrict__ w_gout, int B, int N, int resid, float eps) {
   constexpr int LW = CC + 4, KS = CC / 16;
-  constexpr int XCH = HILO ? CC / 2 : CC;   // channels per X stage fill
   extern __shared__ __attribute__((aligned(16))) op_t olds[];
   float* cbias = reinterpret_cast<float*>(olds);   // [0, CC): p, [CC, 2 CC): g
   float* gam_o = cbias + 2 * CC;
   float* gam_i = gam_o + CC;
   op_t* sWp = olds + 4 * CC * 2;
   op_t* sWg = sWp + CC * LW;
-  op_t* sWpl = sWg + CC * LW;   // HILO only
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  XT* xs = reinterpret_cast<XT*>(sWg + (HILO ? 2 : 1) * CC * LW) + wid * XCH * XSP;   // this wave's X stage
+  XT* xs = reinterpret_cast<XT*>(sWg + CC * LW) + wid * CC * XSP;   // this wave's X stage
   // weights -> LDS (rows are 8-byte aligned: two 8-byte stores per 16-byte load), gamma, and
   // the offsets W beta (one row per thread)
-  float* mu = reinterpret_cast<float*>(xs - wid * XCH * XSP);   // the X stages, free until the tile loop
   constexpr int NT = 64 * TMO_WAVES;
   static_assert(2 * CC <= NT, "one offset row per thread");
-  const int orow = tid;                   // this thread's offset row: p (< CC) or g
-  const bool grow = orow >= CC, gfix = grow && offb_g != nullptr;
-  opx8 rv[CC / 8];                        // g rows with offb_g: the residual of g_out (mean correction)
-  float offb_v = 0.f;
-  // set-up in two batches of global loads (each issued whole before its first use): the weights
-  // and partials, then, while the statistics reduce, the residual rows of the mean correction
   {
-    const bool meanfix = offb_g && stats;
     opx8 vp[stage_per<NT, CC, CC>()], vg[stage_per<NT, CC, CC>()];
     stage_load<NT, CC, CC>(w_pout, vp);
     stage_load<NT, CC, CC>(w_gout, vg);
     const float go = tid < CC ? lno_w[tid] : 0.f, gi = tid < CC ? lni_w[tid] : 0.f;
-    float pv[stats_per<NT>()];
-    if (meanfix) stats_load<NT>(stats, pv);
-    if (orow < 2 * CC && gfix) offb_v = offb_g[orow - CC];
-    if constexpr (HILO) {
-      opx8 vl[stage_per<NT, CC, CC>()];
-      stage_load<NT, CC, CC>(w_pout_lo, vl);
-      stage_store<NT, CC, CC>(sWpl, LW, vl);
-    }
     stage_store<NT, CC, CC>(sWp, LW, vp);
     stage_store<NT, CC, CC>(sWg, LW, vg);
     if (tid < CC) {
       gam_o[tid] = go;
       gam_i[tid] = gi;
     }
-    if constexpr (CC == C)
-      if (orow < 2 * CC && gfix && stats) {
-#pragma unroll
-        for (int c = 0; c < CC / 8; ++c) rv[c] = ld_x8(gout_lo + (orow - CC) * CC + 8 * c);
-      }
-    if (meanfix) stats_reduce<NT>(pv, mu, mu + PS_C);
   }
   __syncthreads();
-  if (orow < 2 * CC) {
-    if (gfix) {   // gate offsets from the exact g_out beta (+ the mean correction)
-      if constexpr (CC == C) cbias[orow] = -LOG2E * corrected_offset_regs<true>(offb_v, rv, stats != nullptr, gam_i, mu);
-    } else {      // W beta from the staged 16-bit weights (p_out with its residual under HILO)
-      const op_t* w = grow ? sWg + (orow - CC) * LW : sWp + orow * LW;
-      const float* bet = grow ? lni_b : lno_b;
-      float acc = 0.f;
+  if (tid < 2 * CC) {   // W beta from the staged weights
+    const bool grow = tid >= CC;
+    const op_t* w = grow ? sWg + (tid - CC) * LW : sWp + tid * LW;
+    const float* bet = grow ? lni_b : lno_b;
+    float acc = 0.f;
 #pragma unroll
-      for (int c = 0; c < CC; c += 8) {
-        const opx4 wa = ld_x4(w + c), wb = ld_x4(w + c + 4);
-        const opx8 w8 = {wa[0], wa[1], wa[2], wa[3], wb[0], wb[1], wb[2], wb[3]};
+    for (int c = 0; c < CC; c += 8) {
+      const opx4 wa = ld_x4(w + c), wb = ld_x4(w + c + 4);
+      const opx8 w8 = {wa[0], wa[1], wa[2], wa[3], wb[0], wb[1], wb[2], wb[3]};
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc += (float)w8[e] * bet[c + e];
-        if constexpr (HILO) {
-          if (!grow) {
-            const opx4 la = ld_x4(sWpl + orow * LW + c), lb = ld_x4(sWpl + orow * LW + c + 4);
-            const opx8 l8 = {la[0], la[1], la[2], la[3], lb[0], lb[1], lb[2], lb[3]};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc += (float)l8[e] * bet[c + e];
-          }
-        }
-      }
-      cbias[orow] = grow ? -LOG2E * acc : acc;
+      for (int e = 0; e < 8; ++e) acc += (float)w8[e] * bet[c + e];
     }
+    cbias[tid] = grow ? -LOG2E * acc : acc;
   }
   __syncthreads();
-  if (nparts > 0) x_scale = 1.f / x_store_scale(planes_amax(amax_parts, nparts), N);   // a power of two
+  const float x_scale = 1.f / x_store_scale(planes_amax(amax_parts, nparts), N);   // a power of two
   const long NN = (long)N * N;
   const uint32_t ntiles = (uint32_t)B * N * N / 32;
   for (uint32_t t = blockIdx.x * TMO_WAVES + wid; t < ntiles; t += gridDim.x * TMO_WAVES) {
@@ -617,26 +682,19 @@ __global__ __launch_bounds__(64 * TMO_WAVES, 1) void tm_out_kernel(
     const long pair = p0 + m;
     opx8 xo[KS], xi[KS];
     {
-      // X[b][ch][q0 .. q0+31]: 16-byte chunk c -> channel c >> 2, pairs 8*(c & 3) ..; with HILO
-      // in two fills of CC/2 channels (chunks q < CC/16 of the output-aligned order are
-      // channels < CC/2).  A wave's LDS accesses complete in order, so the second fill does not
-      // overtake the first one's reads.
+      // X[b][ch][q0 .. q0+31]: 16-byte chunk c -> channel c >> 2, pairs 8*(c & 3) ..  (a wave's
+      // LDS accesses complete in order)
       const XT* src = X + (long)b * CC * NN + (p0 - (long)b * NN);
       float xv[CC / 2];
 #pragma unroll
-      for (int half = 0; half < CC / XCH; ++half) {
-#pragma unroll
-        for (int k = 0; k < XCH / 16; ++k) {
-          const int c = lane + 64 * k, ch = c >> 2, col = (c & 3) * 8;
-          *reinterpret_cast<opx8*>(xs + ch * XSP + col) =
-              *reinterpret_cast<const opx8*>(src + (long)(ch + half * XCH) * NN + col);
-        }
-#pragma unroll
-        for (int q = half * XCH / 8; q < (half + 1) * XCH / 8; ++q)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            xv[4 * q + e] = (float)xs[(oa_channel(q, h) - half * XCH + e) * XSP + m] * x_scale;
+      for (int k = 0; k < CC / 16; ++k) {
+        const int c = lane + 64 * k, ch = c >> 2, col = (c & 3) * 8;
+        *reinterpret_cast<opx8*>(xs + ch * XSP + col) = *reinterpret_cast<const opx8*>(src + (long)ch * NN + col);
       }
+#pragma unroll
+      for (int q = 0; q < CC / 8; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xv[4 * q + e] = (float)xs[(oa_channel(q, h) + e) * XSP + m] * x_scale;
       ln_oa_gamma_to_frag<CC>(xv, h, gam_o, eps, xo);
     }
     float zr[CC / 2];
@@ -651,11 +709,6 @@ __global__ __launch_bounds__(64 * TMO_WAVES, 1) void tm_out_kernel(
       for (int s = 0; s < KS; ++s) {
         P = mfma32(wfrag_oa(wp, s, h), xo[s], P);   // rows = output channel, cols = pair
         G = mfma32(wfrag_oa(wg, s, h), xi[s], G);
-      }
-      if constexpr (HILO) {
-        const op_t* wpl = &sWpl[(32 * ob + m) * LW];
-#pragma unroll
-        for (int s = 0; s < KS; ++s) P = mfma32(wfrag_oa(wpl, s, h), xo[s], P);
       }
       float* orow = out + pair * CC;
 #pragma unroll
@@ -675,6 +728,146 @@ __global__ __launch_bounds__(64 * TMO_WAVES, 1) void tm_out_kernel(
         }
         *reinterpret_cast<f32x4*>(dst) = v;
       }
+    }
+  }
+}
+
+// Output (pf_direct.h): groups of 64 consecutive pairs; wave w owns the output
+// channels 32 (w >> 1) .. + 31 of the pairs 32 (w & 1) .. + 31.  The LayerNorm of X over channels
+// goes through a [channel][pair] stage in LDS.  PLO / GLO: p_out / g_out come with their residuals.
+constexpr int TMDX = 72;   // X stage pitch (elements): 64 pairs + 16 B
+template <int CC>
+constexpr size_t tmod_lds() {
+  return (size_t)(CC * TMDX + 3 * DP_ROWS * (CC + 8) + (2 * CC / 32) * 32 * (CC + 8)) * sizeof(op_t) +
+         3 * CC * sizeof(float);
+}
+template <int CC, bool PLO, int GLO>
+__global__ __launch_bounds__(2 * 2 * CC, 1) void tm_out_direct_kernel(
+    const op_t* __restrict__ X, const float* __restrict__ amax_parts, int nparts, const float* z_in, float* out,
+    const float* __restrict__ lni_w, const float* __restrict__ lni_b, const float* __restrict__ lno_w,
+    const float* __restrict__ lno_b, const op_t* __restrict__ w_p, const op_t* __restrict__ w_g,
+    const op_t* __restrict__ p_lo, const op_t* __restrict__ g_lo, const float* __restrict__ offb_g,
+    const float* __restrict__ stats, int ngroups, int N,
+    int resid, float eps) {
+  constexpr int NW = 2 * CC / 32, KS = CC / 16, LW = CC + 8, NT = 64 * NW;
+  extern __shared__ __attribute__((aligned(16))) op_t odlds[];
+  float* soff = reinterpret_cast<float*>(odlds);   // W_p beta_out [CC], -log2(e) W_g beta_in [CC]
+  float* sgam = soff + 2 * CC;                     // gamma_out [CC]
+  op_t* sxs = odlds + 3 * CC * 2;                  // X stage [CC][TMDX]
+  op_t* sxo = sxs + CC * TMDX;                     // LN_out(X) [64][LW]
+  op_t* sxi = sxo + DP_ROWS * LW;                  // LN_in(z) [2][64][LW]
+  op_t* wbuf = sxi + 2 * DP_ROWS * LW;             // the waves' weight buffers [NW][32][LW]
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tile = wid & 1, ob = wid >> 1;
+  const long NN = (long)N * N;
+  opx8 xv[CC * 8 / NT];   // this thread's 16-byte chunks of the group's X slice
+  DirectLn<CC, NW> ln;
+  auto fetch = [&](int g) PF_INLINE {
+    const long p0 = (long)DP_ROWS * g;   // first pair b*NN + i*N + j
+    const long b = p0 / NN;
+    const op_t* src = X + b * CC * NN + (p0 - b * NN);
+#pragma unroll
+    for (int k = 0; k < CC * 8 / NT; ++k) {
+      const int c = tid + NT * k;
+      xv[k] = ld_x8(src + (long)(c >> 3) * NN + 8 * (c & 7));
+    }
+    ln.load(z_in, [&](int r) PF_INLINE -> long { return p0 + r; }, wid, lane);
+  };
+  fetch(blockIdx.x);
+  ln.load_gamma(lni_w, lane);
+  const int row = 32 * ob + m;
+  DirectW<CC> wp, wg, wpl, wgl;
+  wp.load(w_p + 32 * ob * CC, lane);
+  wg.load(w_g + 32 * ob * CC, lane);
+  if constexpr (PLO) wpl.load(p_lo + 32 * ob * CC, lane);
+  if constexpr (GLO != DL_NONE) wgl.load(g_lo + 32 * ob * CC, lane);
+  const float x_scale = 1.f / x_store_scale(planes_amax(amax_parts, nparts), N);   // a power of two
+  {
+    op_t* wb = wbuf + wid * 32 * LW;
+    wp.turn(wb, lane);
+    wg.turn(wb, lane);
+    if constexpr (PLO) wpl.turn(wb, lane);
+    if constexpr (GLO != DL_NONE) wgl.turn(wb, lane);
+    float cp = direct_wbeta<KS>(wp.v, lno_b, h);
+    if constexpr (PLO) cp += direct_wbeta<KS>(wpl.v, lno_b, h);
+    float cg = offb_g ? offb_g[row] : direct_wbeta<KS>(wg.v, lni_b, h);
+    if constexpr (GLO == DL_MEAN) {
+      float* gm = reinterpret_cast<float*>(sxo);   // free until the tile loop's first barrier
+      direct_gmu<NT>(stats, lni_w, gm, gm + PS_C);
+      __syncthreads();
+      cg += direct_wbeta<KS>(wgl.v, gm, h);
+    }
+    if (tile == 0 && h == 0) {
+      soff[row] = cp;
+      soff[CC + row] = -LOG2E * cg;
+    }
+    if (tid < CC) sgam[tid] = lno_w[tid];
+  }
+  int buf = 0;
+  for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x, buf ^= 1) {
+    const long p0 = (long)DP_ROWS * gi;
+    // (the X stage's readers of the last group are past its second barrier)
+#pragma unroll
+    for (int k = 0; k < CC * 8 / NT; ++k) {
+      const int c = tid + NT * k;
+      st_x8(sxs + (c >> 3) * TMDX + 8 * (c & 7), xv[k]);
+    }
+    op_t* sxib = sxi + buf * DP_ROWS * LW;
+    ln.store(sxib, eps, wid, lane);
+    // the residual in the accumulator's order (this wave alone writes these elements, below)
+    const float* rsrc = (resid == 2 ? out : z_in) + (p0 + 32 * tile + m) * CC + 32 * ob + 4 * h;
+    f32x4 res[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      res[g] = resid ? *reinterpret_cast<const f32x4*>(rsrc + 8 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();   // every z row of the group has been read (out may alias z_in)
+    if (gi + (int)gridDim.x < ngroups) fetch(gi + gridDim.x);
+    // LayerNorm of X over channels: a lane takes channels (lane >> 3) + 8 i of one pair
+    constexpr int RPW = DP_ROWS / NW;
+#pragma unroll
+    for (int it = 0; it < RPW / 8; ++it) {
+      const int pr = wid * RPW + 8 * it + (lane & 7), c0 = lane >> 3;
+      float v[CC / 8], s = 0.f, var = 0.f;
+#pragma unroll
+      for (int i = 0; i < CC / 8; ++i) {
+        v[i] = (float)sxs[(c0 + 8 * i) * TMDX + pr] * x_scale;
+        s += v[i];
+      }
+      s += __shfl_xor(s, 8);
+      s += __shfl_xor(s, 16);
+      const float mean = xor32_sum(s) * (1.f / CC);
+#pragma unroll
+      for (int i = 0; i < CC / 8; ++i) { const float d = v[i] - mean; var += d * d; }
+      var += __shfl_xor(var, 8);
+      var += __shfl_xor(var, 16);
+      const float rstd = rsqrtf(xor32_sum(var) * (1.f / CC) + eps);
+#pragma unroll
+      for (int i = 0; i < CC / 8; ++i) sxo[pr * LW + c0 + 8 * i] = (op_t)((v[i] - mean) * (rstd * sgam[c0 + 8 * i]));
+    }
+    __syncthreads();
+    f32x16 P = zero16(), G = zero16();
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const opx8 xo = ld_x8(sxo + (32 * tile + m) * LW + 16 * s + 8 * h);
+      const opx8 xi = ld_x8(sxib + (32 * tile + m) * LW + 16 * s + 8 * h);
+      P = mfma32(wp.v[s], xo, P);   // rows = output channel, cols = pair
+      G = mfma32(wg.v[s], xi, G);
+      if constexpr (PLO) P = mfma32(wpl.v[s], xo, P);
+      if constexpr (GLO == DL_MFMA) G = mfma32(wgl.v[s], xi, G);
+    }
+    float* dst = out + (p0 + 32 * tile + m) * CC + 32 * ob + 4 * h;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 op = *reinterpret_cast<const f32x4*>(soff + 32 * ob + 8 * g + 4 * h);
+      const f32x4 og = *reinterpret_cast<const f32x4*>(soff + CC + 32 * ob + 8 * g + 4 * h);
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float u = (P[4 * g + e] + op[e]) * rcp_fast(1.f + exp2_fast(fmaf(G[4 * g + e], -LOG2E, og[e])));
+        v[e] = res[g][e] + u;
+      }
+      *reinterpret_cast<f32x4*>(dst + 8 * g) = v;
     }
   }
 }
@@ -720,28 +913,42 @@ int launch_contract(const op_t* opA, const op_t* opB, OutT* X, int planes, int N
 // the PS_WG x 128 partial sums of the mean correction.
 constexpr int TM_MAX_PARTS = 1024;
 
-template <int CC>
-int trimul_run(const pf_trimul_args* a) {
+// The direct kernels (pf_direct.h) on at most `wgs` workgroups.
+template <int CC, int LO>
+int trimul_run_direct(const pf_trimul_args* a, op_t* opA, op_t* opB, op_t* X, float* amax_parts, const float* stats,
+                      int wgs) {
+  hipStream_t st = (hipStream_t)a->stream;
+  const int B = a->B, N = a->N, nt = 2 * 2 * CC, ngroups = (int)((long)B * N * N / DP_ROWS);
+  const int grid = min(ngroups, min(wgs, TM_MAX_PARTS));
+  const float* offb = CC == C ? a->in_offsets : nullptr;
+  {
+    auto kern = a->pair_mask ? tm_proj_direct_kernel<CC, true, LO> : tm_proj_direct_kernel<CC, false, LO>;
+    kern<<<grid, nt, 0, st>>>(a->z_in, a->pair_mask, a->norm_in_w, a->norm_in_b, (const op_t*)a->p_in_w,
+                              (const op_t*)a->g_in_w, (const op_t*)a->p_in_lo, (const op_t*)a->g_in_lo, offb, stats,
+                              opA, opB, amax_parts, ngroups, N, a->direction, a->eps);
+    PF_CHECK_LAUNCH("tm_proj_direct_kernel");
+  }
+  pf_kernel_mark(PF_TIMED_CONTRACT, st, 0);
+  const int rc = launch_contract<op_t>(opA, opB, X, B * CC, N, X_STORE_SCALE, st, amax_parts, grid);
+  pf_kernel_mark(PF_TIMED_CONTRACT, st, 1);
+  if (rc != PF_OK) return rc;
+  const int resid = !a->accumulate ? 0 : (a->out == a->z_in ? 1 : 2);
+  auto kern = CC == C && a->p_out_lo ? tm_out_direct_kernel<CC, CC == C, LO> : tm_out_direct_kernel<CC, false, LO>;
+  if (const int rc2 = pf_reserve_lds((const void*)kern, tmod_lds<CC>(), "tm_out_direct_kernel")) return rc2;
+  kern<<<grid, nt, tmod_lds<CC>(), st>>>(X, amax_parts, grid, a->z_in, a->out, a->norm_in_w, a->norm_in_b,
+                                         a->norm_out_w, a->norm_out_b, (const op_t*)a->p_out_w,
+                                         (const op_t*)a->g_out_w, (const op_t*)a->p_out_lo, (const op_t*)a->g_out_lo,
+                                         offb ? offb + 4 * CC : nullptr, stats, ngroups, N, resid, a->eps);
+  PF_CHECK_LAUNCH("tm_out_direct_kernel");
+  return PF_OK;
+}
+
+// The persistent kernels (c_z = 64).
+int trimul_run_persistent64(const pf_trimul_args* a, op_t* opA, op_t* opB, op_t* X, float* amax_parts, int cus) {
+  constexpr int CC = 64;
   hipStream_t st = (hipStream_t)a->stream;
   const int B = a->B, N = a->N;
-  const size_t planes = (size_t)B * CC * N * N;
-  op_t* opA = (op_t*)a->workspace;
-  op_t* opB = opA + planes;
-  op_t* X = opB + planes;
-  float* amax_parts = reinterpret_cast<float*>(X + planes);
-  float* stats = amax_parts + TM_MAX_PARTS;
-  // mean correction: exact beta offsets, the three residuals, one batch element (c_z = 128)
-  const bool meanfix = CC == C && B == 1 && a->in_offsets && a->p_in_lo && a->g_in_lo && a->g_out_lo;
-  if (meanfix) {
-    pair_stats_kernel<<<PS_WG, 64 * PS_WAVES, 0, st>>>(a->z_in, N, a->eps, stats);
-    PF_CHECK_LAUNCH("pair_stats_kernel");
-  } else {
-    stats = nullptr;
-  }
-  const float* offb = CC == C ? a->in_offsets : nullptr;
   const long positions = (long)B * N * N;
-  const int cus = device_cus();
-  if (cus <= 0) return pf_fail(PF_E_LAUNCH, "pf_trimul_fwd: cannot query the device");
   const int grid_proj = (int)min((long)min(cus, TM_MAX_PARTS), (positions / 32 + TMP_WAVES - 1) / TMP_WAVES);
   const int grid_out = (int)min((long)cus, (positions / 32 + TMO_WAVES - 1) / TMO_WAVES);
   {
@@ -749,39 +956,49 @@ int trimul_run(const pf_trimul_args* a) {
     if (const int rc = pf_reserve_lds((const void*)kern, tmp_lds<CC>(), "tm_proj_kernel")) return rc;
     kern<<<grid_proj, 64 * tmp_waves<CC>(), tmp_lds<CC>(), st>>>(
         a->z_in, a->pair_mask, a->norm_in_w, a->norm_in_b, (const op_t*)a->p_in_w, (const op_t*)a->g_in_w, opA, opB,
-        amax_parts, B, N, a->direction, a->eps, offb, (const op_t*)a->p_in_lo, (const op_t*)a->g_in_lo, stats);
+        amax_parts, B, N, a->direction, a->eps);
     PF_CHECK_LAUNCH("tm_proj_kernel");
   }
   pf_kernel_mark(PF_TIMED_CONTRACT, st, 0);
   const int rc = launch_contract<op_t>(opA, opB, X, B * CC, N, X_STORE_SCALE, st, amax_parts, grid_proj);
   pf_kernel_mark(PF_TIMED_CONTRACT, st, 1);
   if (rc != PF_OK) return rc;
-  {
-    const int resid = !a->accumulate ? 0 : (a->out == a->z_in ? 1 : 2);
-    bool hilo = false;
-    if constexpr (CC == 128) {   // the residual weights exist for c_z = 128
-      if (a->p_out_lo) {
-        hilo = true;
-        if (const int rc2 = pf_reserve_lds((const void*)tm_out_kernel<op_t, CC, true>, tmo_lds<CC, true>(),
-                                           "tm_out_kernel"))
-          return rc2;
-        tm_out_kernel<op_t, CC, true><<<grid_out, 64 * TMO_WAVES, tmo_lds<CC, true>(), st>>>(
-            X, X_LOAD_SCALE, amax_parts, grid_proj, a->z_in, a->out, a->norm_in_w, a->norm_in_b, a->norm_out_w,
-            a->norm_out_b, (const op_t*)a->p_out_w, (const op_t*)a->g_out_w, (const op_t*)a->p_out_lo, B, N, resid,
-            a->eps, offb ? offb + 4 * CC : nullptr, (const op_t*)a->g_out_lo, stats);
-      }
-    }
-    if (!hilo) {
-      if (const int rc2 = pf_reserve_lds((const void*)tm_out_kernel<op_t, CC>, tmo_lds<CC>(), "tm_out_kernel"))
-        return rc2;
-      tm_out_kernel<op_t, CC><<<grid_out, 64 * TMO_WAVES, tmo_lds<CC>(), st>>>(
-          X, X_LOAD_SCALE, amax_parts, grid_proj, a->z_in, a->out, a->norm_in_w, a->norm_in_b, a->norm_out_w,
-          a->norm_out_b, (const op_t*)a->p_out_w, (const op_t*)a->g_out_w, nullptr, B, N, resid, a->eps,
-          offb ? offb + 4 * CC : nullptr, (const op_t*)a->g_out_lo, stats);
-    }
-    PF_CHECK_LAUNCH("tm_out_kernel");
-  }
+  const int resid = !a->accumulate ? 0 : (a->out == a->z_in ? 1 : 2);
+  if (const int rc2 = pf_reserve_lds((const void*)tm_out_kernel<op_t, CC>, tmo_lds<CC>(), "tm_out_kernel")) return rc2;
+  tm_out_kernel<op_t, CC><<<grid_out, 64 * TMO_WAVES, tmo_lds<CC>(), st>>>(
+      X, amax_parts, grid_proj, a->z_in, a->out, a->norm_in_w, a->norm_in_b, a->norm_out_w, a->norm_out_b,
+      (const op_t*)a->p_out_w, (const op_t*)a->g_out_w, B, N, resid, a->eps);
+  PF_CHECK_LAUNCH("tm_out_kernel");
   return PF_OK;
+}
+
+// c_z = 128 runs on the direct kernels at every size; the residuals of p_in, g_in, g_out (one
+// batch element) enter as a second MFMA when all four residuals are given (the mean correction
+// without p_out's stays the mean correction) up to four groups per CU, where the statistics launch
+// costs more (whole trimul, us: N = 64 25 vs 33 with the mean correction, 128 34 vs 41, 256
+// 66 vs 69), and through the mean correction above (N = 384 125 vs 132, 512 206 vs 222, 1024
+// 839 vs 929).  c_z = 64 takes them while every workgroup has one group (two workgroups of four
+// waves per CU; N = 128 20.6 vs 24.7 with the persistent kernels, 4 x 128 36.7 vs 34.0).
+int trimul_run(const pf_trimul_args* a) {
+  hipStream_t st = (hipStream_t)a->stream;
+  const int B = a->B, N = a->N, cus = device_cus();
+  if (cus <= 0) return pf_fail(PF_E_LAUNCH, "pf_trimul_fwd: cannot query the device");
+  const size_t planes = (size_t)B * a->C * N * N;
+  const long ngroups = (long)B * N * N / DP_ROWS;
+  op_t* opA = (op_t*)a->workspace;
+  op_t* opB = opA + planes;
+  op_t* X = opB + planes;
+  float* amax_parts = reinterpret_cast<float*>(X + planes);
+  if (a->C == 64)
+    return ngroups <= 2 * cus ? trimul_run_direct<64, DL_NONE>(a, opA, opB, X, amax_parts, nullptr, 2 * cus)
+                              : trimul_run_persistent64(a, opA, opB, X, amax_parts, cus);
+  if (!(B == 1 && a->in_offsets && a->p_in_lo && a->g_in_lo && a->g_out_lo))
+    return trimul_run_direct<C, DL_NONE>(a, opA, opB, X, amax_parts, nullptr, cus);
+  if (a->p_out_lo && ngroups <= 4 * cus) return trimul_run_direct<C, DL_MFMA>(a, opA, opB, X, amax_parts, nullptr, cus);
+  float* stats = amax_parts + TM_MAX_PARTS;
+  pair_stats_kernel<<<PS_WG, 64 * PS_WAVES, 0, st>>>(a->z_in, N, a->eps, stats);
+  PF_CHECK_LAUNCH("pair_stats_kernel");
+  return trimul_run_direct<C, DL_MEAN>(a, opA, opB, X, amax_parts, stats, cus);
 }
 
 }  // namespace
@@ -817,7 +1034,7 @@ extern "C" int pf_trimul_fwd(const pf_trimul_args* a) {
   const size_t need = pf_trimul_workspace_size(a->B, a->N, a->C);
   if (a->workspace_bytes < need)
     return pf_fail(PF_E_INVALID, "pf_trimul_fwd: workspace too small (%zu < %zu bytes)", a->workspace_bytes, need);
-  return a->C == 128 ? trimul_run<128>(a) : trimul_run<64>(a);
+  return trimul_run(a);
 }
 
 int pf_contract_rect(const void* A, const void* B, void* X, int x_fp32, int planes, int M, int Nc, int K,
