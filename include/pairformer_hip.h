@@ -145,7 +145,8 @@ typedef struct pf_triatt_args {
    * layer_norm.bias), used instead of the 16-bit weights' W16 . beta; with also the residuals
    * of the kernel's gamma-folded weights, w_*_lo = W diag(gamma) - op(op(W) diag(gamma)) in the
    * operand type (op = rounding to it; [H*D][C] for q, k, v, [H][C] for the bias), and B == 1,
-   * the mean correction of pf_trimul_args for those rows. */
+   * the mean correction of pf_trimul_args for those rows (with w_g_lo and w_o_lo given as well,
+   * small grids multiply by these residuals too instead). */
   const float* in_offsets;
   const void* w_q_lo; const void* w_k_lo; const void* w_v_lo; const void* w_bias_lo;
 } pf_triatt_args;
@@ -341,8 +342,8 @@ int pf_transition_mx8_pair_bias_fwd(const pf_transition_mx8_args* t, const pf_ap
 /* Triangle attention in fast mode (same semantics and argument meaning as pf_triatt_fwd,
  * C = 128).  The block-fp8 points are those of the ttnn TriangleAttention under --fast
  * (tt_bio/tenstorrent.py:526-539 weights, 603-614 / 628-639 projections, 580-590 output):
- * linear_{q,k,v,g}.weight MXFP8 along C (pf_quantize_mx8, dequantized per call into the
- * workspace, so the LayerNorm output stays 16-bit as in the reference); q, k, v and g
+ * linear_{q,k,v,g}.weight MXFP8 along C (pf_quantize_mx8, dequantized by the kernels as they
+ * load them, so the LayerNorm output stays 16-bit as in the reference); q, k, v and g
  * quantize-dequantized per head (32 channels) right after their projections; the
  * o-projection's output per 32 channels before the residual.  linear.weight (the triangle
  * bias) and linear_o.weight stay 16-bit, as the reference keeps them bfloat16. */

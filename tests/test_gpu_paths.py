@@ -77,3 +77,34 @@ def test_trimul_c64_direct_line(gpu, B, N):
     want = ref.triangle_multiplication(z, pm, w, "outgoing")
     got = pairformer.TriangleMultiplication(False, w)(z.to(gpu), pm.to(gpu))
     check(f"trimul c64 B={B} N={N}", got, want)
+
+
+# ------------------------------------------------------------------------------ triangle attention
+@pytest.mark.parametrize("B,N", [(1, 64), (1, 256), (1, 320), (2, 192)])
+@pytest.mark.parametrize("ending", [False, True])
+@pytest.mark.parametrize("plain", [False, True])
+def test_triatt_direct(gpu, B, N, ending, plain):
+    """The projections with one group of 64 positions per workgroup and with several, on both sides
+    of the line between the residual MFMA and the mean correction (N = 256 / 320), with plain
+    weights, for a batch, with padded keys, and with the three ways of adding the residual."""
+    w = _sub_w(5, "tri_att_end" if ending else "tri_att_start")
+    wm = {(k[4:] if k.startswith("mha.") else k): v for k, v in w.items()}
+    n = N - 9
+    z = torch.zeros((B, N, N, 128))
+    pm = torch.zeros((B, N, N))
+    for b in range(B):
+        _, zb, _, pmb = _inputs(n, 5 + b, pad_tail=7, rand_mask=True)
+        z[b, :n, :n], pm[b, :n, :n] = zb[0], pmb[0]
+    opt = pairformer.Options(weight_residuals=not plain, mean_correction=not plain)
+    mod = pairformer.TriangleAttention(32, 4, ending, wm, opt)
+    want = ref.triangle_attention(z[:, :n, :n].to(gpu), pm[:, :n, :n].to(gpu), {k: v.to(gpu) for k, v in w.items()},
+                                  not ending)
+    zd, pd = z.to(gpu), pm.to(gpu).contiguous()
+    update = mod(zd, pd, n_valid=n)
+    check("triatt update", update[:, :n, :n], want)
+    other = torch.ones_like(zd)
+    check("triatt out += update", mod(zd, pd, out=other, accumulate=True, n_valid=n)[:, :n, :n] - 1.0, want)
+    inplace = zd.clone()
+    mod(inplace, pd, out=inplace, accumulate=True, n_valid=n)
+    # the same update added to z: one fp32 rounding of the sum apart
+    assert (inplace - (zd + update)).abs().max() <= 2.0 ** -22 * (zd.abs().max() + update.abs().max())

@@ -85,6 +85,55 @@ struct DirectW {
 #pragma unroll
     for (int s = 0; s < CC / 16; ++s) v[s] = ld_x8(buf + (lane & 31) * (CC + 8) + 16 * s + 8 * (lane >> 5));
   }
+  // W diag(gamma), rounded to op_t again
+  PF_DEV void fold(const float* gamma, int h) {
+    // (opaque: the 64 float conversions that an earlier W . beta took are not kept for this)
+#pragma unroll
+    for (int s = 0; s < CC / 16; ++s) asm volatile("" : "+v"(v[s]));
+#pragma unroll
+    for (int s = 0; s < CC / 16; ++s) {
+      const f32x4 g0 = *reinterpret_cast<const f32x4*>(gamma + 16 * s + 8 * h);
+      const f32x4 g1 = *reinterpret_cast<const f32x4*>(gamma + 16 * s + 8 * h + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[s][e] = (op_t)((float)v[s][e] * g0[e]);
+        v[s][4 + e] = (op_t)((float)v[s][4 + e] * g1[e]);
+      }
+      asm volatile("" : "+v"(v[s]));   // done here, not sunk to its use with gamma kept until then
+    }
+  }
+};
+
+// The fragments of a wave's 32 MXFP8 rows (e4m3 bytes [32][CC] at `q`, E8M0 scales [32][CC / 32] at
+// `sc`), loaded, then rounded to op_t (exact for scales in its range; a scale byte 0, an all-zero
+// block, gives zeros).
+template <int CC>
+struct DirectW8 {
+  typedef int i32x2_t __attribute__((ext_vector_type(2)));
+  i32x2_t w[CC / 16];
+  uint32_t e[CC / 32];
+  PF_DEV void load(const uint8_t* __restrict__ q, const uint8_t* __restrict__ sc, int lane) {
+    const int m = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int s = 0; s < CC / 16; ++s) w[s] = *reinterpret_cast<const i32x2_t*>(q + m * CC + 16 * s + 8 * h);
+#pragma unroll
+    for (int k = 0; k < CC / 32; ++k) e[k] = sc[m * (CC / 32) + k];
+  }
+  PF_DEV void dequant(DirectW<CC>& o) const {
+#pragma unroll
+    for (int s = 0; s < CC / 16; ++s) {
+      const float X = __uint_as_float(e[s >> 1] << 23);
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        const auto lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w[s][d], X, false);
+        const auto hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w[s][d], X, true);
+        o.v[s][4 * d + 0] = (op_t)lo[0];
+        o.v[s][4 * d + 1] = (op_t)lo[1];
+        o.v[s][4 * d + 2] = (op_t)hi[0];
+        o.v[s][4 * d + 3] = (op_t)hi[1];
+      }
+    }
+  }
 };
 
 // How a direct kernel uses the rounding residuals of its weights: not at all, as a second MFMA per
@@ -112,6 +161,7 @@ PF_DEV float direct_wbeta(const opx8 (&w)[KS], const float* beta, int h) {
     const f32x4 b1 = *reinterpret_cast<const f32x4*>(beta + 16 * s + 8 * h + 4);
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc += (float)w[s][e] * b0[e] + (float)w[s][4 + e] * b1[e];
+    asm volatile("" : "+v"(acc));   // not all of beta in registers at once
   }
   return xor32_sum(acc);
 }

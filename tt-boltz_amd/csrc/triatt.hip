@@ -18,12 +18,12 @@
 //   ta_attn  flash attention (see the kernel's comment): 16-wave workgroups of 4 frame rows
 //            x 128 queries, LDS-DMA ring, bias / mask / reference max folded into MFMAs,
 //            lazy-max softmax.  Output O (normalized, ungated) op_t [B][N(i)][N(j)][H*D].
-//   ta_out   o-proj epilogue (persistent, W_g / W_o in LDS, output-aligned layout): gate
-//            recomputed from LN(z) (MFMA), o*sigmoid(g) built in registers as linear_o's B
-//            operand, residual added to the z values the lane loaded for the LayerNorm.
+//   ta_out   o-proj epilogue: gate recomputed from LN(z) (MFMA), o*sigmoid(g) as linear_o's B
+//            operand through LDS, residual.
 #include <type_traits>
 
 #include "pf_common.h"
+#include "pf_direct.h"
 #include "pf_internal.h"
 
 namespace {
@@ -54,240 +54,282 @@ PF_DEV op_t mask_term(bool pad, float mv) {
 }
 
 // ---------------------------------------------------------------------------------
-// Projection (persistent): one workgroup of 8 waves per CU keeps W_q, W_k, W_v and the
-// bias rows in LDS with the LayerNorm affine folded in (W' = W diag(gamma) in op_t,
-// c = W beta in fp32 as the accumulator start), so a tile only normalizes.  Each wave
-// walks tiles of 32 frame positions (ip, j0 .. j0+31) and loads the next tile's z rows
-// while it computes the current one.  The MFMA orientation is chosen per output so that
-// the stores are 16-byte runs (8-byte runs write at ~2/3 of the bandwidth):
-//   Q, K  [j][d]:  D[d][pos]   runs of 4 d, paired across lane halves (store_runs16)
-//   V^T   [d][k]:  D[pos][d]   a lane's key runs g = 2p, 2p+1 are 8 adjacent slots
+// Projection (pf_direct.h): 12 waves walk groups of 64 frame positions (ip, j0 .. j0 + 63).  Wave w
+// owns one head of q (w < 4), k (w < 8) or v: its 32 weight rows in registers with the LayerNorm
+// affine folded in (W' = W diag(gamma) in op_t, W beta in fp32 as the accumulator start), so a
+// group is only normalized, by waves 0-7.  Waves 8 and 9 also compute the triangle bias of one
+// 32-position tile each, from the bias rows in LDS.  The MFMA orientation is chosen per output so
+// that the outputs' LDS stage takes 8- or 16-byte writes, and every store instruction writes whole
+// 128-byte lines:
+//   Q, K  [j][d]:  D[d][pos]   a lane holds runs of 4 d of its position
+//   V^T   [d][k]:  D[pos][d]   a lane's key runs g = 2p, 2p+1 are 8 adjacent slots (perm16)
 //   bias  [hd][j]: D[hd][pos]  a lane holds the 4 heads of its position
-// FAST (the fast mode's block-fp8 points): q, k and v are quantize-dequantized per head (one
-// 32-channel block per position) before they are stored.  Q and K blocks are lane pairs of
-// the D[d][pos] accumulator; V's D[pos][d] orientation spreads a block over 32 lanes, so a
-// D[d][pos] copy of V gives each key's block scale, passed through 32 floats of LDS per wave.
+// FAST (the fast mode's block-fp8 points): the weights come as MXFP8 and are dequantized into the
+// registers; q, k and v are quantize-dequantized per head (one 32-channel block per position)
+// before they are stored.  Q and K blocks are lane pairs of the D[d][pos] accumulator; V's D[pos][d]
+// orientation spreads a block over 32 lanes, so a D[d][pos] copy of V gives each key's block scale,
+// passed through 32 floats of LDS per wave.
+// Against weights resident in LDS with one 8-wave workgroup's wave per tile (us a launch): N = 128
+// 20.6 + 5.2 of statistics -> 15.1, 384 54 -> 41, 512 89 -> 65, 1024 314 -> 242.
 // ---------------------------------------------------------------------------------
-constexpr int TAP_WAVES = 8;
-constexpr int TAP_ROWS = 3 * C + 32;   // q, k, v rows, then 32 bias rows (H used, rest zero)
-// LDS: the weights [TAP_ROWS][CC + 8] op_t, their accumulator starts [TAP_ROWS] fp32, then (FAST)
-// the per-wave V block scales or the mean-correction mu [128] and its reduction scratch (the two
-// never coexist)
-template <int CC, bool FAST = false>
+constexpr int TAP_WAVES = 12, TAP_LN = 8;   // waves; the first ones normalize
+constexpr int TAP_SP = 40, TAP_VP = 72;     // stage pitches: [64 positions][32 d + 8], [32 d][64 keys + 8]
+template <int CC>
 constexpr size_t tap_lds() {
-  return (size_t)TAP_ROWS * (CC + 8) * sizeof(op_t) + TAP_ROWS * sizeof(float) +
-         (FAST ? TAP_WAVES * 32 * sizeof(float) : (PS_C + 64 * TAP_WAVES) * sizeof(float));
+  return (size_t)(2 * DP_ROWS * (CC + 8) + 2 * H * (CC + 8)) * sizeof(op_t) +
+         (size_t)TAP_WAVES * (32 * (CC + 8) > DP_ROWS * TAP_SP ? 32 * (CC + 8) : DP_ROWS * TAP_SP) * sizeof(op_t) +
+         (3 * C + 32 + 32 * TAP_WAVES) * sizeof(float);
 }
 
+// W_q, W_k, W_v, W_g: op_t [C][CC], or (FAST) MXFP8 bytes with their scales in `s`.
+struct TaWeights {
+  const void* w[4];
+  const void* s[4] = {nullptr, nullptr, nullptr, nullptr};
+  const op_t *g_lo = nullptr, *o_lo = nullptr;   // the residuals of W_g and W_o (op_t, or null)
+};
+
 // offb (optional, fp32 [3 C + H]): the exact W beta of the q, k, v and bias rows (else computed
-// from the op_t weights); with lo (the residuals of the kernel's gamma-folded weights, W diag(gamma)
-// - op_t(W16 diag(gamma)), four [rows][CC] arrays for q, k, v, bias) and the stats partials also
-// the mean correction of those weights (see pair_stats_kernel).
+// from the op_t weights); lo: the residuals of the kernel's gamma-folded weights (W diag(gamma) -
+// op_t(W16 diag(gamma)), four [rows][CC] arrays for q, k, v, bias), used as DirectLo says, with the
+// stats partials for DL_MEAN.
 struct TaMeanFix { const float* offb; const op_t* lo[4]; const float* stats; };
 
-template <int CC, bool FAST>
+template <int CC, bool FAST, int LO>
 __global__ __launch_bounds__(64 * TAP_WAVES, 1) void ta_proj_kernel(
     const float* __restrict__ z, const float* __restrict__ pair_mask,
-    const float* __restrict__ lnw, const float* __restrict__ lnb,
-    const op_t* __restrict__ wq, const op_t* __restrict__ wk, const op_t* __restrict__ wv,
+    const float* __restrict__ lnw, const float* __restrict__ lnb, TaWeights tw,
     const op_t* __restrict__ wb, op_t* __restrict__ Q, op_t* __restrict__ K,
     op_t* __restrict__ Vt, float* __restrict__ bias32, op_t* __restrict__ mask16,
-    int B, int N, int n_valid, int ending, float qscale, float eps, TaMeanFix mf) {
-  constexpr int LW = CC + 8, KS = CC / 16;
+    int ngroups, int N, int n_valid, int ending, float qscale, float eps, TaMeanFix mf) {
+  constexpr int LW = CC + 8, KS = CC / 16, NT = 64 * TAP_WAVES;
+  constexpr int WB = 32 * LW > DP_ROWS * TAP_SP ? 32 * LW : DP_ROWS * TAP_SP;   // a wave's buffer
   extern __shared__ __attribute__((aligned(16))) op_t plds[];
-  float* cb = reinterpret_cast<float*>(plds + TAP_ROWS * LW);
+  op_t* sx = plds;                                     // normalized positions [2][64][LW]
+  op_t* sbw = sx + 2 * DP_ROWS * LW;                   // bias rows, then (DL_MFMA) their residuals [2][H][LW]
+  op_t* wbuf = sbw + 2 * H * LW;                       // weights, then outputs, per wave
+  float* soff = reinterpret_cast<float*>(wbuf + TAP_WAVES * WB);   // W beta of the q, k, v rows, the bias rows
+  float* vsc = soff + 3 * C + 32;                      // FAST: a wave's per-key V block scales
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  float* vsc = cb + TAP_ROWS + 32 * wid;   // FAST: this wave's per-key V block scales
-  float* mu = cb + TAP_ROWS;               // !FAST: the mean correction's mu
-  auto wrow = [&](int row) -> const op_t* {   // weight rows have CC inputs
-    return row < C ? wq + row * CC : row < 2 * C ? wk + (row - C) * CC
-         : row < 3 * C ? wv + (row - 2 * C) * CC : wb + (row - 3 * C) * CC;
+  const int kind = wid >> 2, hd = wid & 3;             // 0 q, 1 k, 2 v
+  op_t* stg = wbuf + wid * WB;
+  vsc += 32 * wid;
+  auto group = [&](int g) PF_INLINE -> PosTile { return pos_tile(2u * g, N); };
+  // the z pair of frame position c of a group
+  auto zpair = [&](const PosTile& pt, int c) PF_INLINE -> long {
+    return ((long)pt.b * N + (ending ? pt.c0 + c : pt.r)) * N + (ending ? pt.r : pt.c0 + c);
   };
-  {   // every global load of the set-up first (weights, the offset row, partials), then LDS
-    constexpr int NT = 64 * TAP_WAVES, CH = TAP_ROWS * (CC / 8), SPER = (CH + NT - 1) / NT;
-    static_assert(TAP_ROWS <= NT && NT % (CC / 8) == 0, "one offset row per thread; one column per thread");
-    const int col = (tid % (CC / 8)) * 8;   // the same for every chunk of this thread
-    opx8 wv[SPER];
+  DirectLn<CC, TAP_LN> ln;
+  float mv = 1.f;
+  auto fetch = [&](int g) PF_INLINE {
+    const PosTile pt = group(g);
+    if (wid < TAP_LN) ln.load(z, [&](int c) PF_INLINE -> long { return zpair(pt, c); }, wid, lane);
+    if (pair_mask && tid < DP_ROWS) mv = pair_mask[zpair(pt, tid)];
+  };
+  // ---- set-up: every global load first, so that it costs about one memory round trip ----
+  fetch(blockIdx.x);
+  ln.load_gamma(nullptr, lane);
+  DirectW<CC> w, wl;
+  const long r0 = 32l * hd * CC;
+  if constexpr (!FAST) w.load((const op_t*)tw.w[kind] + r0, lane);
+  const int row = 32 * wid + m;   // of the 3 C projection rows
+  const bool exact = !FAST && mf.offb;
+  float c0 = exact ? mf.offb[row] : 0.f;
+  const float gb = tid < 2 * CC ? (tid < CC ? lnw[tid] : lnb[tid - CC]) : 0.f;
+  // bias rows: wave 0 (c_z = 64: half of it), 8 channels bc .. of row br a lane
+  const bool bias_lane = tid < H * CC / 8;
+  const int br = tid / (CC / 8), bc = 8 * (tid % (CC / 8));
+  opx8 bw = zero_x8(), bl = zero_x8();
+  float cb = 0.f;
+  if (bias_lane) {
+    bw = ld_x8(wb + br * CC + bc);
+    if constexpr (LO != DL_NONE) bl = ld_x8(mf.lo[3] + br * CC + bc);
+    if (exact) cb = mf.offb[3 * C + br];
+  }
+  float psum = 0.f;
+  if constexpr (LO == DL_MEAN) {
+    if (tid < 512) {
+      float pv[stats_per<512>()];
+      stats_load<512>(mf.stats, pv);
 #pragma unroll
-    for (int i = 0; i < SPER; ++i) {
-      const int c = tid + NT * i, row = c / (CC / 8);
-      wv[i] = c < CH && row < 3 * C + H ? ld_x8(wrow(row) + col) : zero_x8();
-    }
-    float gcol[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) gcol[e] = lnw[col + e];
-    const bool meanfix = !FAST && mf.offb && mf.stats;
-    const int orow = tid;   // this thread's offset row
-    const bool live_row = orow < 3 * C + H;
-    float pv[stats_per<NT>()];
-    if (meanfix) stats_load<NT>(mf.stats, pv);
-    // the row behind this thread's offset: the residual (mean correction) or the weight (W beta)
-    opx8 rv[CC / 8];
-    float offb_v = 0.f;
-    const bool use_offb = !FAST && mf.offb;
-    if (live_row) {
-      if (use_offb) {
-        offb_v = mf.offb[orow];
-        if constexpr (CC == PS_C)
-          if (mf.stats) {
-            const op_t* lo = mf.lo[orow < 3 * C ? orow / C : 3] + (orow < 3 * C ? orow % C : orow - 3 * C) * CC;
-#pragma unroll
-            for (int c = 0; c < CC / 8; ++c) rv[c] = ld_x8(lo + 8 * c);
-          }
-      } else {
-        const op_t* w = wrow(orow);
-#pragma unroll
-        for (int c = 0; c < CC / 8; ++c) rv[c] = ld_x8(w + 8 * c);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < SPER; ++i) {
-      const int c = tid + NT * i, row = c / (CC / 8);
-      if (c < CH) {
-        opx8 v;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = (op_t)((float)wv[i][e] * gcol[e]);
-        st_x8(plds + row * LW + col, row < 3 * C + H ? v : zero_x8());
-      }
-    }
-    if (meanfix) {
-      stats_reduce<NT>(pv, mu, mu + PS_C);
-      __syncthreads();
-    }
-    if (orow < TAP_ROWS) {   // accumulator starts W beta
-      float acc = 0.f;
-      if (live_row) {
-        if (use_offb) {
-          if constexpr (CC == PS_C) acc = corrected_offset_regs<false>(offb_v, rv, mf.stats != nullptr, nullptr, mu);
-        } else {
-#pragma unroll
-          for (int c = 0; c < CC / 8; ++c)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc += (float)rv[c][e] * lnb[8 * c + e];
-        }
-      }
-      cb[orow] = acc;
+      for (int i = 0; i < stats_per<512>(); ++i) psum += pv[i];
     }
   }
+  DirectW8<CC> w8;
+  if constexpr (FAST)
+    w8.load((const uint8_t*)tw.w[kind] + r0, (const uint8_t*)tw.s[kind] + 32 * hd * (CC / 32), lane);
+  __builtin_amdgcn_sched_barrier(0);
+  float* sgb = reinterpret_cast<float*>(sx + DP_ROWS * LW);   // gamma, beta [2][CC], mu [CC], partial sums [4][128]
+  float* smu = sgb + 2 * CC;                                  // (in sx[1], free until the second group)
+  if (tid < 2 * CC) sgb[tid] = gb;
+  if (LO == DL_MEAN && tid < 512) smu[PS_C + tid] = psum;
+  __syncthreads();
+  if (LO == DL_MEAN && tid < PS_C)
+    smu[tid] = (smu[PS_C + tid] + smu[2 * PS_C + tid]) + (smu[3 * PS_C + tid] + smu[4 * PS_C + tid]);
+  if constexpr (FAST)
+    w8.dequant(w);
+  else
+    w.turn(stg, lane);
+  __builtin_amdgcn_sched_barrier(0);
+  // (the residuals' own round trip runs beside the LayerNorm: with everything in flight at once
+  // the set-up spilled)
+  if constexpr (LO != DL_NONE) wl.load(mf.lo[kind] + r0, lane);
+  if (wid < TAP_LN) ln.store(sx, eps, wid, lane);
+  if (!exact) c0 = direct_wbeta<KS>(w.v, sgb + CC, h);
+  w.fold(sgb, h);
+  if constexpr (LO != DL_NONE) wl.turn(stg, lane);
+  auto bias_sum = [&](float v) PF_INLINE -> float {   // over the CC / 8 lanes of a bias row
+#pragma unroll
+    for (int o = CC / 16; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+  };
+  if (wid == 0) {
+    float d = 0.f;
+    opx8 f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      d += (float)bw[e] * sgb[CC + bc + e];
+      f[e] = (op_t)((float)bw[e] * sgb[bc + e]);
+    }
+    d = bias_sum(d);
+    if (!exact) cb = d;
+    if (bias_lane) {
+      st_x8(sbw + br * LW + bc, f);
+      if constexpr (LO == DL_MFMA) st_x8(sbw + (H + br) * LW + bc, bl);
+    }
+  }
+  if constexpr (LO == DL_MEAN) {
+    __syncthreads();
+    c0 += direct_wbeta<KS>(wl.v, smu, h);
+    if (wid == 0) {
+      float d = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) d += (float)bl[e] * smu[bc + e];
+      cb += bias_sum(d);
+    }
+  }
+  if (h == 0) soff[row] = c0;
+  if (bias_lane && bc == 0) soff[3 * C + br] = cb;
   __syncthreads();
 
-  const uint32_t tiles = (uint32_t)B * N * N / 32;
-  const uint32_t stride = gridDim.x * TAP_WAVES;
-  // frame tile t -> (b, ip, j0) and the z pair this lane's row comes from
-  auto decode = [&](uint32_t t, int& b, int& ip, int& j0) PF_INLINE {
-    const PosTile pt = pos_tile(t, N);
-    b = pt.b;
-    ip = pt.r;
-    j0 = pt.c0;
-  };
-  auto zpair = [&](int b, int ip, int j0) -> long {
-    return ((long)b * N + (ending ? j0 + m : ip)) * N + (ending ? ip : j0 + m);
-  };
-  float xn[CC / 2];
-  uint32_t t = blockIdx.x * TAP_WAVES + wid;
-  if (t < tiles) {
-    int b, ip, j0;
-    decode(t, b, ip, j0);
-    load_row_frag<CC>(z + zpair(b, ip, j0) * CC, h, xn);
-  }
-  for (; t < tiles; t += stride) {
-    int b, ip, j0;
-    decode(t, b, ip, j0);
-    const long pair = zpair(b, ip, j0);
-    opx8 xf[KS];
-    {
-      float x[CC / 2];
-#pragma unroll
-      for (int i = 0; i < CC / 2; ++i) x[i] = xn[i];
-      if (t + stride < tiles) {   // next tile's rows, in flight during this tile
-        int b2, ip2, j02;
-        decode(t + stride, b2, ip2, j02);
-        load_row_frag<CC>(z + zpair(b2, ip2, j02) * CC, h, xn);
-      }
-      ln_norm_to_frag<CC>(x, eps, xf);
+  int buf = 0;
+  for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x, buf ^= 1) {
+    const PosTile pt = group(gi);
+    op_t* sxb = sx + buf * DP_ROWS * LW;
+    if (gi != (int)blockIdx.x) {
+      if (wid < TAP_LN) ln.store(sxb, eps, wid, lane);
+      __syncthreads();   // sx[buf] is whole; every wave is done with sx[buf ^ 1]
     }
-    if (h == 0) {
-      // frame key j0+m of row ip: padding -> excluded; otherwise inf*(mask-1) (log2 units)
-      const float mv = pair_mask ? pair_mask[pair] : 1.f;
-      mask16[((long)b * N + ip) * N + j0 + m] = mask_term(j0 + m >= n_valid, mv);
-    }
-    const long rowh = ((long)b * N + ip) * H;   // (b, ip) head-block index base
-    // Q, K: D[d][pos]; lane (pos m, h) holds d = 8g + 4h + e in acc[4g + e]
-#pragma unroll 1
-    for (int blk = 0; blk < 8; ++blk) {
-      f32x16 acc;
+    if (tid < DP_ROWS)
+      // frame key j0 + tid of row ip: padding -> excluded; otherwise inf*(mask-1) (log2 units)
+      mask16[((long)pt.b * N + pt.r) * N + pt.c0 + tid] = mask_term(pt.c0 + tid >= n_valid, mv);
+    if (gi + (int)gridDim.x < ngroups) fetch(gi + gridDim.x);
+    const long rowh = ((long)pt.b * N + pt.r) * H + hd;   // (b, ip, head) block
+    if (kind < 2) {
+      // Q, K: D[d][pos]; lane (pos m, h) holds d = 8g + 4h + e in acc[4g + e]
+      f32x16 acc[2];
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const f32x4 c4 = *reinterpret_cast<const f32x4*>(cb + 32 * blk + 8 * g + 4 * h);
+        const f32x4 c4 = *reinterpret_cast<const f32x4*>(soff + 32 * wid + 8 * g + 4 * h);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[4 * g + e] = c4[e];
+        for (int e = 0; e < 4; ++e) acc[0][4 * g + e] = acc[1][4 * g + e] = c4[e];
       }
 #pragma unroll
-      for (int s2 = 0; s2 < KS; ++s2) acc = mfma32(ld_x8(plds + (32 * blk + m) * LW + 16 * s2 + 8 * h), xf[s2], acc);
-      if constexpr (FAST) mx_fake_quant16(acc);
-      op_t* dst = blk < 4 ? Q : K;
-      store_runs16(dst + ((rowh + (blk & 3)) * N + j0 + m) * D, acc, blk < 4 ? qscale : 1.f, h);
-    }
-    // V^T: D[pos][d]; lane (d m, h) holds keys j0 + 8g + 4h + e in acc[4g + e]
-#pragma unroll 1
-    for (int hd = 0; hd < H; ++hd) {
-      if constexpr (FAST) {   // block scale of key j0 + m -> vsc[m]
-        f32x16 at;
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const opx8 xf = ld_x8(sxb + (32 * t + m) * LW + 16 * s + 8 * h);
+          acc[t] = mfma32(w.v[s], xf, acc[t]);
+          if constexpr (LO == DL_MFMA) acc[t] = mfma32(wl.v[s], xf, acc[t]);
+          if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // not every fragment read at once
+        }
+      const float sc = kind == 0 ? qscale : 1.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        if constexpr (FAST) mx_fake_quant16(acc[t]);
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const f32x4 c4 = *reinterpret_cast<const f32x4*>(cb + 2 * C + 32 * hd + 8 * g + 4 * h);
+          opx4 v;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) at[4 * g + e] = c4[e];
-        }
-#pragma unroll
-        for (int s2 = 0; s2 < KS; ++s2)
-          at = mfma32(ld_x8(plds + (2 * C + 32 * hd + m) * LW + 16 * s2 + 8 * h), xf[s2], at);
-        float a = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) a = fmaxf(a, fabsf(at[r]));
-        a = xor32_max(a);
-        if (h == 0) vsc[m] = mx_block_scale(a);
-      }
-      const float c0 = cb[2 * C + 32 * hd + m];
-      f32x16 acc;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = c0;
-#pragma unroll
-      for (int s2 = 0; s2 < KS; ++s2)
-        acc = mfma32(xf[s2], ld_x8(plds + (2 * C + 32 * hd + m) * LW + 16 * s2 + 8 * h), acc);
-      if constexpr (FAST) {   // same wave: its LDS accesses complete in order
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4 X4 = *reinterpret_cast<const f32x4*>(vsc + 8 * g + 4 * h);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[4 * g + e] = mx_fake_quant1(acc[4 * g + e], X4[e], 448.f * X4[e]);
+          for (int e = 0; e < 4; ++e) v[e] = (op_t)(acc[t][4 * g + e] * sc);
+          st_x4(stg + (32 * t + m) * TAP_SP + 8 * g + 4 * h, v);
         }
       }
-      // keys 8g + 4h + e of runs g = 2p, 2p+1 sit at storage 16p + 8h .. +7 (perm16)
-      op_t* row = Vt + ((rowh + hd) * D + m) * (long)N + j0;
+      op_t* dst = (kind == 0 ? Q : K) + (rowh * N + pt.c0) * D;   // 64 positions of 32 d: 4 KB
 #pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        opx8 v;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = (op_t)acc[8 * p + e];
-        st_x8(row + 16 * p + 8 * h, v);
+      for (int q = 0; q < 4; ++q) {
+        const int c = lane + 64 * q;
+        st_x8(dst + 8 * c, ld_x8(stg + (c >> 2) * TAP_SP + 8 * (c & 3)));
       }
-    }
-    // bias: D[hd][pos]; rows 0..H-1 are acc[0..3] of the h = 0 lanes
-    {
-      f32x16 acc;
+    } else {
+      // V^T: D[pos][d]; lane (d m, h) holds keys 8g + 4h + e of a tile in acc[4g + e]
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 c4 = *reinterpret_cast<const f32x4*>(cb + 3 * C + 8 * g + 4 * h);
+      for (int t = 0; t < 2; ++t) {
+        const op_t* xr = sxb + (32 * t + m) * LW + 8 * h;
+        if constexpr (FAST) {   // block scale of key 32 t + m -> vsc[m]
+          f32x16 at;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[4 * g + e] = c4[e];
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 c4 = *reinterpret_cast<const f32x4*>(soff + 32 * wid + 8 * g + 4 * h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) at[4 * g + e] = c4[e];
+          }
+#pragma unroll
+          for (int s = 0; s < KS; ++s) at = mfma32(w.v[s], ld_x8(xr + 16 * s), at);
+          float a = 0.f;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) a = fmaxf(a, fabsf(at[r]));
+          a = xor32_max(a);
+          if (h == 0) vsc[m] = mx_block_scale(a);
+        }
+        f32x16 acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = c0;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const opx8 xf = ld_x8(xr + 16 * s);
+          acc = mfma32(xf, w.v[s], acc);
+          if constexpr (LO == DL_MFMA) acc = mfma32(xf, wl.v[s], acc);
+        }
+        if constexpr (FAST) {   // same wave: its LDS accesses complete in order
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 X4 = *reinterpret_cast<const f32x4*>(vsc + 8 * g + 4 * h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[4 * g + e] = mx_fake_quant1(acc[4 * g + e], X4[e], 448.f * X4[e]);
+          }
+        }
+        // keys 8g + 4h + e of runs g = 2p, 2p+1 sit at storage 16p + 8h .. +7 (perm16)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          opx8 v;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = (op_t)acc[8 * p + e];
+          st_x8(stg + m * TAP_VP + 32 * t + 16 * p + 8 * h, v);
+        }
       }
+      op_t* dst = Vt + rowh * D * (long)N + pt.c0;
 #pragma unroll
-      for (int s2 = 0; s2 < KS; ++s2) acc = mfma32(ld_x8(plds + (3 * C + m) * LW + 16 * s2 + 8 * h), xf[s2], acc);
-      if (h == 0) {
+      for (int q = 0; q < 4; ++q) {   // eight lanes write a d's 128 bytes
+        const int d = 8 * q + (lane >> 3), chunk = lane & 7;
+        st_x8(dst + (long)d * N + 8 * chunk, ld_x8(stg + d * TAP_VP + 8 * chunk));
+      }
+      if (hd < 2) {   // the bias of tile hd: D[head][pos]; rows 0..H-1 are acc[0..3] of the h = 0 lanes
+        f32x16 acc = zero16();
+        const op_t* br = sbw + (m & (H - 1)) * LW + 8 * h;   // rows past H repeat and are not stored
+        const op_t* xr = sxb + (32 * hd + m) * LW + 8 * h;
 #pragma unroll
-        for (int r = 0; r < H; ++r) bias32[(((long)b * H + r) * N + ip) * N + j0 + m] = acc[r] * LOG2E;
+        for (int s = 0; s < KS; ++s) {
+          const opx8 xf = ld_x8(xr + 16 * s);
+          acc = mfma32(ld_x8(br + 16 * s), xf, acc);
+          if constexpr (LO == DL_MFMA) acc = mfma32(ld_x8(br + H * LW + 16 * s), xf, acc);
+        }
+        if (h == 0) {
+#pragma unroll
+          for (int r = 0; r < H; ++r)
+            bias32[(((long)pt.b * H + r) * N + pt.r) * N + pt.c0 + 32 * hd + m] =
+                (acc[r] + soff[3 * C + r]) * LOG2E;
+        }
       }
     }
   }
@@ -706,164 +748,148 @@ __global__ __launch_bounds__(64 * TA_WAVES, 1) void ta_attn_kernel(
 }
 
 // ---------------------------------------------------------------------------------
-// Output projection: z[pair(i, j)] (+)= linear_o(O[i, j] * sigmoid(linear_g(LN(z[pair])))).
-// Persistent: one workgroup (8 waves) per CU keeps W_g and W_o in LDS (op_t as given, so rounded
-// once) with the LayerNorm's beta folded into fp32 gate offsets -log2(e) W_g beta (gamma scales
-// the normalized z before its rounding to op_t); each wave walks tiles of 32 frame positions
-// (ip, j0 .. j0+31).  Everything is in the output-aligned layout (pf_common.h): the gate comes
-// out of D[channel][position] = W_g . LN(z) in the same channel order as the O values the lane
-// loads, o * sigmoid(g) is directly the B operand of D[out][position] = W_o . (o * g), and the
-// residual is the z the lane loaded.  Weight rows are 4 op_t longer than their width, so the
-// 8-byte fragment reads of 32 rows fall on distinct banks.
-// FAST (the fast mode's block-fp8 points): the gate's offsets are W_g beta itself, and g
-// (per head: one 32-channel block, a lane pair's 16 + 16 registers) and the projection's
-// output (per 32 output channels) are quantize-dequantized before the sigmoid and before
-// the residual.
+// Output projection (pf_direct.h): z[pair(i, j)] (+)= linear_o(O[i, j] * sigmoid(linear_g(LN(z[pair])))).
+// 8 waves walk groups of 64 frame positions (ip, j0 .. j0 + 63); wave w owns head w >> 1 of the gate
+// and the output channels 32 (w >> 1) .. + 31 (c_z = 64: two of the four) of the positions
+// 32 (w & 1) .. + 31, its rows of W_g and W_o in registers.  The gate comes out of
+// D[channel][position] = W_g . LN(z), o * sigmoid(g) goes through LDS as the B operand of
+// D[out][position] = W_o . (o * g), and the residual is loaded in the accumulator's order.
+// FAST (the fast mode's block-fp8 points): W_g comes as MXFP8, and g (per head: one 32-channel
+// block, a lane pair's 16 + 16 registers) and the projection's output (per 32 output channels) are
+// quantize-dequantized before the sigmoid and before the residual.
+// Against weights resident in LDS with one wave per tile (us a launch): N = 128 19.6 -> 12.4, 384
+// 61 -> 50, 512 96 -> 87, 1024 342 -> 300.
 // ---------------------------------------------------------------------------------
 constexpr int TAO_WAVES = 8;
-// LDS: the gate offsets [C] and gamma [CC] (fp32, first: small immediate offsets), then
-// W_g [C][CC + 4] and W_o [CC][C + 4] op_t, then (HILO) their residuals in the same layout
-template <int CC, bool HILO = false>
+template <int CC>
 constexpr size_t tao_lds() {
-  return (C + CC) * sizeof(float) + (HILO ? 2 : 1) * ((size_t)C * (CC + 4) + (size_t)CC * (C + 4)) * sizeof(op_t);
+  return (size_t)(2 * DP_ROWS * (CC + 8) + DP_ROWS * (C + 8) + TAO_WAVES * 32 * (C + 8)) * sizeof(op_t) +
+         C * sizeof(float);
 }
 
 // resid: 0 -> out = update; 1 -> out = z_in + update (out may alias z_in); 2 -> out += update
-// HILO: W_g and W_o come with their residuals wg_lo = W_g - W_g16, wo_lo = W_o - W_o16 (rounded
-// to op_t), and both products run on hi + lo (two MFMAs per fragment): weights good to ~2^-22
-// of their size instead of the 2^-12 of one 16-bit rounding.  The gate's offsets use hi + lo.
+// HILO: W_g and W_o come with their residuals (rounded to op_t), and both products run on hi + lo
+// (two MFMAs per fragment): weights good to ~2^-22 of their size instead of the 2^-12 of one 16-bit
+// rounding.  The gate's offsets use hi + lo.
 template <int CC, bool FAST, bool HILO = false>
 __global__ __launch_bounds__(64 * TAO_WAVES, 1) void ta_out_kernel(
     const op_t* __restrict__ O, const float* z_in, float* out, const float* __restrict__ lnw,
-    const float* __restrict__ lnb, const op_t* __restrict__ wg, const op_t* __restrict__ wo,
-    const op_t* __restrict__ wg_lo, const op_t* __restrict__ wo_lo,
-    int B, int N, int ending, int resid, float eps) {
-  constexpr int LWG = CC + 4, LWO = C + 4, KS = CC / 16;
+    const float* __restrict__ lnb, TaWeights tw, const op_t* __restrict__ wo, int ngroups, int N, int ending,
+    int resid, float eps) {
+  constexpr int LW = CC + 8, LO_ = C + 8, KS = CC / 16;
   extern __shared__ __attribute__((aligned(16))) op_t tlds[];
-  float* cgate = reinterpret_cast<float*>(tlds);
-  float* gam = cgate + C;
-  op_t* sWg = tlds + 2 * (C + CC);
-  op_t* sWo = sWg + C * LWG;
-  op_t* sWgl = sWo + CC * LWO;   // HILO only
-  op_t* sWol = sWgl + C * LWG;
+  op_t* sx = tlds;                            // normalized positions [2][64][LW]
+  op_t* sog = sx + 2 * DP_ROWS * LW;          // o * sigmoid(g) [64][C + 8]
+  op_t* wbuf = sog + DP_ROWS * LO_;           // the waves' weight buffers [8][32][C + 8]
+  float* soff = reinterpret_cast<float*>(wbuf + TAO_WAVES * 32 * LO_);   // W_g beta (times -log2(e) unless FAST)
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  {   // weights -> LDS: every chunk of this thread loaded before the first store
-    constexpr int NT = 64 * TAO_WAVES;
-    static_assert(CC <= NT, "gamma: one value per thread");
-    opx8 vg[stage_per<NT, C, CC>()], vo[stage_per<NT, CC, C>()];
-    stage_load<NT, C, CC>(wg, vg);
-    stage_load<NT, CC, C>(wo, vo);
-    const float gv = tid < CC ? lnw[tid] : 0.f;
+  const int tile = wid & 1, cb = wid >> 1;
+  const bool has_out = 32 * cb < CC;
+  auto group = [&](int g) PF_INLINE -> PosTile { return pos_tile(2u * g, N); };
+  auto zpair = [&](const PosTile& pt, int c) PF_INLINE -> long {
+    return ((long)pt.b * N + (ending ? pt.c0 + c : pt.r)) * N + (ending ? pt.r : pt.c0 + c);
+  };
+  DirectLn<CC, TAO_WAVES> ln;
+  opx4 ov[4];   // O of channels 32 cb + 8 g + 4 h .. + 3 of position 32 tile + m
+  auto fetch = [&](int g) PF_INLINE {
+    const PosTile pt = group(g);
+    ln.load(z_in, [&](int c) PF_INLINE -> long { return zpair(pt, c); }, wid, lane);
+    const op_t* src = O + ((long)DP_ROWS * g + 32 * tile + m) * C + 32 * cb + 4 * h;
+#pragma unroll
+    for (int gg = 0; gg < 4; ++gg) ov[gg] = ld_x4(src + 8 * gg);
+  };
+  fetch(blockIdx.x);
+  ln.load_gamma(lnw, lane);
+  DirectW<CC> wg, wgl;
+  DirectW<C> wo_, wol;
+  DirectW8<CC> wg8;
+  if constexpr (FAST)
+    wg8.load((const uint8_t*)tw.w[3] + 32l * cb * CC, (const uint8_t*)tw.s[3] + 32 * cb * (CC / 32), lane);
+  else
+    wg.load((const op_t*)tw.w[3] + 32l * cb * CC, lane);
+  const long or0 = has_out ? 32l * cb * C : 0;
+  wo_.load(wo + or0, lane);
+  if constexpr (HILO) {
+    wgl.load(tw.g_lo + 32l * cb * CC, lane);
+    wol.load(tw.o_lo + or0, lane);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    op_t* wb = wbuf + wid * 32 * LO_;
+    if constexpr (FAST)
+      wg8.dequant(wg);
+    else
+      wg.turn(wb, lane);
+    wo_.turn(wb, lane);
+    float c0 = direct_wbeta<KS>(wg.v, lnb, h);
     if constexpr (HILO) {
-      opx8 vgl[stage_per<NT, C, CC>()], vol[stage_per<NT, CC, C>()];
-      stage_load<NT, C, CC>(wg_lo, vgl);
-      stage_load<NT, CC, C>(wo_lo, vol);
-      stage_store<NT, C, CC>(sWgl, LWG, vgl);
-      stage_store<NT, CC, C>(sWol, LWO, vol);
+      wgl.turn(wb, lane);
+      wol.turn(wb, lane);
+      c0 += direct_wbeta<KS>(wgl.v, lnb, h);
     }
-    stage_store<NT, C, CC>(sWg, LWG, vg);
-    stage_store<NT, CC, C>(sWo, LWO, vo);
-    if (tid < CC) gam[tid] = gv;
+    if (tile == 0 && h == 0) soff[32 * cb + m] = FAST ? c0 : -LOG2E * c0;
   }
-  __syncthreads();
-  for (int row = tid; row < C; row += 64 * TAO_WAVES) {   // gate offsets -log2(e) W_g beta (weights from LDS)
-    const op_t* w = sWg + row * LWG;
-    const op_t* wl = sWgl + row * LWG;
-    float acc = 0.f;
+  int buf = 0;
+  for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x, buf ^= 1) {
+    const PosTile pt = group(gi);
+    op_t* sxb = sx + buf * DP_ROWS * LW;
+    ln.store(sxb, eps, wid, lane);
+    const long zp = zpair(pt, 32 * tile + m);
+    const int oc = 32 * cb + 4 * h;   // + 8 g: this lane's output channels
+    f32x4 res[4];
 #pragma unroll
-    for (int c = 0; c < CC; c += 8) {
-      const opx4 wa = ld_x4(w + c), wb = ld_x4(w + c + 4);
-      const opx8 w8 = {wa[0], wa[1], wa[2], wa[3], wb[0], wb[1], wb[2], wb[3]};
+    for (int g = 0; g < 4; ++g)
+      res[g] = resid && has_out ? *reinterpret_cast<const f32x4*>((resid == 2 ? out : z_in) + zp * CC + oc + 8 * g)
+                                : f32x4{0.f, 0.f, 0.f, 0.f};
+    opx4 o4[4];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc += (float)w8[e] * lnb[c + e];
-      if constexpr (HILO) {
-        const opx4 la = ld_x4(wl + c), lb = ld_x4(wl + c + 4);
-        const opx8 l8 = {la[0], la[1], la[2], la[3], lb[0], lb[1], lb[2], lb[3]};
+    for (int g = 0; g < 4; ++g) o4[g] = ov[g];
+    __syncthreads();   // every z row of the group has been read (out may alias z_in)
+    if (gi + (int)gridDim.x < ngroups) fetch(gi + gridDim.x);
+    f32x16 g16 = zero16();
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc += (float)l8[e] * lnb[c + e];
-      }
+    for (int s = 0; s < KS; ++s) {
+      const opx8 xf = ld_x8(sxb + (32 * tile + m) * LW + 16 * s + 8 * h);
+      g16 = mfma32(wg.v[s], xf, g16);   // D[channel][position]
+      if constexpr (HILO) g16 = mfma32(wgl.v[s], xf, g16);
     }
-    cgate[row] = FAST ? acc : -LOG2E * acc;
-  }
-  __syncthreads();
-  const uint32_t ntiles = (uint32_t)B * N * N / 32;
-  const uint32_t stride = gridDim.x * TAO_WAVES;
-  uint32_t t = blockIdx.x * TAO_WAVES + wid;
-  for (; t < ntiles; t += stride) {
-    asm volatile("" ::: "memory");   // the gate offsets are re-read from LDS each tile, not pinned in VGPRs
-    const PosTile pt = pos_tile(t, N);
-    const int b = pt.b, ip = pt.r, j = pt.c0 + m;
-    const long zp = ending ? ((long)b * N + j) * N + ip : ((long)b * N + ip) * N + j;
-    opx8 xf[KS];
-    float zr[CC / 2];
-    load_row_oa<CC>(z_in + zp * CC, h, zr);
-    ln_oa_gamma_to_frag<CC>(zr, h, gam, eps, xf);
-    // o * sigmoid(g) as the B operand of the output projection (k order = output-aligned)
-    opx4 ov4[C / 8];   // O values (C = H * D channels): oa_channel(q, h) + 0..3 of position 32 t + m
+    if constexpr (FAST) {
 #pragma unroll
-    for (int q = 0; q < C / 8; ++q) ov4[q] = ld_x4(O + (32l * t + m) * C + oa_channel(q, h));
-    opx8 og[8];
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 cg = *reinterpret_cast<const f32x4*>(soff + 32 * cb + 8 * g + 4 * h);
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-      const op_t* wrow = &sWg[(32 * cb + m) * LWG];
-      f32x16 g = zero16();
-#pragma unroll
-      for (int s = 0; s < KS; ++s) g = mfma32(wfrag_oa(wrow, s, h), xf[s], g);   // D[channel][position]
-      if constexpr (HILO) {
-        const op_t* wlrow = &sWgl[(32 * cb + m) * LWG];
-#pragma unroll
-        for (int s = 0; s < KS; ++s) g = mfma32(wfrag_oa(wlrow, s, h), xf[s], g);
+        for (int e = 0; e < 4; ++e) g16[4 * g + e] += cg[e];
       }
-#pragma unroll
-      for (int gg = 0; gg < 4; ++gg) {
-        const int q = 4 * cb + gg;            // chunk: channels oa_channel(q, h) + 0..3
-        const opx4 ov = ov4[q];
-        const f32x4 cg = *reinterpret_cast<const f32x4*>(cgate + oa_channel(q, h));
-        if constexpr (FAST) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) g[4 * gg + e] += cg[e];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            og[q >> 1][4 * (q & 1) + e] =
-                (op_t)((float)ov[e] * rcp_fast(1.f + exp2_fast(fmaf(g[4 * gg + e], -LOG2E, cg[e]))));
-        }
-      }
-      if constexpr (FAST) {
-        mx_fake_quant16(g);
-#pragma unroll
-        for (int gg = 0; gg < 4; ++gg) {
-          const int q = 4 * cb + gg;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            og[q >> 1][4 * (q & 1) + e] =
-                (op_t)((float)ov4[q][e] * rcp_fast(1.f + exp2_fast(-LOG2E * g[4 * gg + e])));
-        }
-      }
+      mx_fake_quant16(g16);
     }
 #pragma unroll
-    for (int ob = 0; ob < CC / 32; ++ob) {
-      const op_t* wrow = &sWo[(32 * ob + m) * LWO];
+    for (int g = 0; g < 4; ++g) {
+      opx4 og;
+      const f32x4 cg = *reinterpret_cast<const f32x4*>(soff + 32 * cb + 8 * g + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float ex = FAST ? -LOG2E * g16[4 * g + e] : fmaf(g16[4 * g + e], -LOG2E, cg[e]);
+        og[e] = (op_t)((float)o4[g][e] * rcp_fast(1.f + exp2_fast(ex)));
+      }
+      st_x4(sog + (32 * tile + m) * LO_ + 32 * cb + 8 * g + 4 * h, og);
+    }
+    __syncthreads();
+    if (has_out) {
       f32x16 acc = zero16();
 #pragma unroll
-      for (int s = 0; s < 8; ++s) acc = mfma32(wfrag_oa(wrow, s, h), og[s], acc);   // D[out][position]
-      if constexpr (HILO) {
-        const op_t* wlrow = &sWol[(32 * ob + m) * LWO];
-#pragma unroll
-        for (int s = 0; s < 8; ++s) acc = mfma32(wfrag_oa(wlrow, s, h), og[s], acc);
+      for (int s = 0; s < C / 16; ++s) {
+        const opx8 of = ld_x8(sog + (32 * tile + m) * LO_ + 16 * s + 8 * h);
+        acc = mfma32(wo_.v[s], of, acc);   // D[out][position]
+        if constexpr (HILO) acc = mfma32(wol.v[s], of, acc);
       }
       if constexpr (FAST) mx_fake_quant16(acc);
 #pragma unroll
-      for (int gg = 0; gg < 4; ++gg) {
-        const int q = 4 * ob + gg;
-        float* dst = out + zp * CC + oa_channel(q, h);
+      for (int g = 0; g < 4; ++g) {
         f32x4 v;
-        if (resid == 1) v = f32x4{zr[4 * q], zr[4 * q + 1], zr[4 * q + 2], zr[4 * q + 3]};
-        if (resid == 2) v = *reinterpret_cast<const f32x4*>(dst);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = resid == 0 ? acc[4 * gg + e] : v[e] + acc[4 * gg + e];
-        *reinterpret_cast<f32x4*>(dst) = v;
+        for (int e = 0; e < 4; ++e) v[e] = res[g][e] + acc[4 * g + e];
+        *reinterpret_cast<f32x4*>(out + zp * CC + oc + 8 * g) = v;
       }
     }
   }
@@ -970,92 +996,58 @@ int launch_attn(const TaBuffers& t, float* o32, int B, int N, int n_valid, hipSt
   return PF_OK;
 }
 
-// e4m3 bytes q [rows][K] with E8M0 scale bytes s [rows][K / 32] (pf_quantize_mx8) -> op_t
-// values e4m3 * 2^(s - 127), exact in op_t for the weights' range; n % 4 == 0, K % 32 == 0.
-// A scale byte 0 (an all-zero block) gives zeros.
-__global__ void mx8_dequant_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__ s,
-                                   op_t* __restrict__ out, long n, int K) {
-  for (long e = 4 * ((long)blockIdx.x * blockDim.x + threadIdx.x); e < n; e += 4l * gridDim.x * blockDim.x) {
-    const int word = *reinterpret_cast<const int*>(q + e);
-    const long row = e / K;
-    const float X = __uint_as_float((uint32_t)s[row * (K / 32) + (e - row * K) / 32] << 23);
-    const auto lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(word, X, false);
-    const auto hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(word, X, true);
-    st_x4(out + e, opx4{(op_t)lo[0], (op_t)lo[1], (op_t)hi[0], (op_t)hi[1]});
-  }
-}
-
-// W_q, W_k, W_v, W_g as the kernels read them (op_t [C][CC]); the residuals of W_g and W_o
-// (op_t, or null).
-struct TaWeights { const op_t *q, *k, *v, *g, *g_lo = nullptr, *o_lo = nullptr; };
-
-// The mean correction of ta_proj's weights for a 16-bit call with the exact offsets and the
-// four folded-weight residuals, one batch element, c_z = 128 (else the plain W16 beta offsets).
-template <int CC, bool FAST>
-TaMeanFix ta_mean_fix(const pf_triatt_args* a, const TaBuffers& t, hipStream_t st, int* rc) {
-  TaMeanFix mf{nullptr, {nullptr, nullptr, nullptr, nullptr}, nullptr};
-  *rc = PF_OK;
-  if (FAST || CC != PS_C || !a->in_offsets) return mf;
-  mf.offb = a->in_offsets;
-  if (a->B == 1 && a->w_q_lo && a->w_k_lo && a->w_v_lo && a->w_bias_lo) {
-    mf.lo[0] = (const op_t*)a->w_q_lo; mf.lo[1] = (const op_t*)a->w_k_lo;
-    mf.lo[2] = (const op_t*)a->w_v_lo; mf.lo[3] = (const op_t*)a->w_bias_lo;
-    mf.stats = t.stats;
-    pair_stats_kernel<<<PS_WG, 64 * PS_WAVES, 0, st>>>(a->z_in, a->N, a->eps, t.stats);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) *rc = pf_fail(PF_E_LAUNCH, "pair_stats_kernel launch failed: %s", hipGetErrorString(e));
-  }
-  return mf;
-}
-
-template <int CC, bool FAST>
-int triatt_run(const pf_triatt_args* a, const TaWeights& w) {
+// The residuals of ta_proj's weights for a 16-bit call with the exact offsets and the four
+// folded-weight residuals, one batch element, c_z = 128 (else the plain W16): a second MFMA up to
+// four groups of 64 positions per CU when W_g and W_o come with theirs too, where the statistics
+// launch costs more (whole attention, us, against the weights in LDS it replaced: N = 64 48 -> 27,
+// 128 55 -> 37, 256 84 -> 81), else the mean correction (384 189 -> 168, 1024 1785 -> 1622).
+template <int CC, bool FAST, int LO>
+int triatt_run_lo(const pf_triatt_args* a, const TaWeights& w, const TaBuffers& t, const TaMeanFix& mf, int cus) {
   hipStream_t st = (hipStream_t)a->stream;
   const int B = a->B, N = a->N;
   const int n_valid = a->n_valid ? a->n_valid : N;
-  TaBuffers t = ta_buffers(a->workspace, B, N);
   const float qscale = LOG2E / sqrtf((float)D);
-  const long positions = (long)B * N * N;
-  const int cus = device_cus();
-  if (cus <= 0) return pf_fail(PF_E_LAUNCH, "pf_triatt_fwd: cannot query the device");
-  int mrc = PF_OK;
-  const TaMeanFix mf = ta_mean_fix<CC, FAST>(a, t, st, &mrc);
-  if (mrc) return mrc;
+  const int ngroups = (int)((long)B * N * N / DP_ROWS), grid = min(ngroups, cus);
   {
-    const void* fn = (const void*)ta_proj_kernel<CC, FAST>;
-    if (const int rc = pf_reserve_lds(fn, tap_lds<CC, FAST>(), "ta_proj_kernel")) return rc;
-    const int grid = (int)min((long)cus, (positions / 32 + TAP_WAVES - 1) / TAP_WAVES);
-    ta_proj_kernel<CC, FAST><<<grid, 64 * TAP_WAVES, tap_lds<CC, FAST>(), st>>>(
-        a->z_in, a->pair_mask, a->ln_w, a->ln_b, w.q, w.k, w.v, (const op_t*)a->w_bias, t.Q, t.K, t.Vt, t.bias32,
-        t.mask16, B, N, n_valid, a->ending, qscale, a->eps, mf);
+    auto kern = ta_proj_kernel<CC, FAST, LO>;
+    if (const int rc = pf_reserve_lds((const void*)kern, tap_lds<CC>(), "ta_proj_kernel")) return rc;
+    kern<<<grid, 64 * TAP_WAVES, tap_lds<CC>(), st>>>(a->z_in, a->pair_mask, a->ln_w, a->ln_b, w,
+                                                      (const op_t*)a->w_bias, t.Q, t.K, t.Vt, t.bias32, t.mask16,
+                                                      ngroups, N, n_valid, a->ending, qscale, a->eps, mf);
     PF_CHECK_LAUNCH("ta_proj_kernel");
   }
   int rc = launch_attn<false>(t, nullptr, B, N, n_valid, st);
   if (rc) return rc;
-  {
-    const int grid = (int)min((long)cus, (positions / 32 + TAO_WAVES - 1) / TAO_WAVES);
-    const int resid = !a->accumulate ? 0 : (a->out == a->z_in ? 1 : 2);
-    bool hilo = false;
-    if constexpr (!FAST && CC == 128) {   // the residual weights exist for the 16-bit c_z = 128 path
-      if (w.g_lo && w.o_lo) {
-        hilo = true;
-        const void* fn = (const void*)ta_out_kernel<CC, FAST, true>;
-        if (const int rc = pf_reserve_lds(fn, tao_lds<CC, true>(), "ta_out_kernel")) return rc;
-        ta_out_kernel<CC, FAST, true><<<grid, 64 * TAO_WAVES, tao_lds<CC, true>(), st>>>(
-            t.O, a->z_in, a->out, a->ln_w, a->ln_b, w.g, (const op_t*)a->w_o, w.g_lo, w.o_lo, B, N, a->ending, resid,
-            a->eps);
-      }
-    }
-    if (!hilo) {
-      const void* fn = (const void*)ta_out_kernel<CC, FAST>;
-      if (const int rc = pf_reserve_lds(fn, tao_lds<CC>(), "ta_out_kernel")) return rc;
-      ta_out_kernel<CC, FAST><<<grid, 64 * TAO_WAVES, tao_lds<CC>(), st>>>(
-          t.O, a->z_in, a->out, a->ln_w, a->ln_b, w.g, (const op_t*)a->w_o, nullptr, nullptr, B, N, a->ending,
-          resid, a->eps);
-    }
-    PF_CHECK_LAUNCH("ta_out_kernel");
-  }
+  const int resid = !a->accumulate ? 0 : (a->out == a->z_in ? 1 : 2);
+  constexpr bool CAN_HILO = !FAST && CC == 128;   // the residual weights exist for the 16-bit c_z = 128 path
+  auto kern = CAN_HILO && w.g_lo && w.o_lo ? ta_out_kernel<CC, FAST, CAN_HILO> : ta_out_kernel<CC, FAST, false>;
+  if (const int rc = pf_reserve_lds((const void*)kern, tao_lds<CC>(), "ta_out_kernel")) return rc;
+  kern<<<grid, 64 * TAO_WAVES, tao_lds<CC>(), st>>>(t.O, a->z_in, a->out, a->ln_w, a->ln_b, w, (const op_t*)a->w_o,
+                                                    ngroups, N, a->ending, resid, a->eps);
+  PF_CHECK_LAUNCH("ta_out_kernel");
   return PF_OK;
+}
+
+template <int CC, bool FAST>
+int triatt_run(const pf_triatt_args* a, const TaWeights& w) {
+  const TaBuffers t = ta_buffers(a->workspace, a->B, a->N);
+  const int cus = device_cus();
+  if (cus <= 0) return pf_fail(PF_E_LAUNCH, "pf_triatt_fwd: cannot query the device");
+  TaMeanFix mf{nullptr, {nullptr, nullptr, nullptr, nullptr}, nullptr};
+  if constexpr (!FAST && CC == PS_C) {
+    mf.offb = a->in_offsets;
+    if (a->in_offsets && a->B == 1 && a->w_q_lo && a->w_k_lo && a->w_v_lo && a->w_bias_lo) {
+      mf.lo[0] = (const op_t*)a->w_q_lo; mf.lo[1] = (const op_t*)a->w_k_lo;
+      mf.lo[2] = (const op_t*)a->w_v_lo; mf.lo[3] = (const op_t*)a->w_bias_lo;
+      if (w.g_lo && w.o_lo && (long)a->N * a->N / DP_ROWS <= 4l * cus)
+        return triatt_run_lo<CC, FAST, DL_MFMA>(a, w, t, mf, cus);
+      mf.stats = t.stats;
+      pair_stats_kernel<<<PS_WG, 64 * PS_WAVES, 0, (hipStream_t)a->stream>>>(a->z_in, a->N, a->eps, t.stats);
+      PF_CHECK_LAUNCH("pair_stats_kernel");
+      return triatt_run_lo<CC, FAST, DL_MEAN>(a, w, t, mf, cus);
+    }
+  }
+  return triatt_run_lo<CC, FAST, DL_NONE>(a, w, t, mf, cus);
 }
 
 // The attention kernel addresses a batch's bias ([H][N][N] fp32) through one raw buffer
@@ -1099,12 +1091,13 @@ extern "C" int pf_triatt_fwd(const pf_triatt_args* a) {
       return pf_fail(PF_E_INVALID, "pf_triatt_fwd: the mean correction needs in_offsets and all four residuals "
                                    "(w_q_lo, w_k_lo, w_v_lo, w_bias_lo)");
   }
-  const TaWeights w = {(const op_t*)a->w_q, (const op_t*)a->w_k, (const op_t*)a->w_v, (const op_t*)a->w_g,
-                       (const op_t*)a->w_g_lo, (const op_t*)a->w_o_lo};
+  TaWeights w = {{a->w_q, a->w_k, a->w_v, a->w_g}};
+  w.g_lo = (const op_t*)a->w_g_lo;
+  w.o_lo = (const op_t*)a->w_o_lo;
   return a->C == 128 ? triatt_run<128, false>(a, w) : triatt_run<64, false>(a, w);
 }
 
-// Fast mode: the 16-bit workspace, then W_q, W_k, W_v, W_g dequantized to op_t [4][C][C].
+// Fast mode: the 16-bit workspace (the size keeps 4 C^2 op_t more, part of the interface).
 extern "C" size_t pf_triatt_mx8_workspace_size(int B, int N, int C_, int H_, int D_) {
   if (B <= 0 || N <= 0 || C_ != 128 || H_ != H || D_ != D) return 0;
   return ta_buffers_size(B, N) + 4 * (size_t)C * C * sizeof(op_t);
@@ -1128,21 +1121,13 @@ extern "C" int pf_triatt_mx8_fwd(const pf_triatt_mx8_args* m) {
     return pf_fail(PF_E_INVALID, "pf_triatt_mx8_fwd: workspace too small (%zu < %zu bytes)", m->workspace_bytes, need);
   if (m->n_valid < 0 || m->n_valid > m->N)
     return pf_fail(PF_E_INVALID, "pf_triatt_mx8_fwd: n_valid %d outside [0, N=%d]", m->n_valid, m->N);
-  hipStream_t st = (hipStream_t)m->stream;
-  op_t* wd = reinterpret_cast<op_t*>((char*)m->workspace + ta_buffers_size(m->B, m->N));
-  const void* src[4][2] = {{m->w_q_q, m->w_q_s}, {m->w_k_q, m->w_k_s}, {m->w_v_q, m->w_v_s}, {m->w_g_q, m->w_g_s}};
-  for (int i = 0; i < 4; ++i) {
-    mx8_dequant_kernel<<<16, 256, 0, st>>>((const uint8_t*)src[i][0], (const uint8_t*)src[i][1], wd + i * C * C,
-                                          (long)C * C, C);
-    PF_CHECK_LAUNCH("mx8_dequant_kernel");
-  }
   pf_triatt_args a = {};
   a.B = m->B; a.N = m->N; a.C = m->C; a.H = m->H; a.D = m->D;
   a.ending = m->ending; a.accumulate = m->accumulate; a.n_valid = m->n_valid; a.eps = m->eps;
   a.z_in = m->z_in; a.out = m->out; a.pair_mask = m->pair_mask; a.ln_w = m->ln_w; a.ln_b = m->ln_b;
   a.w_bias = m->w_bias; a.w_o = m->w_o;
   a.workspace = m->workspace; a.workspace_bytes = m->workspace_bytes; a.stream = m->stream;
-  const TaWeights w = {wd, wd + C * C, wd + 2 * C * C, wd + 3 * C * C};
+  const TaWeights w = {{m->w_q_q, m->w_k_q, m->w_v_q, m->w_g_q}, {m->w_q_s, m->w_k_s, m->w_v_s, m->w_g_s}};
   return triatt_run<128, true>(&a, w);
 }
 

@@ -136,7 +136,7 @@ class Options:
     The pair transition's fc3 then takes its residual the same way, (W - W16) . mean(h) over the
     hidden activations of sampled positions, instead of as the hi + lo product (default on;
     c_z = 128, batch 1).  On small grids (N <= 256), with ``weight_residuals`` also on, the triangle
-    multiplication multiplies by these residuals as well instead, which is exact and faster there."""
+    operators multiply by these residuals as well instead, which is exact and faster there."""
 
     def __init__(self, eps: float = 1e-5, operand: str = ops.DEFAULT_VARIANT, overlap_single: bool = True,
                  single_delay: int = 1, weight_residuals: bool = True, mean_correction: bool = True):
