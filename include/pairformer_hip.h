@@ -496,6 +496,14 @@ int pf_token_pair_bias_fwd(const float* z, const float* ln_w, const float* ln_b,
  *   out[i] = a[i] + b[i], fp32, 16-byte aligned pointers; out may alias a or b. */
 int pf_add_fwd(const float* a, const float* b, float* out, long n, void* stream);
 
+/* Zero-padded copy (the boundary's pad to a multiple of 64 or 128 tokens):
+ *   dst[b, i, m, j, c] = src[b, i, m, j, c] for i < N1 and j < N2, else 0,  dst fp32
+ * [B][n1p][M][n2p][C]; src fp32 with element strides sb, s1, sm, s2 for b, i, m, j and contiguous
+ * channels, or NULL: ones in its place.  Fewer than 2^32 elements (2^34 where 16-byte accesses are
+ * possible); dst must not overlap src. */
+int pf_pad_fwd(const float* src, long sb, long s1, long sm, long s2, float* dst, int B, int N1, int M, int N2,
+               int n1p, int n2p, int C, void* stream);
+
 /* ------------------------------------------------------------------------------
  * Measurement aids (no counterpart in the reference: they serve the benchmark's roofline
  * figures and allocate no device memory).

@@ -108,3 +108,33 @@ def test_triatt_direct(gpu, B, N, ending, plain):
     mod(inplace, pd, out=inplace, accumulate=True, n_valid=n)
     # the same update added to z: one fp32 rounding of the sum apart
     assert (inplace - (zd + update)).abs().max() <= 2.0 ** -22 * (zd.abs().max() + update.abs().max())
+
+
+# ------------------------------------------------------------------------------ boundary padding
+@pytest.mark.parametrize("N,n_pad", [(1, 64), (45, 64), (64, 64), (130, 192)])
+@pytest.mark.parametrize("form", ["plain", "transposed", "sliced", "offset", "expanded", "half", "grad"])
+@pytest.mark.parametrize("shape,dims", [("BNNC", (1, 2)), ("BNC", (1,)), ("BNHND", (1, 3)), ("BNN", (1, 2)),
+                                        ("BSN", (2,)), ("BN", (1,))])
+def test_padded(gpu, N, n_pad, form, shape, dims):
+    """The padding kernel against a fill and a copy, exactly: every layout it takes (strides,
+    misaligned data, one channel, an odd channel count, nothing to pad) and what is left to torch."""
+    size = [{"B": 2, "N": N, "C": 20, "H": 3, "D": 5, "S": 7}[c] for c in shape]
+    g = torch.Generator(device=gpu).manual_seed(N)
+    x = torch.randn(size, generator=g, device=gpu)
+    if form == "transposed":
+        d = 2 if len(size) > 2 else 1
+        x = x.transpose(d - 1, d).contiguous().transpose(d - 1, d)
+    elif form == "sliced":
+        x = torch.randn([n + 3 for n in size], generator=g, device=gpu)[tuple(slice(2, 2 + n) for n in size)]
+    elif form == "offset":
+        x = torch.randn(x.numel() + 1, generator=g, device=gpu)[1:].view(size)
+    elif form == "expanded":
+        x = x[:1].expand(size)
+    elif form == "half":
+        x = x.half()
+    elif form == "grad":
+        x.requires_grad_(True)
+    got = ops.padded(x, n_pad, x.device, dims)
+    want = torch.zeros([n_pad if d in dims else n for d, n in enumerate(size)], device=gpu)
+    want[tuple(slice(0, n) for n in size)] = x.detach().float()
+    assert got.is_contiguous() and got.dtype == torch.float32 and torch.equal(got, want)

@@ -161,6 +161,8 @@ SIGNATURES = {
     "pf_pair_ln_linear_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                       c_long, c_int, c_float, c_void_p]),
     "pf_add_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_long, c_void_p]),
+    "pf_pad_fwd": (c_int, [c_void_p, c_long, c_long, c_long, c_long, c_void_p, c_int, c_int, c_int, c_int, c_int,
+                           c_int, c_int, c_void_p]),
     "pf_pair_cond_proj_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_int,
                                       c_float, c_void_p]),
     "pf_token_pair_bias_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int,

@@ -18,7 +18,7 @@ INCLUDE = os.path.join(ROOT, "include")
 OBJDIR = os.path.join(HERE, "_build")
 
 SOURCES = ["api.cpp", "trimul.hip", "triatt.hip", "transition.hip", "single.hip", "fast8.hip", "msa.hip", "diffusion.hip",
-           "measure.hip"]
+           "pad.hip", "measure.hip"]
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

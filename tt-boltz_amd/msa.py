@@ -135,13 +135,14 @@ def device_inputs(emb: torch.Tensor, feats: Mapping[str, torch.Tensor], n_pad: i
     B, S, N = feats["msa"].shape
 
     def per_row(key, dtype):
+        x = feats[key].to(device, dtype)
+        if dtype == torch.float32 and tuple(x.shape) == (B, S, N):
+            return ops.padded(x, n_pad, device, (2,))
         t = torch.zeros((B, S, n_pad), dtype=dtype, device=device)
-        t[:, :, :N] = feats[key].to(device, dtype)
+        t[:, :, :N] = x
         return t
 
-    emb_dev = torch.zeros((B, n_pad, emb.shape[-1]), dtype=torch.float32, device=device)
-    emb_dev[:, :N] = emb.to(device, torch.float32)
-    return {"emb": emb_dev, "msa": per_row("msa", torch.int32), "has_deletion": per_row("has_deletion", torch.float32),
+    return {"emb": ops.padded(emb.to(device, torch.float32), n_pad, device, (1,)), "msa": per_row("msa", torch.int32), "has_deletion": per_row("has_deletion", torch.float32),
             "deletion_value": per_row("deletion_value", torch.float32),
             "msa_paired": per_row("msa_paired", torch.float32), "msa_mask": per_row("msa_mask", torch.float32)}
 

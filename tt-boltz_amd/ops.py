@@ -117,12 +117,49 @@ def padded_len(n: int, pad: int = PAD) -> int:
     return -(-n // pad) * pad
 
 
+def _pads_on_device(x: torch.Tensor, device: torch.device) -> bool:
+    """Whether ``pf_pad_fwd`` can read ``x`` in place of a fill and a copy on ``device``."""
+    return (x.dtype == torch.float32 and x.device == device and x.is_cuda
+            and type(x) in (torch.Tensor, torch.nn.Parameter)
+            and device == torch.device("cuda", torch.cuda.current_device())
+            and not (x.requires_grad and torch.is_grad_enabled()) and not x.is_neg() and x.numel() > 0
+            and x.stride(-1) == 1)
+
+
+def padded(x: torch.Tensor, n_pad: int, device: torch.device, dims: tuple) -> torch.Tensor:
+    """New contiguous fp32 tensor on ``device``: ``x`` with the dimensions in ``dims`` zero-padded to
+    ``n_pad``.  ``dims`` is (1, 2) for [B,N,N,C], (1,) for [B,N,C], (1, 3) for [B,N,H,N,D] and for
+    masks, which have no channels, (1, 2) of [B,N,N], (2,) of [B,S,N] and (1,) of [B,N]."""
+    shape = [n_pad if d in dims else n for d, n in enumerate(x.shape)]
+    total = 1
+    for n in shape:
+        total *= n
+    if _pads_on_device(x, device) and total < (1 << 32) - 4096:
+        out = torch.empty(shape, dtype=torch.float32, device=device)
+        # (batch, first padded, between, second padded or plain, channels) and their strides
+        n, st = list(x.shape), list(x.stride())
+        if len(n) == dims[-1] + 1:   # a mask: one channel
+            n.append(1)
+            st.append(1)
+        if dims == (1,):
+            n, st, np_ = [n[0], 1, 1, n[1], n[2]], [st[0], 0, 0, st[1]], (1, n_pad)
+        elif dims == (2,):
+            n, st, np_ = [n[0], n[1], 1, n[2], n[3]], [st[0], st[1], 0, st[2]], (n[1], n_pad)
+        elif dims == (1, 2):
+            n, st, np_ = [n[0], n[1], 1, n[2], n[3]], [st[0], st[1], 0, st[2]], (n_pad, n_pad)
+        else:
+            np_ = (n_pad, n_pad)
+        _lib.check(_lib.load().pf_pad_fwd(x.data_ptr(), *st[:4], out.data_ptr(), n[0], n[1], n[2], n[3], *np_, n[4],
+                                          _stream()), "pf_pad_fwd")
+        return out
+    out = torch.zeros(shape, dtype=torch.float32, device=device)
+    out[tuple(slice(0, x.shape[d]) for d in range(x.dim()))].copy_(x)
+    return out
+
+
 def pad_pair(z: torch.Tensor, n_pad: int) -> torch.Tensor:
     """Zero-pad [B,N,N,C] to [B,n_pad,n_pad,C] (always returns a new contiguous fp32 tensor)."""
-    B, N, _, C = z.shape
-    out = torch.zeros((B, n_pad, n_pad, C), dtype=torch.float32, device=z.device)
-    out[:, :N, :N] = z
-    return out
+    return padded(z, n_pad, z.device, (1, 2))
 
 
 #: row chunks of a host -> device pair copy: the host copy of one chunk into pinned memory
@@ -136,12 +173,11 @@ def to_device_padded(x: torch.Tensor, n_pad: int, device: torch.device, pair: bo
     caching host allocator) in row chunks with asynchronous DMA, so the host copy of a
     chunk overlaps the transfer of the previous one; a device tensor is padded in place."""
     B, N = x.shape[0], x.shape[1]
+    if x.device.type != "cpu":
+        return padded(x, n_pad, device, (1, 2) if pair else (1,))
     shape = (B, n_pad, n_pad, x.shape[-1]) if pair else (B, n_pad, x.shape[-1])
     out = torch.zeros(shape, dtype=torch.float32, device=device)
     dst = out[:, :N, :N] if pair else out[:, :N]
-    if x.device.type != "cpu":
-        dst.copy_(x)
-        return out
     xf = x if x.dtype == torch.float32 else x.float()
     if xf.is_pinned():
         dst.copy_(xf, non_blocking=True)
@@ -176,6 +212,8 @@ def pad_pair_mask(pair_mask: Optional[torch.Tensor], B: int, N: int, n_pad: int,
     """[B,N,N] 0/1 mask padded with zeros; None when no masking is needed."""
     if pair_mask is None and n_pad == N:
         return None
+    if pair_mask is not None and tuple(pair_mask.shape) == (B, N, N):
+        return padded(pair_mask.to(device=device, dtype=torch.float32), n_pad, device, (1, 2))
     out = torch.zeros((B, n_pad, n_pad), dtype=torch.float32, device=device)
     out[:, :N, :N] = 1.0 if pair_mask is None else pair_mask.to(device=device, dtype=torch.float32)
     return out
@@ -601,21 +639,15 @@ def triangle_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bias: 
 
     def padq(t):
         t = t.to(torch.float32)
-        if n_pad == N:
-            return t.contiguous()
-        o = torch.zeros((B, n_pad, H, n_pad, D), dtype=torch.float32, device=dev)
-        o[:, :N, :, :N] = t
-        return o
+        return t.contiguous() if n_pad == N else padded(t, n_pad, dev, (1, 3))
 
     qp, kp, vp = padq(q), padq(k), padq(v)
     if n_pad == N:   # no padding: the caller's bias and mask as they are (fp32, contiguous)
         bp = bias.reshape(B, H, N, N).to(torch.float32).contiguous()
         mp = None if mask is None else mask.reshape(B, N, N).to(torch.float32).contiguous()
     else:
-        bp = torch.zeros((B, H, n_pad, n_pad), dtype=torch.float32, device=dev)
-        bp[:, :, :N, :N] = bias.reshape(B, H, N, N)
-        mp = torch.zeros((B, n_pad, n_pad), dtype=torch.float32, device=dev)
-        mp[:, :N, :N] = 1.0 if mask is None else mask.reshape(B, N, N).to(torch.float32)
+        bp = padded(bias.reshape(B * H, N, N).to(torch.float32), n_pad, dev, (1, 2))
+        mp = pad_pair_mask(None if mask is None else mask.reshape(B, N, N), B, N, n_pad, dev)
     o = torch.empty((B, n_pad, H, n_pad, D), dtype=torch.float32, device=dev)
     lib = _lib.load(variant)
     ws = workspace(lib.pf_tri_attention_workspace_size(B, n_pad, H, D), dev)
@@ -651,13 +683,14 @@ def attention_pair_bias(s: torch.Tensor, z: torch.Tensor, mask: Optional[torch.T
     def pad_tokens(t):   # [B, N, c] -> [B, n_pad, c] fp32; read-only, so no copy when N needs no padding
         if n_pad == N:
             return t.to(torch.float32).contiguous()
-        o = torch.zeros((B, n_pad) + tuple(t.shape[2:]), dtype=torch.float32, device=dev)
-        o[:, :N] = t
-        return o
-    sp, kp = pad_tokens(s), pad_tokens(k_in)
+        return padded(t.to(torch.float32), n_pad, dev, (1,))
+    sp = pad_tokens(s)
+    kp = sp if k_in is s else pad_tokens(k_in)   # both are only read
     zp = pad_pair(z.to(torch.float32), n_pad) if n_pad != N else z.to(torch.float32).contiguous()
     if mask is not None and n_pad == N:
         mp = mask.to(device=dev, dtype=torch.float32).contiguous()
+    elif mask is not None and tuple(mask.shape) == (B, N):
+        mp = padded(mask.to(device=dev, dtype=torch.float32), n_pad, dev, (1,))
     else:
         mp = torch.zeros((B, n_pad), dtype=torch.float32, device=dev)
         mp[:, :N] = 1.0 if mask is None else mask.to(torch.float32)
