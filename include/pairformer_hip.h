@@ -240,6 +240,10 @@ typedef struct pf_apb_args {
 size_t pf_apb_workspace_size(int B, int N, int c_s, int H);
 int pf_apb_fwd(const pf_apb_args* args);
 
+/* pf_apb_fwd (fast != 0: pf_apb_fwd_mx8) on a pair tensor that is not padded: z is
+ * [B][z_n][z_n][C] with n_valid <= z_n <= N; everything else as there. */
+int pf_apb_fwd_unpadded(const pf_apb_args* args, int z_n, int fast);
+
 /* pf_apb_fwd in two halves, for callers that overlap the single track with the next
  * layer's pair operations on a second stream: pf_apb_pair_bias computes the z-dependent
  * part (bias = proj_z.1(LN(z)), tt_bio/boltz2.py:353-356) into the workspace, and

@@ -138,3 +138,28 @@ def test_padded(gpu, N, n_pad, form, shape, dims):
     want = torch.zeros([n_pad if d in dims else n for d, n in enumerate(size)], device=gpu)
     want[tuple(slice(0, n) for n in size)] = x.detach().float()
     assert got.is_contiguous() and got.dtype == torch.float32 and torch.equal(got, want)
+
+
+# ------------------------------------------------------------------------------ single track
+@pytest.mark.parametrize("B,N", [(1, 33), (1, 64), (2, 100), (1, 413)])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("fast", [False, True])
+def test_attention_pair_bias_unpadded(gpu, B, N, masked, fast):
+    """The pair bias read from an unpadded z (odd row lengths, a batch) against the same call on a
+    padded z: identical bits."""
+    w = {k: v for k, v in _sub_w(9, "attention").items()}
+    g = torch.Generator().manual_seed(N)
+    s, z = torch.randn((B, N, 384), generator=g).to(gpu), torch.randn((B, N, N, 128), generator=g).to(gpu)
+    mask = (torch.rand((B, N), generator=g) > 0.2).float().to(gpu) if masked else None
+    got = ops.attention_pair_bias(s, z, mask, s, w, fast=fast)
+    n_pad = ops.padded_len(N)
+    sp, zp = ops.padded(s, n_pad, s.device, (1,)), ops.pad_pair(z, n_pad)
+    mp = torch.zeros((B, n_pad), device=gpu)
+    mp[:, :N] = 1.0 if mask is None else mask
+    ws = ops.workspace(ops.apb_workspace_bytes(B, n_pad, 384, 16), gpu)
+    out = torch.empty_like(sp)
+    ops.launch_apb(sp, sp, zp, mp, out, ops.convert_weights(w, gpu), 16, ws, accumulate=False, n_valid=N, fast=fast)
+    assert torch.equal(got, out[:, :N])
+    if not fast:
+        check("attention_pair_bias", got, ref.attention_pair_bias(s.cpu(), z.cpu(), torch.ones((B, N)) if mask is None
+                                                                  else mask.cpu(), s.cpu(), w))

@@ -142,6 +142,7 @@ SIGNATURES = {
     "pf_transition_fwd": (c_int, [ctypes.POINTER(TransitionArgs)]),
     "pf_apb_workspace_size": (c_size_t, [c_int, c_int, c_int, c_int]),
     "pf_apb_fwd": (c_int, [ctypes.POINTER(ApbArgs)]),
+    "pf_apb_fwd_unpadded": (c_int, [ctypes.POINTER(ApbArgs), c_int, c_int]),
     "pf_apb_pair_bias": (c_int, [ctypes.POINTER(ApbArgs)]),
     "pf_apb_attend": (c_int, [ctypes.POINTER(ApbArgs)]),
     "pf_apb_fwd_noalloc": (c_int, [ctypes.POINTER(ApbArgs)]),

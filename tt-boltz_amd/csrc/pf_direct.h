@@ -136,6 +136,59 @@ struct DirectW8 {
   }
 };
 
+// A wave's own tile of 32 rows of 128 channels: read fully coalesced (16 lanes a row, as DirectLn),
+// normalized with the affine part, and turned through the wave's own LDS rows of 136 op_t into the
+// 8 MFMA fragments (row lane & 31).  The next tile's loads run beside this tile's use.  No barriers.
+struct DirectTile {
+  f32x4 x[8][2], gm[2], bt[2];
+  template <class RowOf>
+  PF_DEV void load(const float* __restrict__ z, RowOf row_of, int lane) {   // row_of(r): row r of the tile
+    const int g = lane >> 4, q = lane & 15;
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {
+      const float* p = z + row_of(4 * it + g) * 128 + 4 * q;
+      x[it][0] = *reinterpret_cast<const f32x4*>(p);
+      x[it][1] = *reinterpret_cast<const f32x4*>(p + 64);
+    }
+  }
+  PF_DEV void affine(const float* __restrict__ gamma, const float* __restrict__ beta, int lane) {   // null: none
+    const int q = lane & 15;
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      gm[v] = gamma ? *reinterpret_cast<const f32x4*>(gamma + 64 * v + 4 * q) : f32x4{1.f, 1.f, 1.f, 1.f};
+      bt[v] = beta ? *reinterpret_cast<const f32x4*>(beta + 64 * v + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  PF_DEV void normalize(op_t* buf, float eps, int lane) const {
+    const int g = lane >> 4, q = lane & 15;
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {
+      const f32x4 a = x[it][0], b = x[it][1];
+      const float mean = row16_sum((a[0] + a[1]) + (a[2] + a[3]) + (b[0] + b[1]) + (b[2] + b[3])) * (1.f / 128.f);
+      float var = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float d = a[e] - mean, f = b[e] - mean;
+        var += d * d + f * f;
+      }
+      const float rstd = rsqrtf(row16_sum(var) * (1.f / 128.f) + eps);
+      opx4 o0, o1;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o0[e] = (op_t)((a[e] - mean) * rstd * gm[0][e] + bt[0][e]);
+        o1[e] = (op_t)((b[e] - mean) * rstd * gm[1][e] + bt[1][e]);
+      }
+      op_t* row = buf + (4 * it + g) * 136 + 4 * q;
+      st_x4(row, o0);
+      st_x4(row + 64, o1);
+    }
+  }
+  static PF_DEV void fragments(const op_t* buf, int lane, opx8 (&f)[8]) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) f[s] = ld_x8(buf + (lane & 31) * 136 + 16 * s + 8 * (lane >> 5));
+  }
+};
+
 // How a direct kernel uses the rounding residuals of its weights: not at all, as a second MFMA per
 // fragment, or through the mean correction (pair_stats_kernel) in the rows' offsets.
 enum DirectLo { DL_NONE = 0, DL_MFMA = 1, DL_MEAN = 2 };

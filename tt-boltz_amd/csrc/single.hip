@@ -16,41 +16,60 @@
 #include <mutex>
 
 #include "pf_common.h"
+#include "pf_direct.h"
 #include "pf_internal.h"
 
 namespace {
 
-constexpr int C = 128, LDSW = 136;
+constexpr int C = 128;
 
-// One wave = 32 pairs; W_z [H][128] (H <= 32) zero-padded to 32 rows in LDS.
-__global__ __launch_bounds__(256) void apb_zbias_kernel(
+// Persistent; every wave walks tiles of 32 pairs of its own (DirectTile), the heads' weight rows
+// (H <= 32, repeated past H) in registers as MFMA fragments: bound by reading z.  z may be smaller
+// than the bias grid: [B][NZ][NZ][128] with NZ <= N; the bias of pairs past it repeats the last row's
+// or column's (they are padding).  With lanes reading
+// a row each and W_z in LDS this took 27.9 us on the padded grid of N = 413 (z padded first: 31 us
+// more); 22.7 now.
+constexpr int ZB_WAVES = 8;
+__global__ __launch_bounds__(64 * ZB_WAVES, 1) void apb_zbias_kernel(
     const float* __restrict__ z, const float* __restrict__ lnw, const float* __restrict__ lnb,
-    const op_t* __restrict__ wz, float* __restrict__ bias, int B, int N, int H, float eps) {
-  __shared__ __attribute__((aligned(16))) op_t sW[32 * LDSW];
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, h = lane >> 5, m = lane & 31;
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int c = tid + 256 * q;
-    const int row = c >> 4;
-    st_x8(&sW[row * LDSW + (c & 15) * 8], row < H ? ld_x8(wz + row * C + (c & 15) * 8) : zero_x8());
-  }
-  __syncthreads();
+    const op_t* __restrict__ wz, float* __restrict__ bias, int B, int N, int NZ, int H, float eps) {
+  __shared__ __attribute__((aligned(16))) op_t tbuf[ZB_WAVES][32 * 136];
+  const int lane = threadIdx.x & 63, h = lane >> 5, m = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  op_t* buf = tbuf[wid];
   const long NN = (long)N * N;
-  const long pos0 = ((long)blockIdx.x * 4 + wid) * 32;
-  if (pos0 >= (long)B * NN) return;
-  const int b = (int)(pos0 / NN);
-  const long t0 = pos0 - (long)b * NN;   // i*N + j of position 0
-  float x[64];
-  opx8 xf[8];
-  load_row128_frag(z + (pos0 + m) * C, h, x);
-  ln128_to_frag(x, h, lnw, lnb, eps, xf);
-  f32x16 acc = zero16();
+  const uint32_t ntiles = (uint32_t)((long)B * NN / 32), stride = gridDim.x * ZB_WAVES;
+  uint32_t t = blockIdx.x * ZB_WAVES + wid;
+  if (t >= ntiles) return;   // (no barrier below)
+  DirectTile x;
+  auto fetch = [&](uint32_t k) PF_INLINE {
+    const PosTile pt = pos_tile(k, N);
+    const long row0 = ((long)pt.b * NZ + min(pt.r, NZ - 1)) * NZ;
+    x.load(z, [&](int r) PF_INLINE -> long { return row0 + min(pt.c0 + r, NZ - 1); }, lane);
+  };
+  fetch(t);
+  x.affine(lnw, lnb, lane);
+  opx8 w[8];
+  {
+    const op_t* wr = wz + min(m, H - 1) * C + 8 * h;
 #pragma unroll
-  for (int s = 0; s < 8; ++s) acc = mfma32(ld_x8(&sW[m * LDSW + 16 * s + 8 * h]), xf[s], acc);
+    for (int s = 0; s < 8; ++s) w[s] = ld_x8(wr + 16 * s);
+  }
+  for (; t < ntiles; t += stride) {
+    x.normalize(buf, eps, lane);
+    if (t + stride < ntiles) fetch(t + stride);
+    opx8 xf[8];
+    DirectTile::fragments(buf, lane, xf);
+    f32x16 acc = zero16();
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int hd = acc_row(r, h);
-    if (hd < H) bias[((long)b * H + hd) * NN + t0 + m] = acc[r] * 1.4426950408889634f;
+    for (int s = 0; s < 8; ++s) acc = mfma32(w[s], xf[s], acc);   // D[head][pair]
+    const PosTile pt = pos_tile(t, N);
+    float* dst = bias + (long)pt.b * H * NN + (long)pt.r * N + pt.c0 + m;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int hd = acc_row(r, h);
+      if (hd < H) dst[(long)hd * NN] = acc[r] * 1.4426950408889634f;
+    }
   }
 }
 
@@ -61,10 +80,27 @@ __global__ __launch_bounds__(256) void apb_zbias_kernel(
 // zero-padded to 32), in log2 units (Q pre-scaled by log2(e)/sqrt(DH), the bias stored
 // in log2 units); fp32 online softmax per query (a lane owns one query; its two halves
 // hold 16 keys each and meet in one exchange); O^T += V^T P^T (MFMA, P rounded to op_t);
-// the merged output is normalized and gated by sigmoid(g).  V^T
+// the merged output is normalized and gated by sigmoid(g).  Bound by memory round trips (13 key
+// tiles over 8 waves at N = 413): all loads of a tile are issued together, 16 bytes each (22.8 ->
+// 9.8 us there).  V^T
 // fragments are gathered straight from the fp32 rows: the 32 lanes of a half read 32
 // consecutive floats of one key row.
 constexpr int APB_SPLIT = 8;
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // the caller's mask: any alignment
+// d = d0 .. d0 + 7 of a head's row of DH floats (16-byte aligned), times sc; zero past DH
+template <int DH>
+PF_DEV opx8 apb_frag(const float* __restrict__ row, int d0, float sc) {
+  static_assert(DH % 8 == 0, "whole runs of 8");
+  const float* p = row + min(d0, DH - 8);
+  const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+  opx8 f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    f[e] = (op_t)(d0 < DH ? a[e] * sc : 0.f);
+    f[4 + e] = (op_t)(d0 < DH ? b[e] * sc : 0.f);
+  }
+  return f;
+}
 template <int DH>
 __global__ __launch_bounds__(64 * APB_SPLIT) void apb_attn_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
@@ -88,46 +124,43 @@ __global__ __launch_bounds__(64 * APB_SPLIT) void apb_attn_kernel(
   {
     const float* qr = q + (rowb + i0 + m) * c_s + hd * DH;
 #pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int d = 16 * s2 + 8 * h + t;
-        qf[s2][t] = (op_t)(d < DH ? qr[min(d, DH - 1)] * qs : 0.f);
-      }
+    for (int s2 = 0; s2 < 2; ++s2) qf[s2] = apb_frag<DH>(qr, 16 * s2 + 8 * h, qs);
   }
   const float* br = bias + (((long)b * H + hd) * N + i0 + m) * N;   // bias row of query i0 + m
   const float mterm = -inf * LOG2E_;
   f32x16 o = zero16();
   float mref = -INFINITY, lsum = 0.f;
   for (int j0 = 32 * wid; j0 < n_valid; j0 += 32 * APB_SPLIT) {
+    // every load of the tile first (one memory round trip), 16 bytes each but V's gathers
+    f32x4 bv[4], mk[4];
+    const float* kr = k + (rowb + j0 + m) * c_s + hd * DH;
+    opx8 kf[2];
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      bv[g4] = *reinterpret_cast<const f32x4*>(br + j0 + 8 * g4 + 4 * h);
+      mk[g4] = mask ? *reinterpret_cast<const f32x4_any*>(mask + rowb + j0 + 8 * g4 + 4 * h) : f32x4{1.f, 1.f, 1.f, 1.f};
+    }
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) kf[s2] = apb_frag<DH>(kr, 16 * s2 + 8 * h, 1.f);
+    float vv[16];   // register 8 ks + t: key j0 + 16 ks + 8 (t >> 2) + 4 h + (t & 3), d = m
+#pragma unroll
+    for (int r = 0; r < 16; ++r) vv[r] = v[(rowb + j0 + acc_row(r, h)) * c_s + hd * DH + min(m, DH - 1)];
     // S^T init: bias[q][key] + key mask; register 4g + e is key j0 + 8g + 4h + e
     f32x16 sc;
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4) {
-      const f32x4 bv = *reinterpret_cast<const f32x4*>(br + j0 + 8 * g4 + 4 * h);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int key = j0 + 8 * g4 + 4 * h + e;
-        float t = bv[e];
+        float t = bv[g4][e];
         if (key >= n_valid) t = -INFINITY;
-        else if (mask) t += (1.f - mask[rowb + key]) * mterm;
+        else if (mask) t += (1.f - mk[g4][e]) * mterm;
         sc[4 * g4 + e] = t;
       }
     }
     // K (A operand): lane (key j0 + m, half h), k-step s holds d = 16 s + 8 h + t
-    {
-      const float* kr = k + (rowb + j0 + m) * c_s + hd * DH;
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        opx8 kf;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const int d = 16 * s2 + 8 * h + t;
-          kf[t] = (op_t)(d < DH ? kr[min(d, DH - 1)] : 0.f);
-        }
-        sc = mfma32(kf, qf[s2], sc);
-      }
-    }
+    for (int s2 = 0; s2 < 2; ++s2) sc = mfma32(kf[s2], qf[s2], sc);
     // online softmax of the tile (fp32); a fully masked prefix keeps mref = -inf, P = 0
     float mx = sc[0];
 #pragma unroll
@@ -153,10 +186,7 @@ __global__ __launch_bounds__(64 * APB_SPLIT) void apb_attn_kernel(
     for (int ks = 0; ks < 2; ++ks) {
       opx8 vf;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int key = j0 + 16 * ks + 8 * (t >> 2) + 4 * h + (t & 3);
-        vf[t] = (op_t)(m < DH ? v[(rowb + key) * c_s + hd * DH + min(m, DH - 1)] : 0.f);
-      }
+      for (int t = 0; t < 8; ++t) vf[t] = (op_t)(m < DH ? vv[8 * ks + t] : 0.f);
       o = mfma32(vf, pf[ks], o);
     }
   }
@@ -251,22 +281,30 @@ float* pf_apb_bias_ptr(const pf_apb_args* a) {
   return (float*)a->workspace + 5 * (size_t)a->B * a->N * a->c_s;
 }
 
-int pf_pair_logits(const float* z, const float* lnw, const float* lnb, const void* wz, float* out, int B, int N,
-                   int H, float eps, hipStream_t st) {
-  const long pairs = (long)B * N * N;
-  apb_zbias_kernel<<<(unsigned)((pairs / 32 + 3) / 4), 256, 0, st>>>(z, lnw, lnb, (const op_t*)wz, out, B, N, H, eps);
+namespace {
+int launch_zbias(const float* z, const float* lnw, const float* lnb, const void* wz, float* out, int B, int N, int NZ,
+                 int H, float eps, hipStream_t st) {
+  const int cus = device_cus();
+  if (cus <= 0) return pf_fail(PF_E_LAUNCH, "apb_zbias_kernel: cannot query the device");
+  const long tiles = (long)B * N * N / 32;
+  if (tiles >= (1l << 27)) return pf_fail(PF_E_INVALID, "pair bias: B * N * N must be below 2^32 (B=%d N=%d)", B, N);
+  const unsigned grid = (unsigned)min((long)cus, (tiles + ZB_WAVES - 1) / ZB_WAVES);
+  apb_zbias_kernel<<<grid, 64 * ZB_WAVES, 0, st>>>(z, lnw, lnb, (const op_t*)wz, out, B, N, NZ, H, eps);
   PF_CHECK_LAUNCH("apb_zbias_kernel");
   return PF_OK;
+}
+}  // namespace
+
+int pf_pair_logits(const float* z, const float* lnw, const float* lnb, const void* wz, float* out, int B, int N,
+                   int H, float eps, hipStream_t st) {
+  return launch_zbias(z, lnw, lnb, wz, out, B, N, N, H, eps, st);
 }
 
 extern "C" int pf_apb_pair_bias(const pf_apb_args* a) {
   int rc = pf_apb_check(a, "pf_apb_pair_bias", true);
   if (rc) return rc;
-  const long pairs = (long)a->B * a->N * a->N;
-  apb_zbias_kernel<<<(unsigned)((pairs / 32 + 3) / 4), 256, 0, (hipStream_t)a->stream>>>(
-      a->z, a->zln_w, a->zln_b, (const op_t*)a->w_z, pf_apb_bias_ptr(a), a->B, a->N, a->H, a->eps);
-  PF_CHECK_LAUNCH("apb_zbias_kernel");
-  return PF_OK;
+  return launch_zbias(a->z, a->zln_w, a->zln_b, a->w_z, pf_apb_bias_ptr(a), a->B, a->N, a->N, a->H, a->eps,
+                      (hipStream_t)a->stream);
 }
 
 namespace {
@@ -315,6 +353,18 @@ extern "C" int pf_apb_fwd(const pf_apb_args* a) {
   if (rc) return rc;
   if ((rc = pf_apb_pair_bias(a))) return rc;
   return pf_apb_attend(a);
+}
+
+extern "C" int pf_apb_fwd_unpadded(const pf_apb_args* a, int z_n, int fast) {
+  int rc = pf_apb_check(a, "pf_apb_fwd_unpadded", false);
+  if (rc) return rc;
+  const int n_valid = a->n_valid ? a->n_valid : a->N;
+  if (z_n < n_valid || z_n > a->N)
+    return pf_fail(PF_E_INVALID, "pf_apb_fwd_unpadded: z_n %d outside [n_valid=%d, N=%d]", z_n, n_valid, a->N);
+  rc = launch_zbias(a->z, a->zln_w, a->zln_b, a->w_z, pf_apb_bias_ptr(a), a->B, a->N, z_n, a->H, a->eps,
+                    (hipStream_t)a->stream);
+  if (rc) return rc;
+  return apb_attend_impl(a, "pf_apb_fwd_unpadded", fast != 0);
 }
 
 extern "C" int pf_apb_fwd_mx8(const pf_apb_args* a) {

@@ -686,7 +686,7 @@ def attention_pair_bias(s: torch.Tensor, z: torch.Tensor, mask: Optional[torch.T
         return padded(t.to(torch.float32), n_pad, dev, (1,))
     sp = pad_tokens(s)
     kp = sp if k_in is s else pad_tokens(k_in)   # both are only read
-    zp = pad_pair(z.to(torch.float32), n_pad) if n_pad != N else z.to(torch.float32).contiguous()
+    zp = z.to(torch.float32).contiguous()   # read unpadded
     if mask is not None and n_pad == N:
         mp = mask.to(device=dev, dtype=torch.float32).contiguous()
     elif mask is not None and tuple(mask.shape) == (B, N):
@@ -697,8 +697,8 @@ def attention_pair_bias(s: torch.Tensor, z: torch.Tensor, mask: Optional[torch.T
     w = convert_weights(weights, dev, variant)
     out = torch.empty_like(sp)
     ws = workspace(apb_workspace_bytes(B, n_pad, c_s, num_heads, variant), dev)
-    launch_apb(sp, kp, zp, mp, out, w, num_heads, ws, accumulate=False, eps=eps, n_valid=N, variant=variant,
-               fast=fast)
+    a = _apb_args(sp, kp, zp, mp, out, w, num_heads, ws, False, eps, N)
+    _lib.check(_lib.load(variant).pf_apb_fwd_unpadded(ctypes.byref(a), N, int(fast)), "pf_apb_fwd_unpadded", variant)
     return out[:, :N]
 
 
