@@ -163,3 +163,26 @@ def test_attention_pair_bias_unpadded(gpu, B, N, masked, fast):
     if not fast:
         check("attention_pair_bias", got, ref.attention_pair_bias(s.cpu(), z.cpu(), torch.ones((B, N)) if mask is None
                                                                   else mask.cpu(), s.cpu(), w))
+
+
+# ------------------------------------------------------------------------------ pair transition
+@pytest.mark.parametrize("rows", [1, 31, 33, 64, 65, 16384, 16385])
+@pytest.mark.parametrize("hidden", [128, 512])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_transition_split(gpu, rows, hidden, accumulate):
+    """The hidden-split transition up to one workgroup of 64 pairs per CU (16384 on 256 CUs) and the
+    one-chain kernel just above: partial tiles, an odd number of tiles, two blocks per half and
+    more."""
+    from tt_boltz_amd import synthetic
+    shapes = {"norm.weight": (128,), "norm.bias": (128,), "fc1.weight": (hidden, 128), "fc2.weight": (hidden, 128),
+              "fc3.weight": (128, hidden)}
+    raw = synthetic.draw(shapes, 13)
+    w = ops.convert_weights(raw, gpu)
+    w["fc3.weight.lo"] = ops.opw_lo(raw["fc3.weight"], gpu)
+    x = torch.randn((rows, 128), generator=torch.Generator().manual_seed(rows))
+    xd = torch.cat([x, torch.full((64, 128), 7.0)]).to(gpu)   # guard rows behind the last one
+    out = xd.clone()
+    ops.launch_transition(xd[:rows], out[:rows], w, None, accumulate)
+    want = ref.transition(x, raw)
+    check("transition", out[:rows] - x.to(gpu) if accumulate else out[:rows], want)
+    assert torch.equal(out[rows:], xd[rows:])

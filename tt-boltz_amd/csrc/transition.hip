@@ -212,6 +212,110 @@ __global__ __launch_bounds__(64 * TRW, MODE == TR_HILO || MODE == TR_STATS ? 2 :
   }
 }
 
+// TR_HILO for small grids: a workgroup is 2 tiles of 32 pairs x 2 halves of the hidden units, so the
+// serial chain over weight blocks is half as long and there are twice as many workgroups; every half
+// has a ring of its own (128 KB in all).  The second half's partial sums meet the first's in LDS.
+// us (with the fused pair bias) against the one-chain kernel: N = 64 27.5 -> 22, N = 128 30.5 -> 26.
+constexpr size_t TRSP_LDS = 2 * 2 * (size_t)tr_stage<TR_HILO>();
+template <bool ZBIAS>
+__global__ __launch_bounds__(64 * TRW, 1) void tr_pair_split_kernel(
+    const float* x_in, float* out, const float* __restrict__ lnw, const float* __restrict__ lnb,
+    const op_t* __restrict__ w1, const op_t* __restrict__ w2, const op_t* __restrict__ w3,
+    const op_t* __restrict__ w3_lo, long rows, int hidden, int accumulate, float eps, ZBiasArgs zb) {
+  constexpr int STAGE = tr_stage<TR_HILO>();
+  extern __shared__ __attribute__((aligned(16))) char tsl[];
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = wid & 1, tile = wid >> 1;
+  const int nhb = hidden / 64, hb0 = half * nhb;   // blocks of this half
+  const long pos0 = ((long)blockIdx.x * 2 + tile) * 32;
+  char* ring = tsl + half * 2 * STAGE;
+  // DMA: chunk e = 64 tile + lane + 128 i (i = 0..3) of each 8 KB block; layout as tr_pair_kernel
+  const int e0 = 64 * tile + lane, R3 = e0 >> 2;
+  uint32_t o12[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int R = (e0 >> 4) + 8 * i;
+    o12[i] = 2u * (perm16(R) * C + 8 * ((e0 & 15) ^ (R & 15)));
+  }
+  const uint32_t o3 = 2u * (R3 * hidden + 8 * ((e0 & 3) ^ tr_swz4(R3)));   // row R3 + 32 i: same slot
+  const uint32_t o3b = 2u * 32 * hidden;
+  auto issue = [&](int hb, int buf) {
+    char* st = ring + buf * STAGE + 1024 * tile;
+    const char* b1 = (const char*)(w1 + (long)32 * hb * C);
+    const char* b2 = (const char*)(w2 + (long)32 * hb * C);
+    const char* b3 = (const char*)(w3 + 32 * hb);
+    const char* b4 = (const char*)(w3_lo + 32 * hb);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      __builtin_amdgcn_global_load_lds(b1 + o12[i], st + 2048 * i, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(b2 + o12[i], st + TR_BLK + 2048 * i, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(b3 + o3 + o3b * i, st + 2 * TR_BLK + 2048 * i, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(b4 + o3 + o3b * i, st + 3 * TR_BLK + 2048 * i, 16, 0, 0);
+    }
+  };
+  int a12[8], a3[2];
+#pragma unroll
+  for (int s2 = 0; s2 < 8; ++s2) a12[s2] = 256 * m + 16 * ((2 * s2 + h) ^ (m & 15));
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) a3[ks] = 2 * TR_BLK + 64 * m + 16 * ((2 * ks + h) ^ tr_swz4(m));
+  issue(hb0, 0);
+  opx8 xf[8];
+  {   // rows past the end are clamped on load and skipped on store
+    float x[64];
+    load_row128_frag(x_in + min(pos0 + m, rows - 1) * C, h, x);
+    ln128_to_frag(x, h, lnw, lnb, eps, xf);
+  }
+  f32x16 acc[4];
+#pragma unroll
+  for (int ob = 0; ob < 4; ++ob) acc[ob] = zero16();
+  for (int k = 0; k < nhb; ++k) {
+    const int buf = k & 1;
+    __builtin_amdgcn_s_waitcnt(vmcnt_le(0));   // the block landed ...
+    __builtin_amdgcn_s_barrier();              // ... for every wave; the other stage is free
+    asm volatile("" ::: "memory");
+    if (k + 1 < nhb) issue(hb0 + k + 1, buf ^ 1);
+    const char* st = ring + buf * STAGE;
+    f32x16 a1 = zero16(), a2 = zero16();
+#pragma unroll
+    for (int s2 = 0; s2 < 8; ++s2) {
+      a1 = mfma32(lds_x8(st + a12[s2]), xf[s2], a1);            // rows = hidden (perm16), cols = pairs
+      a2 = mfma32(lds_x8(st + TR_BLK + a12[s2]), xf[s2], a2);
+    }
+    opx8 hf[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int t = 0; t < 8; ++t) hf[ks][t] = (op_t)(siluf(a1[8 * ks + t]) * a2[8 * ks + t]);
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        acc[ob] = mfma32(lds_x8(st + a3[ks] + 2048 * ob), hf[ks], acc[ob]);
+        acc[ob] = mfma32(lds_x8(st + TR_BLK + a3[ks] + 2048 * ob), hf[ks], acc[ob]);
+      }
+  }
+  __syncthreads();   // the rings are read out
+  f32x4* part = reinterpret_cast<f32x4*>(tsl) + tile * 16 * 64 + lane;   // [tile][16][64 lanes]
+  if (half == 1) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+      part[64 * q] = f32x4{acc[q >> 2][4 * (q & 3)], acc[q >> 2][4 * (q & 3) + 1], acc[q >> 2][4 * (q & 3) + 2],
+                           acc[q >> 2][4 * (q & 3) + 3]};
+  }
+  __syncthreads();
+  if (half == 0) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const f32x4 v = part[64 * q];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[q >> 2][4 * (q & 3) + e] += v[e];
+    }
+    // (both halves have long read their rows: x_in may alias out)
+    if (pos0 < rows) pair_update_epilogue<ZBIAS>(acc, out, rows, pos0, m, h, accumulate, zb);
+  }
+}
+
 // corr[c] = the sum of np partial rows [np][128]: one workgroup of 1024 threads, thread
 // (quad q of 4 channels, group g of 32) summing rows g, g + 32, ... with all its loads in
 // flight (np <= TRS_PARTIALS), then the 32 groups through LDS.
@@ -283,6 +387,12 @@ int launch_tr_pair(const pf_transition_args* a, const ZBiasArgs& zb) {
     tr_pair_kernel<ZBIAS, TR_MEANFIX><<<grid, 64 * TRW, 0, st>>>(a->x_in, a->out, a->norm_w, a->norm_b, w1, w2, w3,
                                                                 nullptr, a->rows, a->hidden, a->accumulate, a->eps,
                                                                 zb, corr, nullptr);
+  } else if (lo && a->hidden % 64 == 0 && (a->rows + 63) / 64 <= device_cus()) {
+    // one workgroup fills a CU: up to one round of the chip (N = 128), where the chain is the time
+    const void* fn = (const void*)tr_pair_split_kernel<ZBIAS>;
+    if (const int rc = pf_reserve_lds(fn, TRSP_LDS, "tr_pair_split_kernel")) return rc;
+    tr_pair_split_kernel<ZBIAS><<<(unsigned)((a->rows + 63) / 64), 64 * TRW, TRSP_LDS, st>>>(
+        a->x_in, a->out, a->norm_w, a->norm_b, w1, w2, w3, lo, a->rows, a->hidden, a->accumulate, a->eps, zb);
   } else if (lo) {
     tr_pair_kernel<ZBIAS, TR_HILO><<<grid, 64 * TRW, 0, st>>>(a->x_in, a->out, a->norm_w, a->norm_b, w1, w2, w3, lo,
                                                              a->rows, a->hidden, a->accumulate, a->eps, zb, nullptr,
