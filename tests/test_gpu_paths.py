@@ -186,3 +186,53 @@ def test_transition_split(gpu, rows, hidden, accumulate):
     want = ref.transition(x, raw)
     check("transition", out[:rows] - x.to(gpu) if accumulate else out[:rows], want)
     assert torch.equal(out[rows:], xd[rows:])
+
+
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 32 * 1031])
+@pytest.mark.parametrize("hidden", [256, 512])
+@pytest.mark.parametrize("mode", ["update", "accumulate", "inplace", "corrected"])
+def test_transition_direct(gpu, rows, hidden, mode):
+    """The register-weight transition: partial groups of 64 rows, more groups than CUs, the residual
+    from another tensor and in place, and the mean correction (all rows are its sample up to 8192)."""
+    from tt_boltz_amd import synthetic
+    shapes = {"norm.weight": (128,), "norm.bias": (128,), "fc1.weight": (hidden, 128), "fc2.weight": (hidden, 128),
+              "fc3.weight": (128, hidden)}
+    raw = synthetic.draw(shapes, 17)
+    w = ops.convert_weights(raw, gpu)
+    x = torch.randn((rows, 128), generator=torch.Generator().manual_seed(rows))
+    want = ref.transition(x, raw)
+    xd = torch.cat([x, torch.full((64, 128), 7.0)]).to(gpu)   # guard rows behind the last one
+    if mode == "corrected":
+        w["fc3.weight.lo"] = ops.opw_lo(raw["fc3.weight"], gpu)
+        ws = ops.workspace(ops.transition_workspace_bytes(rows, 128, hidden), gpu)
+        out = torch.full_like(xd, 3.0)
+        ops.launch_transition(xd[:rows], out[:rows], w, ws, False, fc3_mean_fix=True)
+        check("transition corrected", out[:rows], want)
+        assert (out[rows:] == 3.0).all()
+        return
+    out = xd if mode == "inplace" else torch.full_like(xd, 3.0)
+    keep = out[rows:].clone()
+    ops.launch_transition(xd[:rows], out[:rows], w, None, mode != "update")
+    base = {"update": 0.0, "accumulate": 3.0, "inplace": x.to(gpu)}[mode]
+    check(f"transition {mode}", out[:rows] - base, want)
+    assert torch.equal(out[rows:], keep)
+
+
+@pytest.mark.parametrize("B,N", [(1, 64), (2, 96), (1, 352)])
+def test_transition_direct_pair_bias(gpu, B, N):
+    """The pair bias of the updated rows from the same kernel against the bias kernel on them (odd
+    numbers of 32-row tiles, a batch)."""
+    w = ops.convert_weights(_sub_w(21, "transition_z"), gpu)
+    wa = ops.convert_weights(_sub_w(22, "attention"), gpu)
+    g = torch.Generator().manual_seed(N)
+    z = torch.randn((B, N, N, 128), generator=g).to(gpu)
+    s = torch.randn((B, N, 384), generator=g).to(gpu)
+    n = ops.apb_workspace_bytes(B, N, 384, 16)
+    ws = [ops.workspace(n, gpu).fill_(0) for _ in range(2)]
+    out = torch.empty_like(z)
+    ops.launch_transition(z, out, w, None, False, pair_bias=(s, wa, 16, ws[0], 1e-5))
+    ops.launch_apb(s, s, out, None, s, wa, 16, ws[1], False, part="bias")
+    start = 5 * B * N * 384 * 4
+    got, want = (t[start:start + B * 16 * N * N * 4].view(torch.float32) for t in ws)
+    # one LayerNorm each, summed in another order: op_t rounding ties aside the bits agree
+    check("fused pair bias", got, want, max_tol=5e-3, mean_tol=1e-4)

@@ -18,6 +18,7 @@
 //                    matrices (tt_bio/boltz2.py:638-731); fp32 in/out, MFMA inside.
 //   pair_ln_linear_kernel  out = base + W LN(x) for C = 128 rows (trunk recycling step).
 #include "pf_common.h"
+#include "pf_direct.h"
 #include "pf_internal.h"
 
 namespace {
@@ -316,6 +317,261 @@ __global__ __launch_bounds__(64 * TRW, 1) void tr_pair_split_kernel(
   }
 }
 
+// The pair transition with its weights in registers (pf_direct.h): 8 waves (one workgroup per CU) walk
+// groups of 64 rows.  Wave w owns hidden units (HID / 8) w .. of fc1 and fc2, and the output channels
+// 32 (w & 3) .. + 31 of half w >> 2 of the hidden units of fc3: at HID = 512 three times 64 registers.
+// A group is normalized once into LDS; the hidden activations (op_t) go through LDS; the two halves
+// of each output meet in LDS, each wave finishing one 32-row tile; and the finished rows leave from
+// LDS whole, 16 lanes a row, with the residual and corr (TR_MEANFIX: added in fp32).  ZBIAS: the
+// workgroup then normalizes the rows it has just written and waves 0 and 1 project them.
+// Against weight blocks streamed through an LDS ring by four-wave workgroups (one LDS read per MFMA,
+// here three for four; the residual re-read from HBM), us, plain weights: hidden 256, N = 128 17.1 ->
+// 10.3, 450 94 -> 83, 1024 434 -> 370; hidden 512, N = 128 24.4 -> 15.5, 1024 602 -> 546; with the
+// mean correction and the pair bias N = 384 111 -> 105, 768 350 -> 338, 1024 601 -> 572.  MFMAs, SwiGLU and LDS traffic take about 3.5, 2.5 and
+// 3.3 us of a group's 8.5 at hidden 512 and hardly overlap with one workgroup per CU: every wave is
+// in the same phase (raising the priority of one wave per SIMD in the first phase changed nothing).
+constexpr int TRD_WAVES = 8, TRD_ZP = 132;
+template <int HID>
+struct TrdLds {   // byte offsets
+  static constexpr int K3L = HID == 512 ? 8 : 0;   // fc3 k-steps of a wave that stay in LDS
+  static constexpr size_t SX = 0;                                            // normalized rows [64][136] op_t
+  static constexpr size_t SH = SX + (size_t)DP_ROWS * LDSW * sizeof(op_t);   // hidden [64][HID + 8] op_t, then rows [64][132] fp32
+  static constexpr size_t SHB = (size_t)DP_ROWS * (HID + 8) * sizeof(op_t);
+  static constexpr size_t ROWB = (size_t)DP_ROWS * TRD_ZP * 4;
+  static constexpr size_t WBUF = (size_t)TRD_WAVES * 32 * LDSW * sizeof(op_t);   // set-up: the weight buffers
+  static_assert(ROWB + (size_t)DP_ROWS * LDSW * sizeof(op_t) <= WBUF, "ZBIAS: normalized rows behind the rows");
+  static constexpr size_t VEC = SH + (SHB > WBUF ? SHB : WBUF > ROWB ? WBUF : ROWB);
+  static constexpr size_t WZ = VEC + 5 * C * 4;                              // norm w, b, corr, zb norm w, b [128] fp32 each
+  static constexpr size_t F3 = WZ + (size_t)16 * LDSW * sizeof(op_t);        // W_z [16][136] op_t
+  static constexpr size_t BYTES = F3 + (size_t)TRD_WAVES * K3L * 64 * 16;    // fragments [8][K3L][64 lanes]
+};
+template <int HID, bool ZBIAS, bool CORR>
+__global__ __launch_bounds__(64 * TRD_WAVES, 1) void tr_direct_kernel(
+    const float* x_in, float* out, const float* __restrict__ lnw, const float* __restrict__ lnb,
+    const op_t* __restrict__ w1, const op_t* __restrict__ w2, const op_t* __restrict__ w3, long rows, int accumulate,
+    float eps, ZBiasArgs zb, const float* __restrict__ corr, int ngroups) {
+  typedef TrdLds<HID> L;
+  constexpr int NB = HID / 256;                  // 32-unit hidden blocks of a wave
+  constexpr int K3 = HID / 32, K3R = K3 - L::K3L;   // fc3 k-steps of a wave, in registers
+  constexpr int LH = HID + 8, ZP = TRD_ZP;
+  extern __shared__ __attribute__((aligned(16))) char dl[];
+  op_t* sx = reinterpret_cast<op_t*>(dl + L::SX);
+  op_t* sh = reinterpret_cast<op_t*>(dl + L::SH);
+  float* zrow = reinterpret_cast<float*>(sh);
+  op_t* sz = reinterpret_cast<op_t*>(dl + L::SH + L::ROWB);
+  float* vec = reinterpret_cast<float*>(dl + L::VEC);
+  op_t* swz = reinterpret_cast<op_t*>(dl + L::WZ);
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  opx8* f3l = reinterpret_cast<opx8*>(dl + L::F3) + wid * L::K3L * 64 + lane;
+  const int ob = wid & 3, kh = wid >> 2;
+  const int g4 = lane >> 4, q4 = lane & 15;
+  // rows 8 wid + 4 it + g4 of a group, channels 4 q4 .. and 64 + 4 q4 ..: loads clamped at the end
+  // (uniform base + 32-bit lane offset: 64-bit lane addresses cost the registers the weights need)
+  f32x4 x[2][2];
+  auto fetch = [&](const float* src, int g, f32x4 (&v)[2][2]) PF_INLINE {
+    const char* base = reinterpret_cast<const char*>(src + (long)DP_ROWS * g * C);
+    const uint32_t last = (uint32_t)min((long)DP_ROWS, rows - (long)DP_ROWS * g) - 1;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const uint32_t off = 4u * (min((uint32_t)(8 * wid + 4 * it + g4), last) * C + 4 * q4);
+      v[it][0] = *reinterpret_cast<const f32x4*>(base + off);
+      v[it][1] = *reinterpret_cast<const f32x4*>(base + off + 256);
+    }
+  };
+  // LayerNorm with affine parameters w, b (LDS) of the wave's 8 rows -> op_t rows of dst
+  auto norm_row = [&](const f32x4 (&v)[2], const float* w, const float* b, float e_, op_t* dst, int r, int q4) PF_INLINE {
+    const float mean = row16_sum((v[0][0] + v[0][1]) + (v[0][2] + v[0][3]) + (v[1][0] + v[1][1]) +
+                                 (v[1][2] + v[1][3])) * (1.f / C);
+    float var = 0.f;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { const float d = v[u][e] - mean; var += d * d; }
+    const float rstd = rsqrtf(row16_sum(var) * (1.f / C) + e_);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const f32x4 gw = *reinterpret_cast<const f32x4*>(w + 64 * u + 4 * q4);
+      const f32x4 gb = *reinterpret_cast<const f32x4*>(b + 64 * u + 4 * q4);
+      opx4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (op_t)((v[u][e] - mean) * rstd * gw[e] + gb[e]);
+      st_x4(dst + r * LDSW + 64 * u + 4 * q4, o);
+    }
+  };
+  fetch(x_in, blockIdx.x, x);
+  DirectW<C> f1[NB], f2[NB];
+  opx8 f3[K3R];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    f1[b].load(w1 + (long)32 * (NB * wid + b) * C, lane);
+    f2[b].load(w2 + (long)32 * (NB * wid + b) * C, lane);
+  }
+  if (tid < C) {
+    vec[tid] = lnw[tid];
+    vec[C + tid] = lnb[tid];
+    if constexpr (CORR) vec[2 * C + tid] = corr[tid];
+    if constexpr (ZBIAS) {
+      vec[3 * C + tid] = zb.lnw[tid];
+      vec[4 * C + tid] = zb.lnb[tid];
+    }
+  }
+  if constexpr (ZBIAS)
+    if (tid < 16 * 16)
+      st_x8(swz + (tid >> 4) * LDSW + 8 * (tid & 15), ld_x8(zb.wz + min(tid >> 4, zb.H - 1) * C + 8 * (tid & 15)));
+  {   // fc3 rows 32 ob + m, columns (HID / 2) kh ..: 128-byte pieces of 8 rows an instruction, turned
+      // 64 columns at a time
+    op_t* wb = sh + wid * 32 * LDSW;   // the waves' buffers (8 x 8.5 KB)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      f1[b].turn(wb, lane);
+      f2[b].turn(wb, lane);
+    }
+    const op_t* src = w3 + (long)32 * ob * HID + (HID / 2) * kh;
+#pragma unroll
+    for (int c = 0; c < K3 / 4; ++c) {
+      opx8 v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = ld_x8(src + (long)(8 * i + (lane >> 3)) * HID + 64 * c + 8 * (lane & 7));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) st_x8(wb + (8 * i + (lane >> 3)) * LDSW + 8 * (lane & 7), v[i]);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const opx8 f = ld_x8(wb + m * LDSW + 16 * s + 8 * h);
+        if (4 * c + s < K3R)
+          f3[4 * c + s < K3R ? 4 * c + s : 0] = f;
+        else
+          f3l[64 * (4 * c + s - K3R)] = f;
+      }
+    }
+  }
+  __syncthreads();   // the weight buffers are read out
+  for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x) {
+#pragma unroll
+    for (int it = 0; it < 2; ++it) norm_row(x[it], vec, vec + C, eps, sx, 8 * wid + 4 * it + g4, q4);
+    __syncthreads();   // sx is whole; sh and the last rows are free
+    // the next group's rows as early as the registers allow
+    const bool more = gi + (int)gridDim.x < ngroups;
+    if (HID == 256 && more) fetch(x_in, gi + gridDim.x, x);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        f32x16 a1 = zero16(), a2 = zero16();
+        const op_t* xr = sx + (32 * t + m) * LDSW + 8 * h;
+        opx8 c0 = ld_x8(xr), c1 = ld_x8(xr + 16);
+#pragma unroll
+        for (int s = 0; s < 8; s += 2) {   // the next two fragments are read beside these four MFMAs
+          const opx8 n0 = ld_x8(xr + 16 * ((s + 2) & 7)), n1 = ld_x8(xr + 16 * ((s + 3) & 7));
+          a1 = mfma32(f1[b].v[s], c0, a1);   // rows = hidden unit, cols = row of x
+          a2 = mfma32(f2[b].v[s], c0, a2);
+          a1 = mfma32(f1[b].v[s + 1], c1, a1);
+          a2 = mfma32(f2[b].v[s + 1], c1, a2);
+          c0 = n0;
+          c1 = n1;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        op_t* dst = sh + (32 * t + m) * LH + 32 * (NB * wid + b) + 4 * h;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          opx4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = (op_t)(siluf(a1[4 * g + e]) * a2[4 * g + e]);
+          st_x4(dst + 8 * g, v);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    __syncthreads();
+    if (HID != 256 && more) fetch(x_in, gi + gridDim.x, x);
+    f32x4 res[2][2];   // the residual, in the rows' final layout
+    if (HID == 256 && accumulate) fetch(out, gi, res);
+    f32x16 acc[2] = {zero16(), zero16()};
+    const op_t* hr = sh + m * LH + (HID / 2) * kh + 8 * h;
+#pragma unroll
+    for (int s = 0; s < K3; ++s) {
+      const opx8 wf = s < K3R ? f3[s < K3R ? s : 0] : f3l[64 * (s - K3R)];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[t] = mfma32(wf, ld_x8(hr + 32 * t * LH + 16 * s), acc[t]);
+      if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();   // sh is read out: the rows go over it, one half's sums, then the other's added
+    if (HID != 256 && accumulate) fetch(out, gi, res);
+    float* zr = zrow + m * ZP + 32 * ob + 4 * h;
+    if (kh == 0) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4*>(zr + 32 * t * ZP + 8 * g) =
+              f32x4{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
+    }
+    __syncthreads();
+    if (kh == 1) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          f32x4 v = *reinterpret_cast<f32x4*>(zr + 32 * t * ZP + 8 * g);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += acc[t][4 * g + e];
+          *reinterpret_cast<f32x4*>(zr + 32 * t * ZP + 8 * g) = v;
+        }
+    }
+    __syncthreads();
+    char* obase = reinterpret_cast<char*>(out + (long)DP_ROWS * gi * C);
+    const int left = (int)min((long)DP_ROWS, rows - (long)DP_ROWS * gi);
+    int fl = lane;
+    asm volatile("" : "+v"(fl));   // the addresses are formed here, not kept across the loop
+    const int q4 = fl & 15;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const int r = 8 * wid + 4 * it + (fl >> 4);
+      f32x4 z[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        z[u] = *reinterpret_cast<const f32x4*>(zrow + r * ZP + 64 * u + 4 * q4);
+        if constexpr (CORR) {
+          const f32x4 c = *reinterpret_cast<const f32x4*>(vec + 2 * C + 64 * u + 4 * q4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) z[u][e] += c[e];
+        }
+        if (accumulate)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) z[u][e] += res[it][u][e];
+        if (r < left) *reinterpret_cast<f32x4*>(obase + 4u * (r * C + 64 * u + 4 * q4)) = z[u];
+      }
+      // ZBIAS: the updated row normalized, behind the rows in sh
+      if constexpr (ZBIAS) norm_row(z, vec + 3 * C, vec + 4 * C, zb.eps, sz, r, q4);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (ZBIAS) {
+      __syncthreads();
+      if (wid < 2) {   // D[head][row] of tile wid (N * N is a multiple of 32)
+        int zl = lane;
+        asm volatile("" : "+v"(zl));   // the addresses are formed here, not kept across the loop
+        const int zm = zl & 31, zh = zl >> 5;
+        f32x16 hb = zero16();
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          hb = mfma32(ld_x8(swz + (zm & 15) * LDSW + 16 * s + 8 * zh), ld_x8(sz + (32 * wid + zm) * LDSW + 16 * s + 8 * zh), hb);
+          if (s % 2) __builtin_amdgcn_sched_barrier(0);
+        }
+        const long p0 = (long)DP_ROWS * gi + 32 * wid;
+        if (p0 < rows) {
+          const long b = p0 / zb.NN;
+          char* brow = reinterpret_cast<char*>(zb.bias + b * zb.H * zb.NN + (p0 - b * zb.NN));
+          const uint32_t boff = 4u * (4u * zh * (uint32_t)zb.NN + zm);
+#pragma unroll
+          for (int r = 0; r < 8; ++r) {   // heads 0..15: registers 0..7
+            if (acc_row(r, zh) < zb.H)
+              *reinterpret_cast<float*>(brow + 4 * acc_row(r, 0) * zb.NN + boff) = hb[r] * 1.4426950408889634f;
+          }
+        }
+      }
+    }
+  }
+}
+
 // corr[c] = the sum of np partial rows [np][128]: one workgroup of 1024 threads, thread
 // (quad q of 4 channels, group g of 32) summing rows g, g + 32, ... with all its loads in
 // flight (np <= TRS_PARTIALS), then the 32 groups through LDS.
@@ -363,6 +619,27 @@ int tr_check_fc3(const pf_transition_args* a, const char* fn) {
   return PF_OK;
 }
 
+// The register-weight transition where it applies (hidden 256 or 512, at most 16 heads); false: not.
+template <bool ZBIAS, bool CORR>
+bool launch_tr_direct(const pf_transition_args* a, const ZBiasArgs& zb, const float* corr, int* rc) {
+  const long groups = (a->rows + DP_ROWS - 1) / DP_ROWS;
+  if ((a->hidden != 256 && a->hidden != 512) || (ZBIAS && zb.H > 16) || groups > 0x3fffffff) return false;
+  const int cus = device_cus();
+  if (cus <= 0) {
+    *rc = pf_fail(PF_E_LAUNCH, "tr_direct_kernel: cannot query the device");
+    return true;
+  }
+  auto kern = a->hidden == 256 ? tr_direct_kernel<256, ZBIAS, CORR> : tr_direct_kernel<512, ZBIAS, CORR>;
+  const size_t lds = a->hidden == 256 ? TrdLds<256>::BYTES : TrdLds<512>::BYTES;
+  if ((*rc = pf_reserve_lds((const void*)kern, lds, "tr_direct_kernel"))) return true;
+  kern<<<(unsigned)min(groups, (long)cus), 64 * TRD_WAVES, lds, (hipStream_t)a->stream>>>(
+      a->x_in, a->out, a->norm_w, a->norm_b, (const op_t*)a->fc1_w, (const op_t*)a->fc2_w, (const op_t*)a->fc3_w,
+      a->rows, a->accumulate, a->eps, zb, corr, (int)groups);
+  const hipError_t e = hipGetLastError();
+  *rc = e == hipSuccess ? PF_OK : pf_fail(PF_E_LAUNCH, "tr_direct_kernel launch failed: %s", hipGetErrorString(e));
+  return true;
+}
+
 // The pair transition's launch over workgroups of TRW tiles of 32 pairs (the last one clamped):
 // plain, hi + lo, or the mean-corrected form after its sampling pass.
 template <bool ZBIAS>
@@ -371,6 +648,7 @@ int launch_tr_pair(const pf_transition_args* a, const ZBiasArgs& zb) {
   const unsigned grid = (unsigned)((a->rows + 32 * TRW - 1) / (32 * TRW));
   const op_t *w1 = (const op_t*)a->fc1_w, *w2 = (const op_t*)a->fc2_w, *w3 = (const op_t*)a->fc3_w;
   const op_t* lo = (const op_t*)a->fc3_lo;
+  int rc = PF_OK;
   if (lo && a->fc3_mean_fix) {
     float* partials = (float*)a->workspace;
     float* corr = partials + (size_t)TRS_PARTIALS * C;
@@ -384,6 +662,7 @@ int launch_tr_pair(const pf_transition_args* a, const ZBiasArgs& zb) {
     }
     tr_corr_kernel<<<1, 1024, 0, st>>>(partials, ns > 0 ? np : 0, corr);   // no sample: corr = 0
     PF_CHECK_LAUNCH("tr_corr_kernel");
+    if (launch_tr_direct<ZBIAS, true>(a, zb, corr, &rc)) return rc;
     tr_pair_kernel<ZBIAS, TR_MEANFIX><<<grid, 64 * TRW, 0, st>>>(a->x_in, a->out, a->norm_w, a->norm_b, w1, w2, w3,
                                                                 nullptr, a->rows, a->hidden, a->accumulate, a->eps,
                                                                 zb, corr, nullptr);
@@ -397,6 +676,8 @@ int launch_tr_pair(const pf_transition_args* a, const ZBiasArgs& zb) {
     tr_pair_kernel<ZBIAS, TR_HILO><<<grid, 64 * TRW, 0, st>>>(a->x_in, a->out, a->norm_w, a->norm_b, w1, w2, w3, lo,
                                                              a->rows, a->hidden, a->accumulate, a->eps, zb, nullptr,
                                                              nullptr);
+  } else if (launch_tr_direct<ZBIAS, false>(a, zb, nullptr, &rc)) {
+    return rc;
   } else {
     tr_pair_kernel<ZBIAS, TR_PLAIN><<<grid, 64 * TRW, 0, st>>>(a->x_in, a->out, a->norm_w, a->norm_b, w1, w2, w3,
                                                               nullptr, a->rows, a->hidden, a->accumulate, a->eps, zb,
