@@ -236,3 +236,43 @@ def test_transition_direct_pair_bias(gpu, B, N):
     got, want = (t[start:start + B * 16 * N * N * 4].view(torch.float32) for t in ws)
     # one LayerNorm each, summed in another order: op_t rounding ties aside the bits agree
     check("fused pair bias", got, want, max_tol=5e-3, mean_tol=1e-4)
+
+
+# ------------------------------------------------------------------------------ diffusion conditioning
+@pytest.mark.parametrize("N", [1, 7, 8, 13, 131])
+@pytest.mark.parametrize("depth,heads", [(1, 32), (24, 16), (16, 32), (4, 24)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_token_bias_blocks(gpu, N, depth, heads, layout):
+    """One to sixteen output blocks (some waves with two), layers that end inside a block, partial
+    and several groups of 64 pairs, both layouts."""
+    from tt_boltz_amd.diffusion import TokenTransformerPairBias
+    g = torch.Generator().manual_seed(N)
+    w = {}
+    for l in range(depth):
+        w[f"token_trans_proj_z.{l}.0.weight"] = 1 + 0.1 * torch.randn(128, generator=g)
+        w[f"token_trans_proj_z.{l}.0.bias"] = 0.1 * torch.randn(128, generator=g)
+        w[f"token_trans_proj_z.{l}.1.weight"] = 0.1 * torch.randn((heads, 128), generator=g)
+    z = torch.randn((1, N, N, 128), generator=g)
+    from oracle import diffusion_ref
+    want = 0.5 * diffusion_ref.token_trans_bias(z, w, depth)
+    M = depth * heads
+    buf = torch.full((N * N * M + 64,), 7.0, device=gpu)   # guard values behind the output
+    out = buf[:N * N * M].view(*((1, N, N, M) if layout == 0 else (M, 1, N, N)))
+    TokenTransformerPairBias(depth, w)(z.to(gpu), layout, 0.5, out)
+    check("token bias", out if layout == 0 else out.permute(1, 2, 3, 0), want)
+    assert (buf[N * N * M:] == 7.0).all()
+
+
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 64 * 256 + 1])
+def test_cond_proj_groups(gpu, rows):
+    """Partial and several groups of 64 pairs."""
+    from oracle.pairformer_ref import layer_norm, linear
+    g = torch.Generator().manual_seed(rows)
+    z, r = (torch.randn((rows, 128), generator=g) for _ in range(2))
+    lw, lb = 1 + 0.1 * torch.randn(256, generator=g), 0.1 * torch.randn(256, generator=g)
+    w = 0.1 * torch.randn((128, 256), generator=g)
+    want = linear(layer_norm(torch.cat((z, r), -1), lw, lb), w)
+    out = torch.full((rows + 64, 128), 7.0, device=gpu)
+    ops.launch_pair_cond_proj(z.to(gpu), r.to(gpu), lw.to(gpu), lb.to(gpu), ops.opw(w, gpu), out[:rows])
+    check("cond proj", out[:rows], want)
+    assert (out[rows:] == 7.0).all()

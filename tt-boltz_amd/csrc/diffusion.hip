@@ -14,101 +14,128 @@
 //                      each layer's affine is folded into its weights when they are staged:
 //                      W'_l = W_l diag(gamma_l), b'_l = W_l beta_l.
 //
-// Both kernels are persistent (one workgroup of 8 waves per CU, weights resident in LDS,
-// rows of 256 bytes with 16-byte chunk c at slot c ^ (R & 15)) and walk tiles of 32 pairs
-// per wave: the LayerNorm runs in registers on the lane's half row, and the MFMA
-// orientation is chosen per output layout so that stores are long contiguous runs
-// (D[output][pair] for pair-major rows of 128 channels and for output planes,
-// D[pair][output] for the wide pair-major bias rows).
+// Both kernels are persistent (one workgroup per CU) with their weights in registers (pf_direct.h):
+// groups of 64 pairs are normalized once into LDS, 16 lanes a row, every wave multiplies them by its
+// own 32 output rows, and the outputs leave through LDS as whole 128-byte lines.
 #include "pf_common.h"
+#include "pf_direct.h"
 #include "pf_internal.h"
 
 namespace {
 
 constexpr int C = 128;       // c_z
-constexpr int DF_WAVES = 8;
-constexpr int TB_MAX_OUT = 512;
-constexpr int TB_WAVES = 12;   // token bias: three waves per SIMD (<= 168 VGPRs: no scratch spills)
+constexpr int CP_WAVES = 8;
+constexpr int TB_MAX_OUT = 512, TB_WAVES = 12;
 
-PF_DEV int slot16(int R, int c) { return R * C + 8 * (c ^ (R & 15)); }
+// rows 64 g + r of a [rows][128] tensor, clamped to the last: uniform base + 32-bit lane offset
+PF_DEV f32x4 group_row4(const float* t, int g, long rows, int r, int c) {
+  const char* base = reinterpret_cast<const char*>(t + (long)DP_ROWS * g * C);
+  const uint32_t last = (uint32_t)min((long)DP_ROWS, rows - (long)DP_ROWS * g) - 1;
+  return *reinterpret_cast<const f32x4*>(base + 4u * (min((uint32_t)r, last) * C + c));
+}
 
 // -------------------------------------------------------------------------------------
 // out[p, :] = W . LN(cat(z[p, :], r[p, :]))  (W [128][256], LN over 256 with affine)
-//          = W' . LNhat(cat(z, r)) + b'
+//          = W' . LNhat(cat(z, r)) + b',  W' = W diag(gamma) in op_t, b' = W beta
+// Wave w: output channels 32 (w >> 1) .. + 31 of the pairs 32 (w & 1) .. + 31, all 256 inputs.
+// Bound by HBM (z and r read, out written once: 61 us at the copy rate for N = 450).  Against W in LDS
+// with a lane per row: N = 37 19.2 -> 8.8 us, 128 20.4 -> 10.5, 450 80 -> 60, 512 96 -> 83.
 // -------------------------------------------------------------------------------------
-__global__ __launch_bounds__(64 * DF_WAVES, 1) void cond_proj_kernel(
+constexpr int CP_LW = 264, CP_ZP = 132;
+struct CpLds {   // byte offsets: normalized pairs [64][264] op_t, outputs [64][132] fp32 / weight buffers, offsets
+  static constexpr size_t ROW = (size_t)DP_ROWS * CP_LW * sizeof(op_t);
+  static constexpr size_t WB = (size_t)CP_WAVES * 32 * (C + 8) * sizeof(op_t);
+  static constexpr size_t OFF = ROW + WB, BYTES = OFF + C * sizeof(float);
+  static_assert(WB >= (size_t)DP_ROWS * CP_ZP * sizeof(float), "outputs over the weight buffers");
+};
+__global__ __launch_bounds__(64 * CP_WAVES, 1) void cond_proj_kernel(
     const float* __restrict__ z, const float* __restrict__ r, const float* __restrict__ lnw,
-    const float* __restrict__ lnb, const op_t* __restrict__ W, float* __restrict__ out, long rows, float eps) {
-  // W split by input half: sw[0] = W[:, 0:128] (z channels), sw[1] = W[:, 128:256]
-  // the LayerNorm affine is folded in: W' = W diag(gamma) (staged), b' = W beta
-  __shared__ __attribute__((aligned(16))) op_t sw[2][C * C];
-  __shared__ float sb[C];
+    const float* __restrict__ lnb, const op_t* __restrict__ W, float* __restrict__ out, long rows, int ngroups,
+    float eps) {
+  extern __shared__ __attribute__((aligned(16))) char cl[];
+  op_t* sx = reinterpret_cast<op_t*>(cl);
+  float* so = reinterpret_cast<float*>(cl + CpLds::ROW);
+  float* soff = reinterpret_cast<float*>(cl + CpLds::OFF);
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-#pragma unroll 4
-  for (int c = tid; c < 2 * C * 16; c += 64 * DF_WAVES) {   // 128 rows x 32 chunks
-    const int R = c >> 5, k = c & 31;
-    const opx8 wv = ld_x8(W + R * 2 * C + 8 * k);
-    opx8 o;
+  const int tile = wid & 1, ob = wid >> 1, g4 = lane >> 4, q4 = lane & 15;
+  f32x4 x[2][4];   // rows 8 wid + 4 it + g4: z channels 4 q4 .., 64 + 4 q4 .., then r's
+  auto fetch = [&](int g) PF_INLINE {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) o[u] = (op_t)((float)wv[u] * lnw[8 * k + u]);
-    st_x8(&sw[k >> 4][slot16(R, k & 15)], o);
-  }
-#pragma unroll 4
-  for (int R = wid; R < C; R += DF_WAVES) {   // one wave per output row, 4 channels per lane
-    float v = 0.f;
+    for (int it = 0; it < 2; ++it)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) v += (float)W[R * 2 * C + 64 * q + lane] * lnb[64 * q + lane];
-    v = wave_sum(v);
-    if (lane == 0) sb[R] = v;
-  }
-  __syncthreads();
-  const long ntiles = (rows + 31) / 32;
-  for (long t = (long)blockIdx.x * DF_WAVES + wid; t < ntiles; t += (long)gridDim.x * DF_WAVES) {
-    const long p0 = 32 * t, row = min(p0 + m, rows - 1);
-    opx8 xf[2][8];
-    {
-      float xz[64], xr[64];
-      load_row128_frag(z + row * C, h, xz);
-      load_row128_frag(r + row * C, h, xr);
-      float s = 0.f;
+      for (int v = 0; v < 4; ++v)
+        x[it][v] = group_row4(v < 2 ? z : r, g, rows, 8 * wid + 4 * it + g4, 64 * (v & 1) + 4 * q4);
+  };
+  fetch(blockIdx.x);
+  DirectW<C> w[2];   // input halves: z channels, r channels
 #pragma unroll
-      for (int i = 0; i < 64; ++i) s += xz[i] + xr[i];
-      const float mean = xor32_sum(s) * (1.f / 256.f);
-      float v = 0.f;
+  for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int i = 0; i < 64; ++i) {
-        const float a = xz[i] - mean, b = xr[i] - mean;
-        v += a * a + b * b;
-      }
-      const float rstd = rsqrtf(xor32_sum(v) * (1.f / 256.f) + eps);
-#pragma unroll
-      for (int s8 = 0; s8 < 8; ++s8)
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          xf[0][s8][u] = (op_t)((xz[8 * s8 + u] - mean) * rstd);
-          xf[1][s8][u] = (op_t)((xr[8 * s8 + u] - mean) * rstd);
-        }
+    for (int i = 0; i < C / 16; ++i) {
+      const int c = lane + 64 * i;
+      w[u].v[i] = ld_x8(W + (long)(32 * ob + (c >> 4)) * 2 * C + C * u + 8 * (c & 15));
     }
-    const bool live = p0 + m < rows;
-    float* dst = out + (p0 + m) * C + 4 * h;
-#pragma unroll 1
-    for (int ob = 0; ob < 4; ++ob) {
-      f32x16 acc = zero16();
+  {
+    op_t* wb = reinterpret_cast<op_t*>(so) + wid * 32 * (C + 8);
+    float off = 0.f;
 #pragma unroll
-      for (int half = 0; half < 2; ++half)
+    for (int u = 0; u < 2; ++u) {
+      w[u].turn(wb, lane);
+      off += direct_wbeta<C / 16>(w[u].v, lnb + C * u, h);
+      w[u].fold(lnw + C * u, h);
+    }
+    if (tile == 0 && h == 0) soff[32 * ob + m] = off;
+  }
+  for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x) {
 #pragma unroll
-        for (int s8 = 0; s8 < 8; ++s8)
-          acc = mfma32(ld_x8(&sw[half][slot16(32 * ob + m, 2 * s8 + h)]), xf[half][s8], acc);
-      // lane (pair m, h): acc[4 g + e] is output 32 ob + 8 g + 4 h + e
-      if (live)
+    for (int it = 0; it < 2; ++it) {
+      float s = 0.f, var = 0.f;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int o = 32 * ob + 8 * g + 4 * h;
-          *reinterpret_cast<f32x4*>(dst + 32 * ob + 8 * g) =
-              f32x4{acc[4 * g] + sb[o], acc[4 * g + 1] + sb[o + 1], acc[4 * g + 2] + sb[o + 2],
-                    acc[4 * g + 3] + sb[o + 3]};
-        }
+      for (int v = 0; v < 4; ++v) s += (x[it][v][0] + x[it][v][1]) + (x[it][v][2] + x[it][v][3]);
+      const float mean = row16_sum(s) * (1.f / 256.f);
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { const float d = x[it][v][e] - mean; var += d * d; }
+      const float rstd = rsqrtf(row16_sum(var) * (1.f / 256.f) + eps);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        opx4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (op_t)((x[it][v][e] - mean) * rstd);
+        st_x4(sx + (8 * wid + 4 * it + g4) * CP_LW + 64 * v + 4 * q4, o);
+      }
+    }
+    __syncthreads();   // sx is whole; the outputs of the last group are read out
+    if (gi + (int)gridDim.x < ngroups) fetch(gi + gridDim.x);
+    f32x16 acc;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 c4 = *reinterpret_cast<const f32x4*>(soff + 32 * ob + 8 * g + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[4 * g + e] = c4[e];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int s = 0; s < C / 16; ++s)
+        acc = mfma32(w[u].v[s], ld_x8(sx + (32 * tile + m) * CP_LW + C * u + 16 * s + 8 * h), acc);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)   // D[channel][pair]
+      *reinterpret_cast<f32x4*>(so + (32 * tile + m) * CP_ZP + 32 * ob + 8 * g + 4 * h) =
+          f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+    __syncthreads();
+    char* obase = reinterpret_cast<char*>(out + (long)DP_ROWS * gi * C);
+    const int left = (int)min((long)DP_ROWS, rows - (long)DP_ROWS * gi);
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const int rr = 8 * wid + 4 * it + g4;
+#pragma unroll
+      for (int v = 0; v < 2; ++v)
+        if (rr < left)
+          *reinterpret_cast<f32x4*>(obase + 4u * (rr * C + 64 * v + 4 * q4)) =
+              *reinterpret_cast<const f32x4*>(so + rr * CP_ZP + 64 * v + 4 * q4);
     }
   }
 }
@@ -117,83 +144,108 @@ __global__ __launch_bounds__(64 * DF_WAVES, 1) void cond_proj_kernel(
 // bias[p, o] = scale * (W'[o] . LNhat(z[p]) + b'[o]),  o = l * H + hd < M
 //   layout 0: out [rows][M]        (the reference's torch.cat(..., dim=-1) layout)
 //   layout 1: out [M][rows]        (one contiguous [B][N][N] plane per (layer, head))
+// Wave w: output blocks w and w + 12 (M <= 512: at most 16 blocks); waves 0-7 normalize.  Layout 0
+// goes through the wave's LDS stage of [64 pairs][32 outputs], so that every store instruction
+// writes eight whole 128-byte runs.  Bound by HBM (M fp32 written per pair: 81 us at the copy rate for
+// N = 450, M = 384).  Against W in LDS with a lane per row and 4-byte stores: N = 37 33.9 -> 7.8 us,
+// 128 38.7 -> 11.8, 450 130 -> 89, 512 142 -> 113 (layout 1: 450 156 -> 137, 512 138 -> 115).
 // -------------------------------------------------------------------------------------
+constexpr int TB_SP = 36;   // stage pitch (floats)
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // the caller's out: any alignment
+struct TbLds {
+  static constexpr size_t ST = (size_t)2 * DP_ROWS * (C + 8) * sizeof(op_t);   // normalized pairs, two buffers
+  static constexpr size_t OFF = ST + (size_t)TB_WAVES * DP_ROWS * TB_SP * sizeof(float);
+  static constexpr size_t BYTES = OFF + TB_MAX_OUT * sizeof(float);
+};
+template <int LAYOUT>
 __global__ __launch_bounds__(64 * TB_WAVES, 1) void token_bias_kernel(
     const float* __restrict__ z, const float* __restrict__ lnw, const float* __restrict__ lnb,
-    const op_t* __restrict__ W, float* __restrict__ out, long rows, int M, int H, int layout, float scale,
-    float eps) {
-  __shared__ __attribute__((aligned(16))) op_t sw[TB_MAX_OUT * C];
-  __shared__ float sb[TB_MAX_OUT];
+    const op_t* __restrict__ W, float* __restrict__ out, long rows, int ngroups, int M, int H, float scale, float eps) {
+  constexpr int LW = C + 8;
+  extern __shared__ __attribute__((aligned(16))) char bl[];
+  op_t* sx = reinterpret_cast<op_t*>(bl);
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // stage W'[o][c] = W[o][c] * gamma_l[c] (16 chunks of 8 channels per row)
-#pragma unroll 4
-  for (int c = tid; c < M * 16; c += 64 * TB_WAVES) {
-    const int R = c >> 4, k = c & 15, l = R / H;
-    const opx8 wv = ld_x8(W + R * C + 8 * k);
-    opx8 o;
+  float* stg = reinterpret_cast<float*>(bl + TbLds::ST) + wid * DP_ROWS * TB_SP;
+  float* sb = reinterpret_cast<float*>(bl + TbLds::OFF);
+  const int nob = M / 32, g4 = lane >> 4, q4 = lane & 15;
+  DirectLn<C, 8> ln;
+  auto fetch = [&](int g) PF_INLINE {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) o[u] = (op_t)((float)wv[u] * lnw[l * C + 8 * k + u]);
-    st_x8(&sw[slot16(R, k)], o);
+    for (int it = 0; it < 2; ++it)
+#pragma unroll
+      for (int v = 0; v < 2; ++v) ln.x[it][v] = group_row4(z, g, rows, 8 * wid + 4 * it + g4, 64 * v + 4 * q4);
+  };
+  if (wid < 8) fetch(blockIdx.x);
+  ln.load_gamma(nullptr, lane);
+  DirectW<C> w[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int ob = wid + TB_WAVES * k;
+    if (ob >= nob) continue;
+    w[k].load(W + (long)32 * ob * C, lane);
+    w[k].turn(reinterpret_cast<op_t*>(stg), lane);
+    const int l = (32 * ob + m) / H;   // this lane's row's layer
+    const float b = direct_wbeta<C / 16>(w[k].v, lnb + l * C, h);
+    w[k].fold(lnw + l * C, h);
+    if (h == 0) sb[32 * ob + m] = b;
   }
-  // b'[o] = sum_c W[o][c] beta_l[c]: one wave per output row, two channels per lane
-#pragma unroll 4
-  for (int R = wid; R < M; R += TB_WAVES) {
-    const int l = R / H;
-    float v = (float)W[R * C + lane] * lnb[l * C + lane] + (float)W[R * C + 64 + lane] * lnb[l * C + 64 + lane];
-    v = wave_sum(v);
-    if (lane == 0) sb[R] = v;
-  }
-  __syncthreads();
-  const long ntiles = (rows + 31) / 32;
-  const int nob = M / 32;
-  for (long t = (long)blockIdx.x * TB_WAVES + wid; t < ntiles; t += (long)gridDim.x * TB_WAVES) {
-    const long p0 = 32 * t;
-    const bool live = p0 + m < rows;
-    opx8 xf[8];
-    {
-      float x[64];
-      load_row128_frag(z + min(p0 + m, rows - 1) * C, h, x);
-      ln128_norm_to_frag(x, eps, xf);
-    }
-    if (layout == 0) {
-      // D[pair][output]: lane (output m, h) holds pairs acc_row(r, h), so each store
-      // instruction writes two full 128-byte runs of one pair's row
-#pragma unroll 1
-      for (int ob = 0; ob < nob; ++ob) {
+  int buf = 0;
+  for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x, buf ^= 1) {
+    op_t* sxb = sx + buf * DP_ROWS * LW;
+    if (wid < 8) ln.store(sxb, eps, wid, lane);
+    __syncthreads();   // sx[buf] is whole; every wave is done with sx[buf ^ 1]
+    if (wid < 8 && gi + (int)gridDim.x < ngroups) fetch(gi + gridDim.x);
+    const long p0 = (long)DP_ROWS * gi;
+    const int left = (int)min((long)DP_ROWS, rows - p0);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int ob = wid + TB_WAVES * k;
+      if (ob >= nob) continue;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
         f32x16 acc = zero16();
 #pragma unroll
-        for (int s8 = 0; s8 < 8; ++s8) acc = mfma32(xf[s8], ld_x8(&sw[slot16(32 * ob + m, 2 * s8 + h)]), acc);
-        const float bo = sb[32 * ob + m];
+        for (int s = 0; s < C / 16; ++s)   // D[output][pair]
+          acc = mfma32(w[k].v[s], ld_x8(sxb + (32 * t + m) * LW + 16 * s + 8 * h), acc);
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr) {
-          const long p = p0 + acc_row(rr, h);
-          if (p < rows) out[p * M + 32 * ob + m] = scale * (acc[rr] + bo);
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 b4 = *reinterpret_cast<const f32x4*>(sb + 32 * ob + 8 * g + 4 * h);
+          f32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = scale * (acc[4 * g + e] + b4[e]);
+          if constexpr (LAYOUT == 0) {
+            *reinterpret_cast<f32x4*>(stg + (32 * t + m) * TB_SP + 8 * g + 4 * h) = v;
+          } else {
+            int zl = lane;
+            asm volatile("" : "+v"(zl));   // the address is formed here, not kept across the loop
+            const int pr = 32 * t + (zl & 31);
+            if (pr < left)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                (out + (long)(32 * ob + 8 * g + e) * rows + p0)[(long)(4 * (zl >> 5)) * rows + pr] = v[e];
+          }
         }
       }
-    } else {
-      // D[output][pair]: lanes write 32 consecutive pairs of one output plane
-#pragma unroll 1
-      for (int ob = 0; ob < nob; ++ob) {
-        f32x16 acc = zero16();
+      if constexpr (LAYOUT == 0) {   // (a wave's LDS accesses complete in order)
+        char* obase = reinterpret_cast<char*>(out + p0 * M + 32 * ob);
 #pragma unroll
-        for (int s8 = 0; s8 < 8; ++s8) acc = mfma32(ld_x8(&sw[slot16(32 * ob + m, 2 * s8 + h)]), xf[s8], acc);
-        if (live)
-#pragma unroll
-          for (int rr = 0; rr < 16; ++rr) {
-            const int o = 32 * ob + acc_row(rr, h);
-            out[(long)o * rows + p0 + m] = scale * (acc[rr] + sb[o]);
-          }
+        for (int i = 0; i < 8; ++i) {
+          const int rr = 8 * i + (lane >> 3), c = 4 * (lane & 7);
+          if (rr < left)
+            *reinterpret_cast<f32x4_any*>(obase + 4u * ((uint32_t)rr * (uint32_t)M + c)) =
+                *reinterpret_cast<const f32x4*>(stg + rr * TB_SP + c);
+        }
       }
     }
   }
 }
 
-int launch_grid(long rows, int waves) {
-  const int cus = device_cus();
-  if (cus <= 0) return -1;
-  const long tiles = (rows + 31) / 32;
-  return (int)min((long)cus, (tiles + waves - 1) / waves);
+// groups of 64 rows and the workgroups that walk them (0: the device cannot be queried)
+int group_grid(long rows, int* ngroups) {
+  const long g = (rows + DP_ROWS - 1) / DP_ROWS;
+  *ngroups = (int)g;
+  return (int)min((long)max(device_cus(), 0), g);
 }
 
 }  // namespace
@@ -206,10 +258,13 @@ extern "C" int pf_pair_cond_proj_fwd(const float* z, const float* rel_pos, const
   if (!z || !rel_pos || !ln_w || !ln_b || !W || !out) return pf_fail(PF_E_INVALID, "pf_pair_cond_proj_fwd: null pointer");
   if (c_z != C || rows <= 0) return pf_fail(PF_E_INVALID, "pf_pair_cond_proj_fwd: need c_z = 128 and rows > 0 (got %d, %ld)", c_z, rows);
   if (out == z || out == rel_pos) return pf_fail(PF_E_INVALID, "pf_pair_cond_proj_fwd: out must not alias an input");
-  const int grid = launch_grid(rows, DF_WAVES);
+  if (rows >= (1l << 36)) return pf_fail(PF_E_INVALID, "pf_pair_cond_proj_fwd: shape too large");
+  int ngroups = 0;
+  const int grid = group_grid(rows, &ngroups);
   if (grid <= 0) return pf_fail(PF_E_LAUNCH, "pf_pair_cond_proj_fwd: cannot query the device");
-  cond_proj_kernel<<<grid, 64 * DF_WAVES, 0, (hipStream_t)stream>>>(z, rel_pos, ln_w, ln_b, (const op_t*)W, out, rows,
-                                                                    eps);
+  if (const int rc = pf_reserve_lds((const void*)cond_proj_kernel, CpLds::BYTES, "cond_proj_kernel")) return rc;
+  cond_proj_kernel<<<grid, 64 * CP_WAVES, CpLds::BYTES, (hipStream_t)stream>>>(z, rel_pos, ln_w, ln_b, (const op_t*)W,
+                                                                              out, rows, ngroups, eps);
   PF_CHECK_LAUNCH("cond_proj_kernel");
   return PF_OK;
 }
@@ -224,10 +279,13 @@ extern "C" int pf_token_pair_bias_fwd(const float* z, const float* ln_w, const f
                    "pf_token_pair_bias_fwd: need c_z = 128, n_layers * n_heads a multiple of 32 up to %d, layout 0/1 "
                    "(got c_z=%d L=%d H=%d layout=%d rows=%ld)", TB_MAX_OUT, c_z, n_layers, n_heads, layout, rows);
   if (rows * M >= (1l << 40)) return pf_fail(PF_E_INVALID, "pf_token_pair_bias_fwd: shape too large");
-  const int grid = launch_grid(rows, TB_WAVES);
+  int ngroups = 0;
+  const int grid = group_grid(rows, &ngroups);
   if (grid <= 0) return pf_fail(PF_E_LAUNCH, "pf_token_pair_bias_fwd: cannot query the device");
-  token_bias_kernel<<<grid, 64 * TB_WAVES, 0, (hipStream_t)stream>>>(z, ln_w, ln_b, (const op_t*)W, out, rows, (int)M,
-                                                                     n_heads, layout, scale, eps);
+  auto kern = layout == 0 ? token_bias_kernel<0> : token_bias_kernel<1>;
+  if (const int rc = pf_reserve_lds((const void*)kern, TbLds::BYTES, "token_bias_kernel")) return rc;
+  kern<<<grid, 64 * TB_WAVES, TbLds::BYTES, (hipStream_t)stream>>>(z, ln_w, ln_b, (const op_t*)W, out, rows, ngroups,
+                                                                  (int)M, n_heads, scale, eps);
   PF_CHECK_LAUNCH("token_bias_kernel");
   return PF_OK;
 }
