@@ -8,6 +8,7 @@ import torch
 
 from oracle import pairformer_ref as ref
 from tt_boltz_amd import ops, pairformer
+from test_gpu_fast import F32_MAX, F32_MEAN, _mx8_trimul_w, check as check_fast
 from test_gpu_parity import _inputs, _sub_w, check
 
 pytestmark = pytest.mark.gpu
@@ -236,6 +237,27 @@ def test_transition_direct_pair_bias(gpu, B, N):
     got, want = (t[start:start + B * 16 * N * N * 4].view(torch.float32) for t in ws)
     # one LayerNorm each, summed in another order: op_t rounding ties aside the bits agree
     check("fused pair bias", got, want, max_tol=5e-3, mean_tol=1e-4)
+
+
+# ------------------------------------------------------------------------------ fast-mode trimul
+@pytest.mark.parametrize("B,N", [(1, 128), (2, 128), (1, 384), (1, 512)])
+@pytest.mark.parametrize("incoming", [False, True])
+@pytest.mark.parametrize("masked", [False, True])
+def test_trimul_mx8_groups(gpu, B, N, incoming, masked):
+    """One group of 128 positions per workgroup and several, a batch, no mask and one with single
+    masked pairs everywhere; the tolerances of the fast-mode parity tests."""
+    w = _sub_w(5, "tri_mul_in" if incoming else "tri_mul_out")
+    z = torch.cat([_inputs(N, 5 + b)[1] for b in range(B)])
+    pm = torch.cat([_inputs(N, 5 + b, pad_tail=7, rand_mask=True)[3] for b in range(B)])
+    pm = pm if masked else torch.ones_like(pm)
+    wd = _mx8_trimul_w(w, gpu)
+    zd, out = z.to(gpu), torch.empty_like(z, device=gpu)
+    ws = ops.workspace(ops.trimul_mx8_workspace_bytes(B, N), gpu)
+    ops.launch_trimul_mx8(zd, out, pm.to(gpu).contiguous() if masked else None, wd, int(incoming), ws,
+                          accumulate=False)
+    want = ref.triangle_multiplication(zd, pm.to(gpu), {k: v.to(gpu) for k, v in w.items()},
+                                       "incoming" if incoming else "outgoing")
+    check_fast("trimul mx8", out, want, F32_MAX, F32_MEAN)
 
 
 # ------------------------------------------------------------------------------ diffusion conditioning

@@ -137,16 +137,6 @@ PF_DEV i32x8 wfrag128(const uint8_t* lds, int row, int s, int h) {
   return cat_i32x4(*reinterpret_cast<const i32x4*>(p), *reinterpret_cast<const i32x4*>(p + 32));
 }
 
-// Copy an fp8 [rows][128] matrix (and its [rows][4] scales) from global to LDS.
-PF_DEV void stage_w128(const uint8_t* __restrict__ q, const uint8_t* __restrict__ sc, int rows, uint8_t* lq,
-                       uint8_t* ls, int tid, int nthreads) {
-  for (int c = tid; c < rows * 8; c += nthreads)
-    *reinterpret_cast<i32x4*>(lq + (c >> 3) * WROW + (c & 7) * 16) =
-        *reinterpret_cast<const i32x4*>(q + (c >> 3) * 128 + (c & 7) * 16);
-  for (int c = tid; c < rows; c += nthreads)
-    *reinterpret_cast<int*>(ls + 4 * c) = *reinterpret_cast<const int*>(sc + 4 * c);
-}
-
 // ---------------------------------------------------------------------------------
 // Quantize rows of K fp32 values in blocks of 32 along K.  One thread per block.
 // perm = 1 stores each block in the order its values come out of a 32x32 MFMA
@@ -178,111 +168,171 @@ __global__ void mx8_quantize_kernel(const float* __restrict__ x, uint8_t* __rest
 }
 
 // ---------------------------------------------------------------------------------
-// Triangle multiplication input projection.  One wave = 32 consecutive positions of
-// one operand-plane row; p_in / g_in ([256][128] fp8 each) resident in LDS.  The
-// projection is computed as D[position][channel], so a lane holds one channel for 16
-// of the 32 positions and the partner lane the other 16: the MX block of the
-// contraction (32 consecutive k = positions) is reduced with one exchange.  The LayerNorm's
-// gamma / beta sit in LDS after the weights; the next tile's z rows (and mask entry) are
-// loaded while a tile is computed; MASKED = false skips the mask.
+// Triangle multiplication input projection.
 //   A8/B8 planes [B][128][N][N] e4m3, scales SA/SB [B][128][N][N/32] E8M0.
+// Persistent, two 8-wave workgroups per CU; a workgroup takes groups of 128 consecutive positions
+// of one operand-plane row.  Wave w keeps the p_in / g_in rows 32 w .. 32 w + 31 in registers (40
+// VGPRs); the workgroup normalizes and quantizes a group's rows into LDS once (16 lanes a row,
+// fully coalesced; the next group's rows are loaded meanwhile) and every wave reads its MFMA
+// fragments from there.  The projection is computed as D[position][channel]: a lane holds one
+// channel for 16 of a tile's 32 positions and the partner lane the other 16, so the contraction's
+// MX block (32 consecutive k = positions) is reduced with one exchange.  A channel's 128 bytes
+// (its four blocks) and four scale bytes leave as one line and one dword.
+// Bound by HBM (z read, the planes written: 61 us at the copy rate for N = 640).  Against weights in
+// LDS, a lane per row and 32-byte stores: N = 128 14.9 -> 11.9 us, 384 48 -> 39, 640 119 -> 98, 1024
+// 272 -> 221.
 // ---------------------------------------------------------------------------------
-constexpr size_t TM8P_LDS = 2 * 256 * WROW + 2 * 256 * 4 + 2 * C * 4;   // + LayerNorm gamma, beta
+constexpr int TM8P_ROWS = 128, TM8P_WAVES = 8;
+// LDS: the quantized rows (two groups), their scale dwords, the waves' output stages, the masks,
+// the LayerNorm's gamma and beta
+constexpr int T8_X = TM8P_ROWS * WROW, T8_S = TM8P_ROWS * 4, T8_O = 32 * WROW;
+constexpr size_t TM8P_LDS = 2 * T8_X + 2 * T8_S + TM8P_WAVES * T8_O + 2 * TM8P_ROWS * 4 + 2 * C * 4;
+
+PF_DEV float row8_max(float v) {   // over each 8 consecutive lanes
+  v = fmaxf(v, dpp_f<0xB1>(v));
+  v = fmaxf(v, dpp_f<0x4E>(v));
+  return fmaxf(v, dpp_f<0x141>(v));
+}
 
 template <bool MASKED>
-__global__ __launch_bounds__(256, 2) void tm8_proj_kernel(
+__global__ __launch_bounds__(64 * TM8P_WAVES, 4) void tm8_proj_kernel(
     const float* __restrict__ z, const float* __restrict__ mask, const float* __restrict__ lnw,
     const float* __restrict__ lnb, const uint8_t* __restrict__ wp_q, const uint8_t* __restrict__ wp_s,
     const uint8_t* __restrict__ wg_q, const uint8_t* __restrict__ wg_s, uint8_t* __restrict__ A8,
-    uint8_t* __restrict__ B8, uint8_t* __restrict__ SA, uint8_t* __restrict__ SB, int B, int N, int incoming,
+    uint8_t* __restrict__ B8, uint8_t* __restrict__ SA, uint8_t* __restrict__ SB, int ngroups, int N, int incoming,
     float eps) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds8[];
-  uint8_t* lp = lds8;
-  uint8_t* lg = lp + 256 * WROW;
-  uint8_t* lps = lg + 256 * WROW;
-  uint8_t* lgs = lps + 256 * 4;
-  float* lnp = reinterpret_cast<float*>(lgs + 256 * 4);   // gamma [128], beta [128]
-  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
+  uint8_t* sx = lds8;                                     // [2][128][WROW]
+  uint8_t* ss = sx + 2 * T8_X;                            // [2][128][4]
+  uint8_t* so = ss + 2 * T8_S;                            // [8][32][WROW]
+  float* smask = reinterpret_cast<float*>(so + TM8P_WAVES * T8_O);   // [2][128]
+  float* lnp = smask + 2 * TM8P_ROWS;                     // gamma [128], beta [128]
+  const int tid = threadIdx.x;
+  int lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  stage_w128(wp_q, wp_s, 256, lp, lps, tid, 256);
-  stage_w128(wg_q, wg_s, 256, lg, lgs, tid, 256);
+  const int NB = N / 32;
+  // pair of a group's first position (uniform), pairs between neighbouring positions
+  auto pair0_of = [&](const PosTile& pt) PF_INLINE -> long {
+    return incoming ? ((long)pt.b * N + pt.c0) * N + pt.r : ((long)pt.b * N + pt.r) * N + pt.c0;
+  };
+  const uint32_t pstep = incoming ? N : 1;
+  // wave wid normalizes rows 16 wid .. 16 wid + 15 of a group; lane (row 4 it + (lane >> 4), q)
+  // holds channels 4 q .. and 64 + 4 q .. of it
+  int rq = lane & 15, rg = 16 * wid + (lane >> 4);
+  f32x4 x[4][2];
+  float mv = 1.f;
+  auto fetch = [&](int g) PF_INLINE {
+    const long p0 = pair0_of(pos_tile(4u * g, N));
+    const char* base = reinterpret_cast<const char*>(z + p0 * C);
+    uint32_t off = 4u * (pstep * rg * C + 4 * rq);   // (bytes; below 2^31 for every N that is taken)
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      x[it][0] = *reinterpret_cast<const f32x4*>(base + off);
+      x[it][1] = *reinterpret_cast<const f32x4*>(base + off + 256);
+      off += 16u * pstep * C;
+    }
+    if (MASKED) mv = mask[p0 + (long)(pstep * (rg + rq % 4 * 4))];   // row rg + 4 (q % 4) of the wave's 16
+  };
+  auto normalize = [&](int buf) PF_INLINE {
+    f32x4 gm[2], bt[2];
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      gm[v] = *reinterpret_cast<const f32x4*>(lnp + 64 * v + 4 * rq);
+      bt[v] = *reinterpret_cast<const f32x4*>(lnp + C + 64 * v + 4 * rq);
+    }
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const f32x4 a = x[it][0], b = x[it][1];
+      const float mean = row16_sum((a[0] + a[1]) + (a[2] + a[3]) + (b[0] + b[1]) + (b[2] + b[3])) * (1.f / C);
+      float var = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float d = a[e] - mean, f = b[e] - mean;
+        var += d * d + f * f;
+      }
+      const float rstd = rsqrtf(row16_sum(var) * (1.f / C) + eps);
+      const int r = rg + 4 * it;
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {   // channels 64 v + 4 q ..: MX block 2 v + (q >> 3), eight lanes
+        float y[4], am = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          y[e] = (x[it][v][e] - mean) * rstd * gm[v][e] + bt[v][e];
+          am = fmaxf(am, fabsf(y[e]));
+        }
+        const int byte = mx_scale_byte(row8_max(am));
+        const float inv = mx_inv_scale(byte);
+        *reinterpret_cast<int*>(sx + buf * T8_X + r * WROW + 64 * v + 4 * rq) =
+            e4m3_pack4(y[0] * inv, y[1] * inv, y[2] * inv, y[3] * inv);
+        if ((rq & 7) == 0) ss[buf * T8_S + 4 * r + 2 * v + (rq >> 3)] = (uint8_t)byte;
+      }
+    }
+    if (MASKED && rq < 4) smask[buf * TM8P_ROWS + rg + 4 * rq] = mv;
+  };
+
+  fetch(blockIdx.x);
+  i32x8 wp[2], wg[2];
+  int sp[2], sg[2];
+  {
+    const int h = lane >> 5, row = 32 * wid + (lane & 31);   // output unit of this lane's column
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const uint8_t* p = wp_q + row * C + 64 * s + 16 * h;
+      const uint8_t* g = wg_q + row * C + 64 * s + 16 * h;
+      wp[s] = cat_i32x4(*reinterpret_cast<const i32x4*>(p), *reinterpret_cast<const i32x4*>(p + 32));
+      wg[s] = cat_i32x4(*reinterpret_cast<const i32x4*>(g), *reinterpret_cast<const i32x4*>(g + 32));
+      sp[s] = wp_s[4 * row + 2 * s + h];
+      sg[s] = wg_s[4 * row + 2 * s + h];
+    }
+  }
   if (tid < C) {
     lnp[tid] = lnw[tid];
     lnp[C + tid] = lnb[tid];
   }
   __syncthreads();
-
-  uint32_t ln_a = lds_addr(lnp) + 64 * h;   // gamma of this lane half's first channel
-  asm volatile("" : "+v"(ln_a));
-  const uint32_t ntiles = (uint32_t)B * N * N / 32;
-  const uint32_t stride = gridDim.x * 4;
-  const int NB = N / 32;
-  auto zpair = [&](uint32_t tile) -> long {
-    const PosTile pt = pos_tile(tile, N);
-    const int zi = incoming ? pt.c0 + m : pt.r;
-    const int zj = incoming ? pt.r : pt.c0 + m;
-    return ((long)pt.b * N + zi) * N + zj;
-  };
-  // the next tile's z row (and mask entry) are loaded while this tile is computed
-  float xn[4][16];
-  float mn = 1.f;
-  uint32_t tile = blockIdx.x * 4 + wid;
-  if (tile < ntiles) {
-    const long pair = zpair(tile);
-    load_row128_x8order(z + pair * C, h, xn);
-    if (MASKED) mn = mask[pair];
-  }
-  for (; tile < ntiles; tile += stride) {
-    // the LayerNorm parameters are re-read from LDS each tile instead of pinning 128 VGPRs
-    asm volatile("" ::: "memory");
-    const PosTile pt = pos_tile(tile, N);
-    const int b = pt.b, orow = pt.r, ocol0 = pt.c0;
-    X8 xq;
-    float mr[16];
-    {
-      float x[4][16];
+  uint8_t* stg = so + wid * T8_O;
+  int buf = 0;
+  for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x, buf ^= 1) {
+    // opaque: addresses are formed again in each group, not kept in registers
+    asm volatile("" : "+v"(lane), "+v"(rq), "+v"(rg));
+    const int h = lane >> 5, m = lane & 31;
+    normalize(buf);
+    __syncthreads();   // buffer buf is whole; every wave is done with the other
+    if (gi + (int)gridDim.x < ngroups) fetch(gi + gridDim.x);
+    int bytes = 0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int t = 0; t < 16; ++t) x[j][t] = xn[j][t];
-      const float maskv = mn;
-      if (tile + stride < ntiles) {
-        const long pair2 = zpair(tile + stride);
-        load_row128_x8order(z + pair2 * C, h, xn);
-        if (MASKED) mn = mask[pair2];
-      }
-      ln128_to_x8_lds(x, ln_a, eps, xq, h);
-      if (MASKED) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mr[r] = __shfl(maskv, acc_row(r, h));
-      }
-    }
-
-    // unrolled, so that the next tile's wait for its prefetched rows can count the stores issued
-    // after them; the empty asm keeps each block's LDS reads in its own block
-#pragma unroll
-    for (int cb = 0; cb < 8; ++cb) {
-      asm volatile("" ::: "memory");
-      const int row = 32 * cb + m;   // weight row = output unit of this lane's column
+    for (int t = 0; t < 4; ++t) {
+      __builtin_amdgcn_sched_barrier(0);   // one tile's accumulators at a time
+      const uint8_t* xrow = sx + buf * T8_X + (32 * t + m) * WROW + 16 * h;
+      const uint32_t sc = *reinterpret_cast<const uint32_t*>(ss + buf * T8_S + 4 * (32 * t + m)) >> (8 * h);
       f32x16 P = zero16(), G = zero16();
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        P = mfma8(xq.q[s], wfrag128(lp, row, s, h), P, xq.sc[s], lps[4 * row + 2 * s + h]);
-        G = mfma8(xq.q[s], wfrag128(lg, row, s, h), G, xq.sc[s], lgs[4 * row + 2 * s + h]);
+        const i32x8 xf = cat_i32x4(*reinterpret_cast<const i32x4*>(xrow + 64 * s),
+                                   *reinterpret_cast<const i32x4*>(xrow + 64 * s + 32));
+        const int xs = (int)((sc >> (16 * s)) & 0xffu);
+        P = mfma8(xf, wp[s], P, xs, sp[s]);
+        G = mfma8(xf, wg[s], G, xs, sg[s]);
       }
       float v[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        v[r] = P[r] * sigmoidf_fast(G[r]);
-        if (MASKED) v[r] *= mr[r];
+      for (int g = 0; g < 4; ++g) {   // lane half h holds positions 8 g + 4 h + e
+        f32x4 mr = {1.f, 1.f, 1.f, 1.f};
+        if (MASKED) {
+          asm volatile("" ::: "memory");   // four mask values at a time
+          mr = *reinterpret_cast<const f32x4*>(smask + buf * TM8P_ROWS + 32 * t + 8 * g + 4 * h);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[4 * g + e] = P[4 * g + e] * sigmoidf_fast(G[4 * g + e]);
+          if (MASKED) v[4 * g + e] *= mr[e];
+        }
       }
       int byte;
       const i32x4 q = quantize16(v, byte);
-      const int ch = 32 * (cb & 3) + m;
-      uint8_t* plane = (cb < 4 ? A8 : B8) + (((long)b * C + ch) * N + orow) * N + ocol0;
-      // dword g of lane half h holds positions 8g + 4h .. +3; one v_permlane32_swap per
-      // dword pair gives half 0 positions 0..15 and half 1 positions 16..31, so the
-      // 32-byte plane-row segment leaves as two 16-byte stores instead of eight 4-byte ones
+      bytes |= byte << (8 * t);
+      // dword g of lane half h holds positions 8g + 4h .. +3; one v_permlane32_swap per dword pair
+      // gives half 0 positions 0..15 and half 1 positions 16..31
       i32x4 o;
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
@@ -291,9 +341,18 @@ __global__ __launch_bounds__(256, 2) void tm8_proj_kernel(
         o[2 * k] = h ? (int)r[0] : q[k];
         o[2 * k + 1] = h ? q[2 + k] : (int)r[1];
       }
-      *reinterpret_cast<i32x4*>(plane + 16 * h) = o;
-      if (h == 0) (cb < 4 ? SA : SB)[(((long)b * C + ch) * N + orow) * NB + ocol0 / 32] = (uint8_t)byte;
+      *reinterpret_cast<i32x4*>(stg + m * WROW + 32 * t + 16 * h) = o;
     }
+    const PosTile pt = pos_tile(4u * gi, N);
+    const long prow = ((long)pt.b * C + 32 * (wid & 3)) * N + pt.r;   // plane row of the block's first channel
+    uint8_t* dst = (wid < 4 ? A8 : B8) + prow * N + pt.c0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {   // eight lanes write a channel's 128 bytes
+      const int ch = 8 * q + (lane >> 3), c = 16 * (lane & 7);
+      *reinterpret_cast<i32x4*>(dst + (long)ch * N * N + c) = *reinterpret_cast<const i32x4*>(stg + ch * WROW + c);
+    }
+    if (h == 0)
+      *reinterpret_cast<int*>((wid < 4 ? SA : SB) + (prow + (long)m * N) * NB + pt.c0 / 32) = bytes;
   }
 }
 
@@ -720,7 +779,6 @@ Tm8Buffers tm8_buffers(void* ws, int B, int N) {
 }
 
 // grid of a wave-tile loop: enough workgroups to fill the chip several times over
-int tile_grid(long ntiles) { const long g = (ntiles + 3) / 4; return (int)(g < 2048 ? g : 2048); }
 
 }  // namespace
 
@@ -776,17 +834,15 @@ extern "C" int pf_trimul_mx8_fwd(const pf_trimul_mx8_args* a) {
   hipStream_t st = (hipStream_t)a->stream;
   const int B = a->B, N = a->N;
   Tm8Buffers t = tm8_buffers(a->workspace, B, N);
-  const long ntiles = (long)B * N * N / 32;
   const int cus = device_cus();
   if (cus <= 0) return pf_fail(PF_E_LAUNCH, "pf_trimul_mx8_fwd: cannot query the device");
-  // up to 2048 workgroups (several rounds per CU): a persistent grid of two per CU projects
-  // as fast but leaves the planes in an order the contraction reads 6 % slower
-  const int grid = tile_grid(ntiles);
+  const int ngroups = (int)((long)B * N * N / TM8P_ROWS);
   // the A plane (channels 0..127 of the projection) holds a, the B plane b; the
   // 2C-row p_in / g_in matrices are [a rows ; b rows]
-  (a->pair_mask ? tm8_proj_kernel<true> : tm8_proj_kernel<false>)<<<grid, 256, TM8P_LDS, st>>>(
+  (a->pair_mask ? tm8_proj_kernel<true> : tm8_proj_kernel<false>)<<<min(ngroups, 2 * cus), 64 * TM8P_WAVES, TM8P_LDS,
+                                                                     st>>>(
       a->z_in, a->pair_mask, a->norm_in_w, a->norm_in_b, (const uint8_t*)a->p_in_q, (const uint8_t*)a->p_in_s,
-      (const uint8_t*)a->g_in_q, (const uint8_t*)a->g_in_s, t.A8, t.B8, t.SA, t.SB, B, N, a->direction, a->eps);
+      (const uint8_t*)a->g_in_q, (const uint8_t*)a->g_in_s, t.A8, t.B8, t.SA, t.SB, ngroups, N, a->direction, a->eps);
   PF_CHECK_LAUNCH("tm8_proj_kernel");
   const int tpd = (N + BT - 1) / BT;
   const int total = B * C * tpd * tpd;
