@@ -6,10 +6,10 @@ against the fp32 oracle.
 import pytest
 import torch
 
-from oracle import pairformer_ref as ref
+from oracle import msa_ref, pairformer_ref as ref
 from tt_boltz_amd import ops, pairformer
 from test_gpu_fast import F32_MAX, F32_MEAN, _mx8_trimul_w, check as check_fast
-from test_gpu_parity import _inputs, _sub_w, check
+from test_gpu_parity import _inputs, _msa_sub, _sub_w, check
 
 pytestmark = pytest.mark.gpu
 
@@ -298,3 +298,28 @@ def test_cond_proj_groups(gpu, rows):
     ops.launch_pair_cond_proj(z.to(gpu), r.to(gpu), lw.to(gpu), lb.to(gpu), ops.opw(w, gpu), out[:rows])
     check("cond proj", out[:rows], want)
     assert (out[rows:] == 7.0).all()
+
+
+@pytest.mark.parametrize("B,S,N", [(1, 1, 64), (1, 31, 128), (2, 33, 64), (1, 700, 192)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_pair_weighted_averaging_groups(gpu, B, S, N, masked):
+    """One and several groups of 64 tokens and tiles of 32 sequences a workgroup, remainders of
+    sequences, batches; into another tensor and in place."""
+    w = {k: v.to(gpu) for k, v in _msa_sub(5, "pair_weighted_averaging").items()}
+    g = torch.Generator().manual_seed(S + N)
+    m = torch.randn((B, S, N, 64), generator=g).to(gpu)
+    z = torch.randn((B, N, N, 128), generator=g).to(gpu)
+    pm = torch.ones((B, N, N), device=gpu)
+    if masked:
+        pm[:, :, N - 13:] = 0
+    want = msa_ref.pair_weighted_averaging(m, z, pm, w)
+    wd = ops.convert_weights(w, gpu, ops.DEFAULT_VARIANT)
+    ws = ops.workspace(ops.pwa_workspace_bytes(B, S, N), gpu)
+    out = torch.full((B * S * N + 64, 64), 7.0, device=gpu)
+    dst = out[:B * S * N].view_as(m)
+    ops.launch_pwa(m, z, pm if masked else None, dst, wd, ws, accumulate=False)
+    check(f"pwa B={B} S={S} N={N}", dst, want)
+    assert (out[B * S * N:] == 7.0).all()
+    want = m + dst
+    ops.launch_pwa(m, z, pm if masked else None, m, wd, ws)
+    assert torch.equal(m, want)

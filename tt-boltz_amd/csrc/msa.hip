@@ -212,39 +212,71 @@ __global__ __launch_bounds__(256) void pwa_softmax_kernel(const float* __restric
   for (int j = lane; j < N; j += 64) w[j] = (op_t)(exp2_fast(val(j) - mx) * inv);
 }
 
-// v projection: a wave takes 32 consecutive tokens j of one (b, s); W_m [256][64] sits in
-// LDS (128-byte rows, 16-byte chunk c of row R at slot c ^ swz8r(R)).  D[(h, d)][j]: lane
-// (j, half) writes v_t rows ((b*H + h)*S + s)*32 + d at column j (64 contiguous bytes per
-// row and register).
-__global__ __launch_bounds__(512) void pwa_proj_kernel(
+// v projection: persistent, a workgroup walks groups of 64 consecutive tokens j of one (b, s).
+// Wave w keeps head w's 32 rows of W_m in registers; the workgroup normalizes a group once into
+// LDS (16 lanes a row, two stages: one barrier a group) and every head reads it there.  D[j][d]
+// goes through the wave's own LDS rows, so that v_t row ((b*H + h)*S + s)*32 + d leaves as the
+// whole 128 bytes of its 64 tokens.  Bound by HBM (m read, v_t written: 6.2 TB/s at N = 512, S = 1024).
+// Against W_m staged in LDS for every 8 tiles and 64-byte pieces of rows stored: 89 -> 65 us there.
+constexpr int PVP = CM + 8;   // LDS pitch of 64 op_t
+__global__ __launch_bounds__(64 * PH, 4) void pwa_proj_kernel(
     const float* __restrict__ m, const float* __restrict__ lnw, const float* __restrict__ lnb,
-    const op_t* __restrict__ wm, op_t* __restrict__ vt, int B, int S, int N, float eps) {
-  __shared__ __attribute__((aligned(16))) op_t sw[PHD * CM];
-  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, mm = lane & 31;
+    const op_t* __restrict__ wm, op_t* __restrict__ vt, long ngroups, int S, int N, float eps) {
+  __shared__ __attribute__((aligned(16))) op_t sx[2][64 * PVP];
+  __shared__ __attribute__((aligned(16))) op_t sv[PH][PD * PVP];
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, mm = lane & 31, g4 = lane >> 4, q4 = lane & 15;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  for (int c = tid; c < PHD * 8; c += 512) {
-    const int R = c >> 3, k = c & 7;
-    st_x8(sw + R * CM + 8 * (k ^ swz8r(R)), ld_x8(wm + R * CM + 8 * k));
-  }
-  __syncthreads();
-  const int nj = N / 32;
-  const long wv = (long)blockIdx.x * 8 + wid;
-  if (wv >= (long)B * S * nj) return;
-  const int j0 = 32 * (int)(wv % nj);
-  const long bs = wv / nj;   // b * S + s
-  const int s = (int)(bs % S), b = (int)(bs / S);
-  opx8 xf[4];
-  ln64_to_frag(m + (bs * N + j0 + mm) * CM, h, lnw, lnb, eps, xf);
-  const int sw8 = swz8r(mm);
-#pragma unroll 1
-  for (int blk = 0; blk < PH; ++blk) {
-    f32x16 acc = zero16();
+  f32x4 x[2];   // rows 8 wid + 4 it + g4, channels 4 q4 .. + 3
+  auto fetch = [&](long g) PF_INLINE {
 #pragma unroll
-    for (int st = 0; st < 4; ++st)
-      acc = mfma32(ld_x8(sw + (32 * blk + mm) * CM + 8 * ((2 * st + h) ^ sw8)), xf[st], acc);   // rows = (h, d)
-    op_t* dst = vt + (((long)b * PH + blk) * S + s) * PD * (long)N + j0 + mm;
+    for (int it = 0; it < 2; ++it)
+      x[it] = *reinterpret_cast<const f32x4*>(m + (64 * g + 8 * wid + 4 * it + g4) * CM + 4 * q4);
+  };
+  fetch(blockIdx.x);   // the grid is at most ngroups
+  opx8 w[4];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) dst[(long)acc_row(r, h) * N] = (op_t)acc[r];
+  for (int st = 0; st < 4; ++st) w[st] = ld_x8(wm + (PD * wid + mm) * CM + 16 * st + 8 * h);
+  const f32x4 gm = *reinterpret_cast<const f32x4*>(lnw + 4 * q4), bt = *reinterpret_cast<const f32x4*>(lnb + 4 * q4);
+  const int nj = N / 64;
+  int buf = 0;
+  for (long gi = blockIdx.x; gi < ngroups; gi += gridDim.x, buf ^= 1) {
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const float mean = row16_sum((x[it][0] + x[it][1]) + (x[it][2] + x[it][3])) * (1.f / CM);
+      float var = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { const float d = x[it][e] - mean; var += d * d; }
+      const float rstd = rsqrtf(row16_sum(var) * (1.f / CM) + eps);
+      opx4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (op_t)((x[it][e] - mean) * rstd * gm[e] + bt[e]);
+      st_x4(sx[buf] + (8 * wid + 4 * it + g4) * PVP + 4 * q4, o);
+    }
+    __syncthreads();   // this stage is whole; the group before last, its last reader, is done everywhere
+    if (gi + gridDim.x < ngroups) fetch(gi + gridDim.x);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f32x16 acc = zero16();
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+        acc = mfma32(ld_x8(sx[buf] + (32 * t + mm) * PVP + 16 * st + 8 * h), w[st], acc);   // rows = token, cols = d
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        opx4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (op_t)acc[4 * g + e];
+        st_x4(sv[wid] + mm * PVP + 32 * t + 8 * g + 4 * h, o);
+      }
+    }
+    // (a wave's LDS accesses complete in order: its own rows need no barrier)
+    const long bs = gi / nj;   // b * S + s
+    const long b = bs / S, s = bs - b * S;
+    op_t* dst = vt + ((b * PH + wid) * S + s) * PD * (long)N + 64 * (gi - bs * nj);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = 8 * u + (lane >> 3), c = 8 * (lane & 7);
+      st_x8(dst + (long)r * N + c, ld_x8(sv[wid] + r * PVP + c));
+    }
   }
 }
 
@@ -469,7 +501,8 @@ extern "C" int pf_pwa_fwd(const pf_pwa_args* a) {
   if (a->workspace_bytes < need)
     return pf_fail(PF_E_INVALID, "pf_pwa_fwd: workspace too small (%zu < %zu bytes)", a->workspace_bytes, need);
   hipStream_t st = (hipStream_t)a->stream;
-  const int B = a->B, S = a->S, N = a->N;
+  const int B = a->B, S = a->S, N = a->N, cus = device_cus();
+  if (cus <= 0) return pf_fail(PF_E_LAUNCH, "pf_pwa_fwd: cannot query the device");
   const size_t bh = (size_t)B * PH, nn = (size_t)N * N, sn = (size_t)S * PD * N;
   float* logits = (float*)a->workspace;
   op_t* Wt = (op_t*)(logits + bh * nn);
@@ -479,9 +512,9 @@ extern "C" int pf_pwa_fwd(const pf_pwa_args* a) {
   if (rc) return rc;
   pwa_softmax_kernel<<<(unsigned)((bh * N + 3) / 4), 256, 0, st>>>(logits, a->pair_mask, Wt, B, N);
   PF_CHECK_LAUNCH("pwa_softmax_kernel");
-  const long vw = (long)B * S * (N / 32);
-  pwa_proj_kernel<<<(unsigned)((vw + 7) / 8), 512, 0, st>>>(a->m, a->norm_m_w, a->norm_m_b, (const op_t*)a->w_m, vt,
-                                                           B, S, N, a->eps);
+  const long vg = (long)B * S * (N / 64);
+  pwa_proj_kernel<<<(unsigned)min(2l * cus, vg), 64 * PH, 0, st>>>(a->m, a->norm_m_w, a->norm_m_b,
+                                                                  (const op_t*)a->w_m, vt, vg, S, N, a->eps);
   PF_CHECK_LAUNCH("pwa_proj_kernel");
   // rows (s, d) of v_t are the Nc dimension; S*32 is a multiple of 32
   if ((rc = pf_contract_rect(Wt, vt, O, 0, (int)bh, N, S * PD, N, 1.f, st))) return rc;
