@@ -33,12 +33,9 @@ __global__ __launch_bounds__(256) void opm_proj_kernel(
     float eps) {
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, mm = lane & 31;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nsb = Sp / 32;
-  const long wv = (long)blockIdx.x * 4 + wid;
-  if (wv >= (long)B * N * nsb) return;
-  const int sb = (int)(wv % nsb);
-  const long bi = wv / nsb;
-  const int i = (int)(bi % N), b = (int)(bi / N);
+  const int np = Sp / 64, ni = N / 2;   // 2 tokens x 64 sequences a workgroup
+  const int i = 2 * (int)(blockIdx.x % ni) + (wid >> 1);
+  const int bp = (int)(blockIdx.x / ni), b = bp / np, sb = 2 * (bp - b * np) + (wid & 1);
   const int s = 32 * sb + mm;
   const float mk = s < S ? (msa_mask ? msa_mask[((long)b * S + s) * N + i] : 1.f) : 0.f;
   const float* row = m + (((long)b * S + min(s, S - 1)) * N + i) * CM;
@@ -286,7 +283,14 @@ __global__ __launch_bounds__(64 * PH, 4) void pwa_proj_kernel(
 // block -- the B-operand order of the W_o product; each such fragment is multiplied by
 // the matching 16 bytes of O and fed to D[o][s] += W_o . og.  Residual into m in the
 // output-aligned layout (16-byte loads / stores).
-__global__ __launch_bounds__(512) void pwa_out_kernel(
+// Persistent, two workgroups per CU (64 KB of LDS each): the weights are staged once instead of
+// per 8 tiles, and O is loaded PWA_AHEAD heads ahead of its use, the first of them beside the
+// LayerNorm (4 heads spill).  The workgroup's waves take 8 consecutive tokens: 2 KB runs of a
+// sequence's row of m, where 256-byte pieces N rows apart all fell on the same memory channels.
+// N = 512, S = 1024: 155 -> 141 us (the token order alone 150, the persistent form alone 155);
+// the bytes (O and m read, m written) are 85 us at the copy rate, the sigmoids about 33.
+constexpr int PWA_AHEAD = 3;
+__global__ __launch_bounds__(512, 4) void pwa_out_kernel(
     const float* m_in, float* m_out, const float* __restrict__ lnw, const float* __restrict__ lnb,
     const op_t* __restrict__ wg, const op_t* __restrict__ wo, const op_t* __restrict__ O, int B, int S, int N,
     int accumulate, float eps) {
@@ -303,53 +307,63 @@ __global__ __launch_bounds__(512) void pwa_out_kernel(
     st_x8(so + R * PHD + 8 * (k ^ (R & 15)), ld_x8(wo + R * PHD + 8 * k));
   }
   __syncthreads();
-  const int ns = (S + 31) / 32;
-  const long wv = (long)blockIdx.x * 8 + wid;
-  if (wv >= (long)B * N * ns) return;
-  const int s0 = 32 * (int)(wv % ns);
-  const long bi = wv / ns;   // b * N + i
-  const int i = (int)(bi % N), b = (int)(bi / N);
-  const int s = min(s0 + mm, S - 1);   // rows past S are computed on a clamped row and not stored
-  const long mrow = (((long)b * S + s) * N + i) * CM;
-  opx8 xf[4];
-  ln64_to_frag(m_in + mrow, h, lnw, lnb, eps, xf);
-  const int gr = perm16(mm), sg8 = swz8r(gr);
-  f32x16 acc[2] = {zero16(), zero16()};
-#pragma unroll 1
-  for (int blk = 0; blk < PH; ++blk) {
-    f32x16 g = zero16();
+  const int ns = (S + 31) / 32, ni = N / 8, tiles = B * ns * ni;
+  const long ostep = (long)N * S * PD;   // O of the next head
+  for (int t8 = blockIdx.x; t8 < tiles; t8 += gridDim.x) {
+    const int bs = t8 / ni, i = 8 * (t8 - bs * ni) + wid;
+    const int b = bs / ns, s0 = 32 * (bs - b * ns);
+    const int s = min(s0 + mm, S - 1);   // rows past S are computed on a clamped row and not stored
+    const long mrow = (((long)b * S + s) * N + i) * CM;
+    const op_t* orow = O + ((long)b * PH * N + i) * ((long)S * PD) + (long)s * PD + 8 * h;
+    opx8 ov[PWA_AHEAD][2];
 #pragma unroll
-    for (int st = 0; st < 4; ++st)
-      g = mfma32(ld_x8(sg + (32 * blk + gr) * CM + 8 * ((2 * st + h) ^ sg8)), xf[st], g);   // rows = k (perm16)
-    const op_t* orow = O + ((long)(b * PH + blk) * N + i) * ((long)S * PD) + (long)s * PD + 8 * h;
+    for (int blk = 0; blk < PWA_AHEAD; ++blk)
 #pragma unroll
-    for (int sp = 0; sp < 2; ++sp) {
-      const opx8 ov = ld_x8(orow + 16 * sp);
-      opx8 og;
+      for (int sp = 0; sp < 2; ++sp) ov[blk][sp] = ld_x8(orow + blk * ostep + 16 * sp);
+    opx8 xf[4];
+    const float *gamma = lnw, *beta = lnb;
+    asm volatile("" : "+s"(gamma), "+s"(beta));   // (their 64 values are not kept over the loop)
+    ln64_to_frag(m_in + mrow, h, gamma, beta, eps, xf);
+    f32x16 acc[2] = {zero16(), zero16()};
 #pragma unroll
-      for (int t = 0; t < 8; ++t) og[t] = (op_t)((float)ov[t] * sigmoidf_fast(g[8 * sp + t]));
-      const int kc = 2 * (2 * blk + sp) + h;   // 16-byte chunk of the W_o row: k = 32 blk + 16 sp + 8 h
+    for (int blk = 0; blk < PH; ++blk) {
+      int mr = mm;
+      asm volatile("" : "+v"(mr) : : "memory");   // one head's weights and LDS addresses at a time in registers
+      const int gr = perm16(mr), sg8 = swz8r(gr);
+      f32x16 g = zero16();
 #pragma unroll
-      for (int ob = 0; ob < 2; ++ob) {
-        const int R = 32 * ob + mm;
-        acc[ob] = mfma32(ld_x8(so + R * PHD + 8 * (kc ^ (R & 15))), og, acc[ob]);   // rows = output channel
+      for (int st = 0; st < 4; ++st)
+        g = mfma32(ld_x8(sg + (32 * blk + gr) * CM + 8 * ((2 * st + h) ^ sg8)), xf[st], g);   // rows = k (perm16)
+#pragma unroll
+      for (int sp = 0; sp < 2; ++sp) {
+        opx8 og;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) og[t] = (op_t)((float)ov[blk % PWA_AHEAD][sp][t] * sigmoidf_fast(g[8 * sp + t]));
+        if (blk + PWA_AHEAD < PH) ov[blk % PWA_AHEAD][sp] = ld_x8(orow + (blk + PWA_AHEAD) * ostep + 16 * sp);
+        const int kc = 2 * (2 * blk + sp) + h;   // 16-byte chunk of the W_o row: k = 32 blk + 16 sp + 8 h
+#pragma unroll
+        for (int ob = 0; ob < 2; ++ob) {
+          const int R = 32 * ob + mr;
+          acc[ob] = mfma32(ld_x8(so + R * PHD + 8 * (kc ^ (R & 15))), og, acc[ob]);   // rows = output channel
+        }
       }
     }
-  }
-  if (s0 + mm >= S) return;
-  // lane (s, h): acc[ob][4 g + e] is channel 32 ob + 8 g + 4 h + e
-  const float* src = m_in + mrow;
-  float* dst = m_out + mrow;
-  f32x4 res[8];
+    if (s0 + mm < S) {
+      // lane (s, h): acc[ob][4 g + e] is channel 32 ob + 8 g + 4 h + e
+      const float* src = m_in + mrow;
+      float* dst = m_out + mrow;
+      f32x4 res[8];
 #pragma unroll
-  for (int q = 0; q < 8; ++q)
-    res[q] = accumulate ? *reinterpret_cast<const f32x4*>(src + oa_channel(q, h)) : f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int q = 0; q < 8; ++q)
+        res[q] = accumulate ? *reinterpret_cast<const f32x4*>(src + oa_channel(q, h)) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    f32x4 v;
+      for (int q = 0; q < 8; ++q) {
+        f32x4 v;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = acc[q >> 2][4 * (q & 3) + e] + res[q][e];
-    *reinterpret_cast<f32x4*>(dst + oa_channel(q, h)) = v;
+        for (int e = 0; e < 4; ++e) v[e] = acc[q >> 2][4 * (q & 3) + e] + res[q][e];
+        *reinterpret_cast<f32x4*>(dst + oa_channel(q, h)) = v;
+      }
+    }
   }
 }
 
@@ -460,8 +474,7 @@ extern "C" int pf_opm_fwd(const pf_opm_args* a) {
   op_t* Mt = Bt + rows * Sp;
   op_t* Z = Mt + (size_t)B * N * Sp;
   float* cnt = (float*)(Z + rows * N * CH);
-  const long waves = (long)B * N * (Sp / 32);
-  opm_proj_kernel<<<(unsigned)((waves + 3) / 4), 256, 0, st>>>(a->m, a->msa_mask, a->norm_w, a->norm_b,
+  opm_proj_kernel<<<(unsigned)((long)B * (N / 2) * (Sp / 64)), 256, 0, st>>>(a->m, a->msa_mask, a->norm_w, a->norm_b,
                                                               (const op_t*)a->w_a, (const op_t*)a->w_b, At, Bt, Mt,
                                                               B, S, Sp, N, a->eps);
   PF_CHECK_LAUNCH("opm_proj_kernel");
@@ -518,8 +531,8 @@ extern "C" int pf_pwa_fwd(const pf_pwa_args* a) {
   PF_CHECK_LAUNCH("pwa_proj_kernel");
   // rows (s, d) of v_t are the Nc dimension; S*32 is a multiple of 32
   if ((rc = pf_contract_rect(Wt, vt, O, 0, (int)bh, N, S * PD, N, 1.f, st))) return rc;
-  const long ow = (long)B * N * ((S + 31) / 32);
-  pwa_out_kernel<<<(unsigned)((ow + 7) / 8), 512, 0, st>>>(a->m, a->out, a->norm_m_w, a->norm_m_b,
+  const long ow = (long)B * (N / 8) * ((S + 31) / 32);
+  pwa_out_kernel<<<(unsigned)min(2l * cus, ow), 512, 0, st>>>(a->m, a->out, a->norm_m_w, a->norm_m_b,
                                                           (const op_t*)a->w_g, (const op_t*)a->w_o, O, B, S, N,
                                                           a->accumulate, a->eps);
   PF_CHECK_LAUNCH("pwa_out_kernel");
