@@ -480,13 +480,13 @@ def summarize_probe(N: int, kt_dir: str, pmc_dirs) -> None:
     w_fac = COPY_BYTES / (mean(copy["WRITE_SIZE"]) * 1024)
     copy_us = mean([d for d in dur["copy (torch.mul, calibration)"] if d > 20])
     P = N * N
-    alg = {"tm_proj_kernel": P * 128 * 4 + 2 * P * 128 * 2,
+    alg = {"tm_proj_direct_kernel": P * 128 * 4 + 2 * P * 128 * 2,
            "tm_contract_dma_kernel": 3 * P * 128 * 2,
-           "tm_out_kernel": P * 128 * 2 + 2 * P * 128 * 4,
+           "tm_out_direct_kernel": P * 128 * 2 + 2 * P * 128 * 4,
            "ta_proj_kernel": P * 128 * 4 + 3 * P * 128 * 2 + 4 * P * 4 + P * 2,
            "ta_attn_kernel": 3 * P * 128 * 2 + 4 * P * 4 + P * 2 + P * 128 * 2,
            "ta_out_kernel": P * 128 * 2 + 2 * P * 128 * 4,
-           "tr_pair_kernel": 2 * P * 128 * 4 + 16 * P * 4}
+           "tr_direct_kernel": 2 * P * 128 * 4 + 16 * P * 4}
     rows = []
     for k in sorted(cnt, key=lambda k: -sum(dur.get(k, [0]))):
         c, d = cnt[k], dur.get(k, [])
