@@ -128,6 +128,12 @@ def _pads_on_device(x: torch.Tensor, device: torch.device) -> bool:
             and x.stride(-1) == 1)
 
 
+def _shaped(t: torch.Tensor, shape: tuple) -> torch.Tensor:
+    """``t`` in the call's own ``shape``, broadcast to it where its sizes are 1 (a view), RuntimeError
+    where they do not fit: the kernels read a whole tensor of that shape from the pointer."""
+    return t if t.shape == shape else t.expand(shape)
+
+
 def padded(x: torch.Tensor, n_pad: int, device: torch.device, dims: tuple) -> torch.Tensor:
     """New contiguous fp32 tensor on ``device``: ``x`` with the dimensions in ``dims`` zero-padded to
     ``n_pad``.  ``dims`` is (1, 2) for [B,N,N,C], (1,) for [B,N,C], (1, 3) for [B,N,H,N,D] and for
@@ -640,7 +646,7 @@ def triangle_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bias: 
     n_pad = padded_len(N)
 
     def padq(t):
-        t = t.to(torch.float32)
+        t = _shaped(t.to(torch.float32), (B, N, H, N, D))
         return t.contiguous() if n_pad == N else padded(t, n_pad, dev, (1, 3))
 
     qp, kp, vp = padq(q), padq(k), padq(v)
