@@ -69,3 +69,48 @@ def test_triangle_attention_refuses_other_shapes(lib, N, size):
         with pytest.raises(RuntimeError):
             ops.triangle_attention(q, k, v, torch.zeros((2, 1, 4, N, N)))
     assert not lib.calls
+
+
+# ------------------------------------------------------------------------------ single track
+def _apb(B, N, k_in=None, z=None, mask=None):
+    g = torch.Generator().manual_seed(2)
+    w = {f"proj_{k}.weight": torch.randn((384, 384), generator=g) for k in "qkvgo"}
+    w.update({"proj_q.bias": torch.zeros(384), "proj_z.0.weight": torch.ones(128), "proj_z.0.bias": torch.zeros(128),
+              "proj_z.1.weight": torch.randn((16, 128), generator=g)})
+    s = torch.randn((B, N, 384), generator=g)
+    z = torch.randn((B, N, N, 128), generator=g) if z is None else z
+    return ops.attention_pair_bias(s, z, mask, s if k_in is None else k_in, w)
+
+
+def _apb_args_of(lib):
+    (name, args), = lib.calls
+    assert name == "pf_apb_fwd_unpadded"
+    return args[0]._obj, args[1]
+
+
+@pytest.mark.parametrize("N", [50, 64])
+@pytest.mark.parametrize("size", [(1, None, 384), (2, 1, 384), (2, None, 1)])
+def test_attention_pair_bias_broadcasts_k_in(lib, N, size):
+    k_in = torch.randn([N if n is None else n for n in size])
+    _apb(2, N, k_in)
+    a, _ = _apb_args_of(lib)
+    got = lib.tensors[a.k_in]
+    assert got.shape == (2, 64, 384)
+    assert torch.equal(got[:, :N], k_in.expand(2, N, 384)) and got[:, N:].abs().sum() == 0
+
+
+@pytest.mark.parametrize("N", [50, 64])
+@pytest.mark.parametrize("size", [(3, None, 384), (2, 40, 384), (2, 80, 384), (2, None, 383)])
+def test_attention_pair_bias_refuses_other_k_in(lib, N, size):
+    with pytest.raises(RuntimeError):
+        _apb(2, N, torch.zeros([N if n is None else n for n in size]))
+    assert not lib.calls
+
+
+@pytest.mark.parametrize("N", [50, 64])
+@pytest.mark.parametrize("size", [(1, None), (None,), (2, 1), (1, 2, None)])
+def test_attention_pair_bias_broadcasts_mask(lib, N, size):
+    mask = torch.ones([N if n is None else n for n in size])
+    _apb(2, N, mask=mask)
+    a, _ = _apb_args_of(lib)
+    assert torch.equal(lib.tensors[a.mask], torch.nn.functional.pad(torch.ones(2, N), (0, 64 - N)))

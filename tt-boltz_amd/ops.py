@@ -129,9 +129,14 @@ def _pads_on_device(x: torch.Tensor, device: torch.device) -> bool:
 
 
 def _shaped(t: torch.Tensor, shape: tuple) -> torch.Tensor:
-    """``t`` in the call's own ``shape``, broadcast to it where its sizes are 1 (a view), RuntimeError
-    where they do not fit: the kernels read a whole tensor of that shape from the pointer."""
-    return t if t.shape == shape else t.expand(shape)
+    """``t`` in the call's own ``shape``, broadcast to it as an assignment to a slice of that shape
+    would (a view), RuntimeError where it does not fit: the kernels read a whole tensor of that shape
+    from the pointer."""
+    if t.shape == shape:
+        return t
+    while t.dim() > len(shape) and t.shape[0] == 1:
+        t = t[0]
+    return t.expand(shape)
 
 
 def padded(x: torch.Tensor, n_pad: int, device: torch.device, dims: tuple) -> torch.Tensor:
@@ -688,20 +693,20 @@ def attention_pair_bias(s: torch.Tensor, z: torch.Tensor, mask: Optional[torch.T
     B, N, c_s = s.shape
     n_pad = padded_len(N)
 
-    def pad_tokens(t):   # [B, N, c] -> [B, n_pad, c] fp32; read-only, so no copy when N needs no padding
+    def pad_tokens(t):   # [B, N, c_s] -> [B, n_pad, c_s] fp32; read-only, so no copy when N needs no padding
+        t = _shaped(t, (B, N, c_s))
         if n_pad == N:
             return t.to(torch.float32).contiguous()
         return padded(t.to(torch.float32), n_pad, dev, (1,))
     sp = pad_tokens(s)
     kp = sp if k_in is s else pad_tokens(k_in)   # both are only read
     zp = z.to(torch.float32).contiguous()   # read unpadded
-    if mask is not None and n_pad == N:
-        mp = mask.to(device=dev, dtype=torch.float32).contiguous()
-    elif mask is not None and tuple(mask.shape) == (B, N):
-        mp = padded(mask.to(device=dev, dtype=torch.float32), n_pad, dev, (1,))
+    if mask is not None:
+        mask = _shaped(mask, (B, N)).to(device=dev, dtype=torch.float32)
+        mp = mask.contiguous() if n_pad == N else padded(mask, n_pad, dev, (1,))
     else:
         mp = torch.zeros((B, n_pad), dtype=torch.float32, device=dev)
-        mp[:, :N] = 1.0 if mask is None else mask.to(torch.float32)
+        mp[:, :N] = 1.0
     w = convert_weights(weights, dev, variant)
     out = torch.empty_like(sp)
     ws = workspace(apb_workspace_bytes(B, n_pad, c_s, num_heads, variant), dev)
