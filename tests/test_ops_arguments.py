@@ -114,3 +114,32 @@ def test_attention_pair_bias_broadcasts_mask(lib, N, size):
     _apb(2, N, mask=mask)
     a, _ = _apb_args_of(lib)
     assert torch.equal(lib.tensors[a.mask], torch.nn.functional.pad(torch.ones(2, N), (0, 64 - N)))
+
+
+# ------------------------------------------------------------------------------ padded copies
+PAIR_COPIES = {"pad_pair": lambda z, n: ops.pad_pair(z, n),
+               # (a CPU tensor takes another path there: the meta device stands for the GPU)
+               "to_device_padded": lambda z, n: ops.to_device_padded(z, n, z.device, True)}
+
+
+@pytest.mark.parametrize("copy", PAIR_COPIES)
+@pytest.mark.parametrize("size", [(1, 50, 40, 8), (1, 40, 50, 8), (1, 65, 65, 8), (1, 1, 50, 8)])
+def test_pair_copies_refuse_what_is_not_square(copy, size):
+    z = torch.ones(size, device="cpu" if copy == "pad_pair" else "meta")
+    with pytest.raises(RuntimeError):
+        PAIR_COPIES[copy](z, 64)
+
+
+def test_pad_pair_broadcasts_one_column():
+    z = torch.randn((2, 50, 1, 8))
+    got = ops.pad_pair(z, 64)
+    assert torch.equal(got[:, :50, :50], z.expand(2, 50, 50, 8)) and got.sum() == got[:, :50, :50].sum()
+    assert ops.to_device_padded(z.to("meta"), 64, torch.device("meta"), True).shape == (2, 64, 64, 8)
+
+
+@pytest.mark.parametrize("N", [50, 64])
+def test_triangle_multiplication_refuses_what_is_not_square(lib, N):
+    for size in ((1, N, N - 10, 128), (1, N, N + 1, 128)):
+        with pytest.raises(RuntimeError):
+            ops.triangle_multiplicative_update(torch.ones(size))
+    assert not lib.calls

@@ -172,7 +172,8 @@ def padded(x: torch.Tensor, n_pad: int, device: torch.device, dims: tuple) -> to
 
 def pad_pair(z: torch.Tensor, n_pad: int) -> torch.Tensor:
     """Zero-pad [B,N,N,C] to [B,n_pad,n_pad,C] (always returns a new contiguous fp32 tensor)."""
-    return padded(z, n_pad, z.device, (1, 2))
+    B, N, _, C = z.shape
+    return padded(_shaped(z, (B, N, N, C)), n_pad, z.device, (1, 2))
 
 
 #: row chunks of a host -> device pair copy: the host copy of one chunk into pinned memory
@@ -187,7 +188,9 @@ def to_device_padded(x: torch.Tensor, n_pad: int, device: torch.device, pair: bo
     chunk overlaps the transfer of the previous one; a device tensor is padded in place."""
     B, N = x.shape[0], x.shape[1]
     if x.device.type != "cpu":
-        return padded(x, n_pad, device, (1, 2) if pair else (1,))
+        if pair:
+            return padded(_shaped(x, (B, N, N, x.shape[-1])), n_pad, device, (1, 2))
+        return padded(_shaped(x, (B, N, x.shape[-1])), n_pad, device, (1,))
     shape = (B, n_pad, n_pad, x.shape[-1]) if pair else (B, n_pad, x.shape[-1])
     out = torch.zeros(shape, dtype=torch.float32, device=device)
     dst = out[:, :N, :N] if pair else out[:, :N]
@@ -614,7 +617,8 @@ def triangle_multiplicative_update(x: torch.Tensor, direction: str = "outgoing",
     dev = _require_gpu(x)
     B, N, _, C = x.shape
     n_pad = padded_len(N)
-    zp = pad_pair(x.to(torch.float32), n_pad) if n_pad != N else x.to(torch.float32).contiguous()
+    x = _shaped(x, (B, N, N, C)).to(torch.float32)
+    zp = pad_pair(x, n_pad) if n_pad != N else x.contiguous()
     m3 = None if mask is None else (mask.unsqueeze(0) if mask.dim() == 2 else mask)
     if m3 is not None and n_pad == N and tuple(m3.shape) == (B, N, N):
         mp = m3.to(device=dev, dtype=torch.float32).contiguous()   # read-only: no padded copy needed
