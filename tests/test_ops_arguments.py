@@ -143,3 +143,39 @@ def test_triangle_multiplication_refuses_what_is_not_square(lib, N):
         with pytest.raises(RuntimeError):
             ops.triangle_multiplicative_update(torch.ones(size))
     assert not lib.calls
+
+
+@pytest.mark.parametrize("N", [50, 64])
+def test_attention_pair_bias_reads_z_of_its_own_length(lib, N):
+    z = torch.randn((2, N, N, 128))
+    _apb(2, N, z=z)
+    a, z_n = _apb_args_of(lib)
+    assert z_n == N and lib.tensors[a.z] is z   # unpadded, where it is
+
+
+@pytest.mark.parametrize("N", [50, 64])
+@pytest.mark.parametrize("tokens", [40, 1, 60])
+def test_attention_pair_bias_pads_z_of_other_tokens(lib, N, tokens):
+    """As the padded copy always was: zeros past z's own tokens, in the s grid's row length."""
+    z = torch.randn((2, tokens, tokens, 128))
+    _apb(2, N, z=z)
+    a, z_n = _apb_args_of(lib)
+    pad = 64 - tokens
+    assert z_n == 64
+    assert torch.equal(lib.tensors[a.z], torch.nn.functional.pad(z, (0, 0, 0, pad, 0, pad)))
+
+
+@pytest.mark.parametrize("N", [50, 64])
+def test_attention_pair_bias_broadcasts_z(lib, N):
+    z = torch.randn((1, N, N, 128))
+    _apb(2, N, z=z)
+    a, z_n = _apb_args_of(lib)
+    assert z_n == N and torch.equal(lib.tensors[a.z], z.expand(2, N, N, 128))
+
+
+@pytest.mark.parametrize("N", [50, 64])
+@pytest.mark.parametrize("size", [(2, 65, 65, 128), (2, 50, 40, 128), (3, 50, 50, 128), (2, 64, 64, 64)])
+def test_attention_pair_bias_refuses_other_z(lib, N, size):
+    with pytest.raises(RuntimeError):
+        _apb(2, N, z=torch.zeros(size))
+    assert not lib.calls

@@ -704,7 +704,9 @@ def attention_pair_bias(s: torch.Tensor, z: torch.Tensor, mask: Optional[torch.T
         return padded(t.to(torch.float32), n_pad, dev, (1,))
     sp = pad_tokens(s)
     kp = sp if k_in is s else pad_tokens(k_in)   # both are only read
-    zp = z.to(torch.float32).contiguous()   # read unpadded
+    z = _shaped(z, (B,) + tuple(z.shape[1:3]) + (C_Z,)).to(torch.float32)
+    # read unpadded where it has the tokens of s, else through a padded copy
+    zp, z_n = (z.contiguous(), N) if tuple(z.shape[1:3]) == (N, N) else (pad_pair(z, n_pad), n_pad)
     if mask is not None:
         mask = _shaped(mask, (B, N)).to(device=dev, dtype=torch.float32)
         mp = mask.contiguous() if n_pad == N else padded(mask, n_pad, dev, (1,))
@@ -715,7 +717,7 @@ def attention_pair_bias(s: torch.Tensor, z: torch.Tensor, mask: Optional[torch.T
     out = torch.empty_like(sp)
     ws = workspace(apb_workspace_bytes(B, n_pad, c_s, num_heads, variant), dev)
     a = _apb_args(sp, kp, zp, mp, out, w, num_heads, ws, False, eps, N)
-    _lib.check(_lib.load(variant).pf_apb_fwd_unpadded(ctypes.byref(a), N, int(fast)), "pf_apb_fwd_unpadded", variant)
+    _lib.check(_lib.load(variant).pf_apb_fwd_unpadded(ctypes.byref(a), z_n, int(fast)), "pf_apb_fwd_unpadded", variant)
     return out[:, :N]
 
 
