@@ -179,3 +179,24 @@ def test_attention_pair_bias_refuses_other_z(lib, N, size):
     with pytest.raises(RuntimeError):
         _apb(2, N, z=torch.zeros(size))
     assert not lib.calls
+
+
+# ------------------------------------------------------------------------------ MSA inputs
+def _msa_inputs(emb, B=2, S=3, N=50):
+    feats = {k: torch.ones((B, S, N)) for k in ("has_deletion", "deletion_value", "msa_paired", "msa_mask")}
+    feats["msa"] = torch.zeros((B, S, N), dtype=torch.int64)
+    return msa.device_inputs(emb, feats, 64, torch.device("cpu"))
+
+
+@pytest.mark.parametrize("size", [(2, 50, 6), (1, 50, 6), (50, 6), (2, 1, 6), (1, 2, 50, 6)])
+def test_msa_inputs_broadcast_emb(size):
+    emb = torch.randn(size)
+    got = _msa_inputs(emb)["emb"]
+    want = emb if emb.dim() < 4 else emb[0]
+    assert torch.equal(got, torch.nn.functional.pad(want.expand(2, 50, 6), (0, 0, 0, 14)))
+
+
+@pytest.mark.parametrize("size", [(2, 40, 6), (2, 60, 6), (3, 50, 6)])
+def test_msa_inputs_refuse_other_emb(size):
+    with pytest.raises(RuntimeError):
+        _msa_inputs(torch.ones(size))

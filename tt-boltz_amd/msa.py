@@ -142,7 +142,9 @@ def device_inputs(emb: torch.Tensor, feats: Mapping[str, torch.Tensor], n_pad: i
         t[:, :, :N] = x
         return t
 
-    return {"emb": ops.padded(emb.to(device, torch.float32), n_pad, device, (1,)), "msa": per_row("msa", torch.int32), "has_deletion": per_row("has_deletion", torch.float32),
+    emb = ops.shaped(emb, (B, N, emb.shape[-1])).to(device, torch.float32)
+    return {"emb": ops.padded(emb, n_pad, device, (1,)), "msa": per_row("msa", torch.int32),
+            "has_deletion": per_row("has_deletion", torch.float32),
             "deletion_value": per_row("deletion_value", torch.float32),
             "msa_paired": per_row("msa_paired", torch.float32), "msa_mask": per_row("msa_mask", torch.float32)}
 

@@ -128,7 +128,7 @@ def _pads_on_device(x: torch.Tensor, device: torch.device) -> bool:
             and x.stride(-1) == 1)
 
 
-def _shaped(t: torch.Tensor, shape: tuple) -> torch.Tensor:
+def shaped(t: torch.Tensor, shape: tuple) -> torch.Tensor:
     """``t`` in the call's own ``shape``, broadcast to it as an assignment to a slice of that shape
     would (a view), RuntimeError where it does not fit: the kernels read a whole tensor of that shape
     from the pointer."""
@@ -173,7 +173,7 @@ def padded(x: torch.Tensor, n_pad: int, device: torch.device, dims: tuple) -> to
 def pad_pair(z: torch.Tensor, n_pad: int) -> torch.Tensor:
     """Zero-pad [B,N,N,C] to [B,n_pad,n_pad,C] (always returns a new contiguous fp32 tensor)."""
     B, N, _, C = z.shape
-    return padded(_shaped(z, (B, N, N, C)), n_pad, z.device, (1, 2))
+    return padded(shaped(z, (B, N, N, C)), n_pad, z.device, (1, 2))
 
 
 #: row chunks of a host -> device pair copy: the host copy of one chunk into pinned memory
@@ -189,8 +189,8 @@ def to_device_padded(x: torch.Tensor, n_pad: int, device: torch.device, pair: bo
     B, N = x.shape[0], x.shape[1]
     if x.device.type != "cpu":
         if pair:
-            return padded(_shaped(x, (B, N, N, x.shape[-1])), n_pad, device, (1, 2))
-        return padded(_shaped(x, (B, N, x.shape[-1])), n_pad, device, (1,))
+            return padded(shaped(x, (B, N, N, x.shape[-1])), n_pad, device, (1, 2))
+        return padded(shaped(x, (B, N, x.shape[-1])), n_pad, device, (1,))
     shape = (B, n_pad, n_pad, x.shape[-1]) if pair else (B, n_pad, x.shape[-1])
     out = torch.zeros(shape, dtype=torch.float32, device=device)
     dst = out[:, :N, :N] if pair else out[:, :N]
@@ -617,7 +617,7 @@ def triangle_multiplicative_update(x: torch.Tensor, direction: str = "outgoing",
     dev = _require_gpu(x)
     B, N, _, C = x.shape
     n_pad = padded_len(N)
-    x = _shaped(x, (B, N, N, C)).to(torch.float32)
+    x = shaped(x, (B, N, N, C)).to(torch.float32)
     zp = pad_pair(x, n_pad) if n_pad != N else x.contiguous()
     m3 = None if mask is None else (mask.unsqueeze(0) if mask.dim() == 2 else mask)
     if m3 is not None and n_pad == N and tuple(m3.shape) == (B, N, N):
@@ -655,7 +655,7 @@ def triangle_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bias: 
     n_pad = padded_len(N)
 
     def padq(t):
-        t = _shaped(t.to(torch.float32), (B, N, H, N, D))
+        t = shaped(t.to(torch.float32), (B, N, H, N, D))
         return t.contiguous() if n_pad == N else padded(t, n_pad, dev, (1, 3))
 
     qp, kp, vp = padq(q), padq(k), padq(v)
@@ -698,17 +698,17 @@ def attention_pair_bias(s: torch.Tensor, z: torch.Tensor, mask: Optional[torch.T
     n_pad = padded_len(N)
 
     def pad_tokens(t):   # [B, N, c_s] -> [B, n_pad, c_s] fp32; read-only, so no copy when N needs no padding
-        t = _shaped(t, (B, N, c_s))
+        t = shaped(t, (B, N, c_s))
         if n_pad == N:
             return t.to(torch.float32).contiguous()
         return padded(t.to(torch.float32), n_pad, dev, (1,))
     sp = pad_tokens(s)
     kp = sp if k_in is s else pad_tokens(k_in)   # both are only read
-    z = _shaped(z, (B,) + tuple(z.shape[1:3]) + (C_Z,)).to(torch.float32)
+    z = shaped(z, (B,) + tuple(z.shape[1:3]) + (C_Z,)).to(torch.float32)
     # read unpadded where it has the tokens of s, else through a padded copy
     zp, z_n = (z.contiguous(), N) if tuple(z.shape[1:3]) == (N, N) else (pad_pair(z, n_pad), n_pad)
     if mask is not None:
-        mask = _shaped(mask, (B, N)).to(device=dev, dtype=torch.float32)
+        mask = shaped(mask, (B, N)).to(device=dev, dtype=torch.float32)
         mp = mask.contiguous() if n_pad == N else padded(mask, n_pad, dev, (1,))
     else:
         mp = torch.zeros((B, n_pad), dtype=torch.float32, device=dev)
