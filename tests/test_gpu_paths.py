@@ -166,6 +166,56 @@ def test_attention_pair_bias_unpadded(gpu, B, N, masked, fast):
                                                                   else mask.cpu(), s.cpu(), w))
 
 
+# ------------------------------------------------------------------------------ alignment
+def _odd(t):
+    """A contiguous copy of ``t`` that begins 4 bytes past a 16-byte boundary."""
+    out = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    return out.copy_(t)
+
+
+@pytest.mark.parametrize("op", ["apb", "trimul", "triatt", "token_bias", "cond_proj", "pwa"])
+@pytest.mark.parametrize("N", [50, 64])
+def test_caller_arrays_at_odd_addresses(gpu, op, N):
+    """A z read where it is and LayerNorm vectors off 16-byte boundaries: identical bits."""
+    g = torch.Generator().manual_seed(N)
+    z = torch.randn((1, N, N, 128), generator=g).to(gpu)
+    sub = {"apb": "attention", "trimul": "tri_mul_out", "triatt": "tri_att_start"}
+    if op in sub:
+        w = ops.convert_weights(_sub_w(31, sub[op]), gpu, strip="mha.")
+    elif op == "pwa":
+        w = ops.convert_weights({k: v.to(gpu) for k, v in _msa_sub(5, "pair_weighted_averaging").items()}, gpu)
+    else:
+        c = 256 if op == "cond_proj" else 4 * 128
+        w = {"w": 1 + 0.1 * torch.randn(c, generator=g).to(gpu), "b": 0.1 * torch.randn(c, generator=g).to(gpu)}
+        rows = (0.1 * torch.randn((128, 256 if op == "cond_proj" else 128), generator=g)).half().to(gpu)
+    zp = ops.pad_pair(z, 64)
+
+    def run(w, z):
+        if op == "apb":
+            s = torch.randn((1, N, 384), generator=torch.Generator().manual_seed(3)).to(gpu)
+            return ops.attention_pair_bias(s, z, None, s, w)
+        if op == "trimul":
+            out, ws = torch.empty_like(zp), ops.workspace(ops.trimul_workspace_bytes(1, 64), gpu)
+            ops.launch_trimul(zp, out, None, w, 0, ws, False)
+        elif op == "triatt":
+            out, ws = torch.empty_like(zp), ops.workspace(ops.triatt_workspace_bytes(1, 64), gpu)
+            ops.launch_triatt(zp, out, None, w, False, ws, False, n_valid=N)
+        elif op == "token_bias":
+            out = torch.empty((N * N, 128), device=gpu)
+            ops.launch_token_pair_bias(z, w["w"], w["b"], rows, out, 4, 32, 0, 1.0)
+        elif op == "cond_proj":
+            out = torch.empty((N * N, 128), device=gpu)
+            ops.launch_pair_cond_proj(z, 2 * z, w["w"], w["b"], rows, out)
+        else:
+            m = torch.randn((1, 5, 64, 64), generator=torch.Generator().manual_seed(4)).to(gpu)
+            out, ws = torch.empty_like(m), ops.workspace(ops.pwa_workspace_bytes(1, 5, 64), gpu)
+            ops.launch_pwa(m, zp, None, out, w, ws, accumulate=False)
+        return out
+    want = run(w, z)
+    got = run({k: _odd(v) if v.dim() == 1 and v.dtype == torch.float32 else v for k, v in w.items()}, _odd(z))
+    assert torch.equal(got, want)
+
+
 # ------------------------------------------------------------------------------ pair transition
 @pytest.mark.parametrize("rows", [1, 31, 33, 64, 65, 16384, 16385])
 @pytest.mark.parametrize("hidden", [128, 512])

@@ -31,7 +31,7 @@ constexpr int TB_MAX_OUT = 512, TB_WAVES = 12;
 PF_DEV f32x4 group_row4(const float* t, int g, long rows, int r, int c) {
   const char* base = reinterpret_cast<const char*>(t + (long)DP_ROWS * g * C);
   const uint32_t last = (uint32_t)min((long)DP_ROWS, rows - (long)DP_ROWS * g) - 1;
-  return *reinterpret_cast<const f32x4*>(base + 4u * (min((uint32_t)r, last) * C + c));
+  return *reinterpret_cast<const f32x4_any*>(base + 4u * (min((uint32_t)r, last) * C + c));
 }
 
 // -------------------------------------------------------------------------------------
@@ -151,7 +151,6 @@ __global__ __launch_bounds__(64 * CP_WAVES, 1) void cond_proj_kernel(
 // 128 38.7 -> 11.8, 450 130 -> 89, 512 142 -> 113 (layout 1: 450 156 -> 137, 512 138 -> 115).
 // -------------------------------------------------------------------------------------
 constexpr int TB_SP = 36;   // stage pitch (floats)
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // the caller's out: any alignment
 struct TbLds {
   static constexpr size_t ST = (size_t)2 * DP_ROWS * (C + 8) * sizeof(op_t);   // normalized pairs, two buffers
   static constexpr size_t OFF = ST + (size_t)TB_WAVES * DP_ROWS * TB_SP * sizeof(float);

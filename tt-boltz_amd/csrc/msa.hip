@@ -233,7 +233,8 @@ __global__ __launch_bounds__(64 * PH, 4) void pwa_proj_kernel(
   opx8 w[4];
 #pragma unroll
   for (int st = 0; st < 4; ++st) w[st] = ld_x8(wm + (PD * wid + mm) * CM + 16 * st + 8 * h);
-  const f32x4 gm = *reinterpret_cast<const f32x4*>(lnw + 4 * q4), bt = *reinterpret_cast<const f32x4*>(lnb + 4 * q4);
+  const f32x4 gm = *reinterpret_cast<const f32x4_any*>(lnw + 4 * q4),
+              bt = *reinterpret_cast<const f32x4_any*>(lnb + 4 * q4);
   const int nj = N / 64;
   int buf = 0;
   for (long gi = blockIdx.x; gi < ngroups; gi += gridDim.x, buf ^= 1) {

@@ -36,6 +36,9 @@ typedef op_t opx8 __attribute__((ext_vector_type(8)));
 typedef op_t opx4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// 16 bytes of a caller's fp32 array, which need not begin on a 16-byte boundary (the same one
+// global load or store; LDS keeps to f32x4)
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 #define PF_DEV __device__ __forceinline__
 // Device lambdas: always inlined (an outlined lambda moves captured state through memory).

@@ -37,7 +37,7 @@ struct DirectLn {
     const int q = lane & 15;
 #pragma unroll
     for (int v = 0; v < NV; ++v)
-      gm[v] = gamma ? *reinterpret_cast<const f32x4*>(gamma + 64 * v + 4 * q) : f32x4{1.f, 1.f, 1.f, 1.f};
+      gm[v] = gamma ? *reinterpret_cast<const f32x4_any*>(gamma + 64 * v + 4 * q) : f32x4{1.f, 1.f, 1.f, 1.f};
   }
   PF_DEV void store(op_t* dst, float eps, int wid, int lane) const {
     const int g = lane >> 4, q = lane & 15;
@@ -85,15 +85,16 @@ struct DirectW {
 #pragma unroll
     for (int s = 0; s < CC / 16; ++s) v[s] = ld_x8(buf + (lane & 31) * (CC + 8) + 16 * s + 8 * (lane >> 5));
   }
-  // W diag(gamma), rounded to op_t again
+  // W diag(gamma), rounded to op_t again.  V: f32x4 for a gamma in LDS.
+  template <class V = f32x4_any>
   PF_DEV void fold(const float* gamma, int h) {
     // (opaque: the 64 float conversions that an earlier W . beta took are not kept for this)
 #pragma unroll
     for (int s = 0; s < CC / 16; ++s) asm volatile("" : "+v"(v[s]));
 #pragma unroll
     for (int s = 0; s < CC / 16; ++s) {
-      const f32x4 g0 = *reinterpret_cast<const f32x4*>(gamma + 16 * s + 8 * h);
-      const f32x4 g1 = *reinterpret_cast<const f32x4*>(gamma + 16 * s + 8 * h + 4);
+      const f32x4 g0 = *reinterpret_cast<const V*>(gamma + 16 * s + 8 * h);
+      const f32x4 g1 = *reinterpret_cast<const V*>(gamma + 16 * s + 8 * h + 4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         v[s][e] = (op_t)((float)v[s][e] * g0[e]);
@@ -110,12 +111,13 @@ struct DirectW {
 template <int CC>
 struct DirectW8 {
   typedef int i32x2_t __attribute__((ext_vector_type(2)));
+  typedef int i32x2_any __attribute__((ext_vector_type(2), aligned(4)));   // the caller's bytes, in dwords
   i32x2_t w[CC / 16];
   uint32_t e[CC / 32];
   PF_DEV void load(const uint8_t* __restrict__ q, const uint8_t* __restrict__ sc, int lane) {
     const int m = lane & 31, h = lane >> 5;
 #pragma unroll
-    for (int s = 0; s < CC / 16; ++s) w[s] = *reinterpret_cast<const i32x2_t*>(q + m * CC + 16 * s + 8 * h);
+    for (int s = 0; s < CC / 16; ++s) w[s] = *reinterpret_cast<const i32x2_any*>(q + m * CC + 16 * s + 8 * h);
 #pragma unroll
     for (int k = 0; k < CC / 32; ++k) e[k] = sc[m * (CC / 32) + k];
   }
@@ -147,16 +149,16 @@ struct DirectTile {
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
       const float* p = z + row_of(4 * it + g) * 128 + 4 * q;
-      x[it][0] = *reinterpret_cast<const f32x4*>(p);
-      x[it][1] = *reinterpret_cast<const f32x4*>(p + 64);
+      x[it][0] = *reinterpret_cast<const f32x4_any*>(p);
+      x[it][1] = *reinterpret_cast<const f32x4_any*>(p + 64);
     }
   }
   PF_DEV void affine(const float* __restrict__ gamma, const float* __restrict__ beta, int lane) {   // null: none
     const int q = lane & 15;
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
-      gm[v] = gamma ? *reinterpret_cast<const f32x4*>(gamma + 64 * v + 4 * q) : f32x4{1.f, 1.f, 1.f, 1.f};
-      bt[v] = beta ? *reinterpret_cast<const f32x4*>(beta + 64 * v + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+      gm[v] = gamma ? *reinterpret_cast<const f32x4_any*>(gamma + 64 * v + 4 * q) : f32x4{1.f, 1.f, 1.f, 1.f};
+      bt[v] = beta ? *reinterpret_cast<const f32x4_any*>(beta + 64 * v + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
   }
   PF_DEV void normalize(op_t* buf, float eps, int lane) const {
@@ -204,14 +206,15 @@ PF_DEV void direct_gmu(const float* __restrict__ stats, const float* __restrict_
   if (threadIdx.x < PS_C) gm[threadIdx.x] *= g;   // written by the same thread
 }
 
-// W row . beta in fp32 from the row's fragments (both lane halves get the sum).
-template <int KS>
+// W row . beta in fp32 from the row's fragments (both lane halves get the sum).  V: f32x4 for a
+// beta in LDS.
+template <int KS, class V = f32x4_any>
 PF_DEV float direct_wbeta(const opx8 (&w)[KS], const float* beta, int h) {
   float acc = 0.f;
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
-    const f32x4 b0 = *reinterpret_cast<const f32x4*>(beta + 16 * s + 8 * h);
-    const f32x4 b1 = *reinterpret_cast<const f32x4*>(beta + 16 * s + 8 * h + 4);
+    const f32x4 b0 = *reinterpret_cast<const V*>(beta + 16 * s + 8 * h);
+    const f32x4 b1 = *reinterpret_cast<const V*>(beta + 16 * s + 8 * h + 4);
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc += (float)w[s][e] * b0[e] + (float)w[s][4 + e] * b1[e];
     asm volatile("" : "+v"(acc));   // not all of beta in registers at once

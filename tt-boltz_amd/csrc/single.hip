@@ -86,7 +86,6 @@ __global__ __launch_bounds__(64 * ZB_WAVES, 1) void apb_zbias_kernel(
 // fragments are gathered straight from the fp32 rows: the 32 lanes of a half read 32
 // consecutive floats of one key row.
 constexpr int APB_SPLIT = 8;
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // the caller's mask: any alignment
 // d = d0 .. d0 + 7 of a head's row of DH floats (16-byte aligned), times sc; zero past DH
 template <int DH>
 PF_DEV opx8 apb_frag(const float* __restrict__ row, int d0, float sc) {

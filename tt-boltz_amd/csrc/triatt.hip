@@ -175,8 +175,8 @@ __global__ __launch_bounds__(64 * TAP_WAVES, 1) void ta_proj_kernel(
   // the set-up spilled)
   if constexpr (LO != DL_NONE) wl.load(mf.lo[kind] + r0, lane);
   if (wid < TAP_LN) ln.store(sx, eps, wid, lane);
-  if (!exact) c0 = direct_wbeta<KS>(w.v, sgb + CC, h);
-  w.fold(sgb, h);
+  if (!exact) c0 = direct_wbeta<KS, f32x4>(w.v, sgb + CC, h);
+  w.template fold<f32x4>(sgb, h);
   if constexpr (LO != DL_NONE) wl.turn(stg, lane);
   auto bias_sum = [&](float v) PF_INLINE -> float {   // over the CC / 8 lanes of a bias row
 #pragma unroll
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(64 * TAP_WAVES, 1) void ta_proj_kernel(
   }
   if constexpr (LO == DL_MEAN) {
     __syncthreads();
-    c0 += direct_wbeta<KS>(wl.v, smu, h);
+    c0 += direct_wbeta<KS, f32x4>(wl.v, smu, h);
     if (wid == 0) {
       float d = 0.f;
 #pragma unroll

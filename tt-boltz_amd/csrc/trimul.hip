@@ -265,8 +265,8 @@ __global__ __launch_bounds__(2 * 2 * CC, 1) void tm_proj_direct_kernel(
   if constexpr (LO == DL_MEAN) {
     __syncthreads();
     const float* gm = reinterpret_cast<const float*>(sx[1]);
-    cp += direct_wbeta<KS>(wpl.v, gm, h);
-    cg += direct_wbeta<KS>(wgl.v, gm, h);
+    cp += direct_wbeta<KS, f32x4>(wpl.v, gm, h);
+    cg += direct_wbeta<KS, f32x4>(wgl.v, gm, h);
   }
   if (!offb) {
     cp = direct_wbeta<KS>(wp.v, lnb, h);
@@ -796,7 +796,7 @@ __global__ __launch_bounds__(2 * 2 * CC, 1) void tm_out_direct_kernel(
       float* gm = reinterpret_cast<float*>(sxo);   // free until the tile loop's first barrier
       direct_gmu<NT>(stats, lni_w, gm, gm + PS_C);
       __syncthreads();
-      cg += direct_wbeta<KS>(wgl.v, gm, h);
+      cg += direct_wbeta<KS, f32x4>(wgl.v, gm, h);
     }
     if (tile == 0 && h == 0) {
       soff[row] = cp;
