@@ -39,6 +39,28 @@ def test_attention_reference_and_mask_tiles(gpu, shift, first_masked):
     check(f"attention shift={shift} first_masked={first_masked}", got, want)
 
 
+@pytest.mark.parametrize("level", [0.0, -3.0, -6.0, -9.5, -12.0])
+@pytest.mark.parametrize("depth", [8.0, 12.2, 15.2])
+@pytest.mark.parametrize("n_first", [32, 16, 1])
+def test_attention_small_weights(gpu, level, depth, n_first):
+    """Keys ``depth`` log2 units below a row's largest logits keep their share wherever the logits as a
+    whole lie.  ``n_first`` of the first 32 keys have ``level``, all others ``depth`` less; v marks
+    the others, so the output is their share alone.  A weight is rounded to fp16 with the largest at
+    1 or above: half a spacing of subnormals, 2^-25, beside 2^-depth, and 2^-11 each for the sum and
+    the output."""
+    N, H, D, ln2 = 512, 4, 32, 0.6931471805599453
+    q = torch.zeros((1, N, H, N, D), device=gpu)
+    bias = torch.full((1, 1, H, N, N), (level - depth) * ln2, device=gpu)
+    bias[..., :n_first] = level * ln2
+    v = torch.ones_like(q)
+    v[:, :, :, :n_first] = 0.0
+    got = ops.triangle_attention(q, q, v, bias).double()
+    small = (N - n_first) * 2.0 ** -depth
+    want = small / (small + n_first)
+    bar = 2.0 ** (depth - 25) + 2.0 ** -10
+    assert ((got - want).abs().max() / want).item() < bar
+
+
 # ------------------------------------------------------------------------------ trimul
 @pytest.mark.parametrize("B,N", [(1, 64), (1, 192), (1, 256), (1, 320), (2, 64), (2, 320)])
 @pytest.mark.parametrize("incoming", [False, True])

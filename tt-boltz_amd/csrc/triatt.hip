@@ -13,7 +13,7 @@
 //              Q, K    op_t [B][N(row i)][H][N(j)][D]
 //              Vt      op_t [B][N(row i)][H][D][N(k)], keys stored at perm16(k) (bits 2
 //                      and 3 swapped) so a P.V operand fragment is one 16-byte run
-//              bias32  fp32 [B][H][N(j)][N(k)]   (shared by all rows i)
+//              bias32  fp32 [B][H][N(j)][N(k)]   (shared by all rows i; x log2(e) + REF_SHIFT)
 //              mask16  op_t [B][N(i)][N(k)]      0, or -inf for masked / padding keys
 //   ta_attn  flash attention (see the kernel's comment): 16-wave workgroups of 4 frame rows
 //            x 128 queries, LDS-DMA ring, bias / mask / reference max folded into MFMAs,
@@ -33,6 +33,10 @@ namespace {
 constexpr int C = 128, H = 4, D = 32, LDSW = 136;
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float RESCALE_SLACK = 8.f;   // log2 units: P values stay <= 2^8 between rescales
+// Log2 units that every stored bias is raised by.  The softmax does not see it, but rows of logits
+// about 0 then pass the first tile's test for 0 as their reference (LSTEP_MIN; mean P of a lane's keys
+// 2^-4 to 2^6 without it) and their P still reach 1.
+constexpr float REF_SHIFT = 4.f;
 
 typedef op_t opx2 __attribute__((ext_vector_type(2)));
 
@@ -328,7 +332,7 @@ __global__ __launch_bounds__(64 * TAP_WAVES, 1) void ta_proj_kernel(
 #pragma unroll
           for (int r = 0; r < H; ++r)
             bias32[(((long)pt.b * H + r) * N + pt.r) * N + pt.c0 + 32 * hd + m] =
-                (acc[r] + soff[3 * C + r]) * LOG2E;
+                fmaf(acc[r] + soff[3 * C + r], LOG2E, REF_SHIFT);
         }
       }
     }
@@ -377,10 +381,10 @@ constexpr int TS_V = 98304, TV_STAGE = 16384;
 constexpr int TS_MASK = 131072, TM_STAGE = 1024;
 constexpr size_t TA_LDS = (size_t)TS_MASK + 2 * TM_STAGE;
 constexpr float LSTEP_MAX = 16384.f;   // per-lane row sum of one tile that forces a rescale
-// A lane's row sum (16 keys) of a head's first tile from which on 0 serves as the reference: the
-// larger P are then at least 2^-10, far inside op_t's normal range, and what the P below it lose
-// (2^-25 each in fp16) is below the rounding of the larger ones.
-constexpr float LSTEP_MIN = 1.f / 64.f;
+// A lane's row sum (16 keys) of a head's first tile from which on 0 serves as the reference: one of
+// its P is then at least 1, what the first tile's maximum as the reference would give, so the smaller
+// P keep as many bits in op_t.
+constexpr float LSTEP_MIN = 16.f;
 
 // 16-byte chunk swizzles: rows of 8 chunks (V^T) and of 4 chunks (K).  A fragment read takes
 // one chunk from each of 32 consecutive rows; any 16 consecutive rows land in 16 distinct
@@ -939,7 +943,7 @@ __global__ void ta_prep_bias_kernel(const float* __restrict__ bias, const float*
                                     float* __restrict__ bias32, op_t* __restrict__ mask16,
                                     long nbias, long nmask, int N, int n_valid) {
   for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < nbias; e += (long)gridDim.x * blockDim.x) {
-    bias32[e] = bias[e] * LOG2E;
+    bias32[e] = fmaf(bias[e], LOG2E, REF_SHIFT);
     if (e < nmask) mask16[e] = mask_term((int)(e % N) >= n_valid, mask ? mask[e] : 1.f);
   }
 }
