@@ -163,6 +163,22 @@ def test_padded(gpu, N, n_pad, form, shape, dims):
     assert got.is_contiguous() and got.dtype == torch.float32 and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("copy", ["pad_pair", "to_device_padded"])
+def test_padded_copies_under_torch_transforms(gpu, copy):
+    """A forward-mode tangent is padded along, and traces replay the padding on another input."""
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    fn = (lambda t: ops.pad_pair(t, 64)) if copy == "pad_pair" else \
+        (lambda t: ops.to_device_padded(t, 64, t.device, True))
+    z, other = torch.randn((2, 1, 45, 45, 8), generator=torch.Generator().manual_seed(1)).to(gpu)
+    want = torch.nn.functional.pad(other, (0, 0, 0, 19, 0, 19))
+    with forward_ad.dual_level():
+        out = forward_ad.unpack_dual(fn(forward_ad.make_dual(z, other)))
+        assert torch.equal(out.tangent, want)
+    assert torch.equal(torch.jit.trace(fn, z, check_trace=False)(other), want)
+    assert torch.equal(make_fx(fn)(z)(other), want)
+
+
 # ------------------------------------------------------------------------------ single track
 @pytest.mark.parametrize("B,N", [(1, 33), (1, 64), (2, 100), (1, 413)])
 @pytest.mark.parametrize("masked", [False, True])

@@ -22,6 +22,7 @@ import weakref
 from typing import Mapping, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -121,6 +122,10 @@ def padded_len(n: int, pad: int = PAD) -> int:
 
 def _pads_on_device(x: torch.Tensor, device: torch.device) -> bool:
     """Whether ``pf_pad_fwd`` can read ``x`` in place of a fill and a copy on ``device``."""
+    # what watches torch's own operations has to see the fill and the copy: torch.jit.trace, dispatch
+    # modes (make_fx) and forward-mode tangents
+    if torch._C._is_tracing() or torch._C._len_torch_dispatch_stack() or forward_ad._current_level >= 0:
+        return False
     return (x.dtype == torch.float32 and x.device == device and x.is_cuda
             and type(x) in (torch.Tensor, torch.nn.Parameter)
             and device.index == torch._C._cuda_getDevice()
