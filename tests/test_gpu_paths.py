@@ -39,7 +39,7 @@ def test_attention_reference_and_mask_tiles(gpu, shift, first_masked):
     check(f"attention shift={shift} first_masked={first_masked}", got, want)
 
 
-@pytest.mark.parametrize("level", [0.0, -3.0, -6.0, -9.5, -12.0])
+@pytest.mark.parametrize("level", [11.8, 7.8, 0.0, -3.0, -6.0, -9.5, -12.0])
 @pytest.mark.parametrize("depth", [8.0, 12.2, 15.2])
 @pytest.mark.parametrize("n_first", [32, 16, 1])
 def test_attention_small_weights(gpu, level, depth, n_first):

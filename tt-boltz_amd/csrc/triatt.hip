@@ -32,10 +32,12 @@ namespace {
 // projection kernels) is 128 in the trunk and 64 in the template stack.
 constexpr int C = 128, H = 4, D = 32, LDSW = 136;
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr float RESCALE_SLACK = 8.f;   // log2 units: P values stay <= 2^8 between rescales
+constexpr float RESCALE_SLACK = 8.f;   // log2 units: a rescale leaves queries whose P stay <= 2^8 as they are
 // Log2 units that every stored bias is raised by.  The softmax does not see it, but rows of logits
-// about 0 then pass the first tile's test for 0 as their reference (LSTEP_MIN; mean P of a lane's keys
-// 2^-4 to 2^6 without it) and their P still reach 1.
+// about 0 then pass the first tile's test for 0 as their reference (LSTEP_MIN) and their P still reach
+// 1: a mean P of a lane's keys between 2^-4 and 2^8 (without the shift) is accepted.  The middle of the
+// range that fp16 leaves: over random blocks at most 3 % of the tiles take the third MFMA, with 2
+// 0 - 37 %, with 6 0 - 28 %, and with 4 but LSTEP_MAX = 2^14 0 - 27 %.
 constexpr float REF_SHIFT = 4.f;
 
 typedef op_t opx2 __attribute__((ext_vector_type(2)));
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(64 * TAP_WAVES, 1) void ta_proj_kernel(
 // op_t value (exact as an MFMA operand).  It starts at 0, which a head's first tile accepts when
 // every lane's row sum is at least LSTEP_MIN, and moves lazily: to the first tile's maximum when
 // 0 is not accepted, while a query has seen no unmasked key, or when a tile's row sum exceeds
-// 2^14 (some P above 2^9).  A P that would overflow op_t fails the same test before it reaches
+// LSTEP_MAX.  A P that would overflow op_t fails the same test before it reaches
 // the P.V MFMA, and the tile is then repacked from S' with the new reference.  (Against a third
 // MFMA in every tile and a reference that always moved at the first: N = 1024 1083 -> 1051 us a
 // launch, 4 x N = 256 108 -> 105 us.)  A wave's two key halves of a step are processed
@@ -380,7 +382,8 @@ constexpr int TS_K = 65536, TK_STAGE = 16384;
 constexpr int TS_V = 98304, TV_STAGE = 16384;
 constexpr int TS_MASK = 131072, TM_STAGE = 1024;
 constexpr size_t TA_LDS = (size_t)TS_MASK + 2 * TM_STAGE;
-constexpr float LSTEP_MAX = 16384.f;   // per-lane row sum of one tile that forces a rescale
+// A lane's row sum (16 keys) of one tile that forces a rescale: every P is then still finite in fp16.
+constexpr float LSTEP_MAX = 61440.f;
 // A lane's row sum (16 keys) of a head's first tile from which on 0 serves as the reference: one of
 // its P is then at least 1, what the first tile's maximum as the reference would give, so the smaller
 // P keep as many bits in op_t.
@@ -576,9 +579,9 @@ __global__ __launch_bounds__(64 * TA_WAVES, 1) void ta_attn_kernel(
   };
   // One step (stage STG) of a live row: the block's two 32x32 tiles (key halves u) one after the
   // other: scores (bias as the accumulator start, K.Q^T, the mask / reference fold), the softmax
-  // against the current reference, one check, and the two P.V MFMAs.  When the check fails (no
-  // reference yet -- every head's first tile -- or a tile row sum above LSTEP_MAX) the reference
-  // moves to the tile's maximum first; the next tile's scores already use the new reference.
+  // against the current reference, one check, and the two P.V MFMAs.  When the check fails (a query
+  // without a reference -- a head's first tile -- that does not accept 0, or a tile row sum above
+  // LSTEP_MAX) the reference moves to the tile's maximum first; the next tile's scores already use the new reference.
   auto step2 = [&](auto stg, int kb0) PF_INLINE {
     constexpr int STG = decltype(stg)::value;
 #pragma unroll
