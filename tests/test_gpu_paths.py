@@ -133,6 +133,49 @@ def test_triatt_direct(gpu, B, N, ending, plain):
     assert (inplace - (zd + update)).abs().max() <= 2.0 ** -22 * (zd.abs().max() + update.abs().max())
 
 
+@pytest.mark.parametrize("B,N", [(1, 192), (3, 192)])
+@pytest.mark.parametrize("ending", [False, True])
+def test_triatt_c64_groups(gpu, B, N, ending):
+    """c_z = 64 with several groups of 64 positions per workgroup and an uneven last round (576 and 1728
+    groups on 256 CUs), padded keys, out of place and in place."""
+    from tt_boltz_amd import synthetic
+    prefix = "tri_att_end" if ending else "tri_att_start"
+    w = ref.sub(synthetic.draw({k: v for k, v in synthetic.layer_shapes(64, transform_s=False).items()
+                                if k.startswith(prefix + ".")}, 6), prefix)
+    mod = pairformer.TriangleAttention(32, 4, ending, {(k[4:] if k.startswith("mha.") else k): v for k, v in w.items()})
+    g = torch.Generator().manual_seed(N + B)
+    n = N - 9
+    z, pm = torch.zeros((B, N, N, 64)), torch.zeros((B, N, N))
+    z[:, :n, :n] = torch.randn((B, n, n, 64), generator=g)
+    pm[:, :n, :n] = (torch.rand((B, n, n), generator=g) > 0.1).float()
+    want = ref.triangle_attention(z[:, :n, :n].to(gpu), pm[:, :n, :n].to(gpu), {k: v.to(gpu) for k, v in w.items()},
+                                  not ending)
+    zd, pd = z.to(gpu), pm.to(gpu)
+    update = mod(zd, pd, n_valid=n)
+    check("triatt c64 update", update[:, :n, :n], want)
+    inplace = zd.clone()
+    mod(inplace, pd, out=inplace, accumulate=True, n_valid=n)
+    # the same update added to z: one fp32 rounding of the sum apart
+    assert (inplace - (zd + update)).abs().max() <= 2.0 ** -22 * (zd.abs().max() + update.abs().max())
+
+
+def test_template_stack_groups(gpu):
+    """Two templates of 200 tokens through the c_z = 64 stack: eight groups per workgroup."""
+    from tt_boltz_amd import synthetic
+    N = 200
+    w = synthetic.stack_weights(2, 44, c_z=64, transform_s=False)
+    z = torch.randn((2, N, N, 64), generator=torch.Generator().manual_seed(45))
+    m = torch.ones((2, N))
+    m[0, 181:], m[1, 190:] = 0, 0
+    pm = m[:, :, None] * m[:, None, :]
+    want = torch.cat([ref.pairformer_stack(None, z[b:b + 1].to(gpu), None, pm[b:b + 1].to(gpu),
+                                           {k: v.to(gpu) for k, v in w.items()}, 2)[1] for b in range(2)])
+    mod = pairformer.PairformerModule(2, 32, 4, None, None, False)
+    mod.load_state_dict(w)
+    _, got = mod(None, z.to(gpu), pair_mask=pm.to(gpu))
+    check("template stack", got, want)
+
+
 # ------------------------------------------------------------------------------ boundary padding
 @pytest.mark.parametrize("N,n_pad", [(1, 64), (45, 64), (64, 64), (130, 192)])
 @pytest.mark.parametrize("form", ["plain", "transposed", "sliced", "offset", "expanded", "half", "grad"])

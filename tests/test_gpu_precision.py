@@ -5,9 +5,11 @@
   itself, which must give the result of the plain kernel on the doubled weight (an exact
   doubling in the operand type) up to fp32 summation order; accuracy by the recycling
   projection's agreement with fp32 to ~1e-6 (both sides split).
-* the mean correction of the trimul's LN_in-side weights: on a pair tensor whose rows share a
-  strong channel pattern, the per-channel mean over positions of the GPU's update error (the
-  coherent part that a deep stack accumulates) must fall well below the uncorrected kernel's.
+* the projections' residuals, as a second MFMA (small grids) and through the mean correction: wiring
+  the same way, and against the correction added to the offsets by the host.
+* what they are for: on a pair tensor whose rows share a strong channel pattern, the per-channel mean
+  over positions of the trimul's update error (the coherent part that a deep stack accumulates) must
+  fall well below the uncorrected kernel's.
 """
 import pytest
 import torch
@@ -20,13 +22,13 @@ from test_gpu_parity import _dev_w, _inputs, _sub_w, check, stats
 pytestmark = pytest.mark.gpu
 
 
-def _same(a, b, name, mean_tol=2e-6):
+def _same(a, b, name, mean_tol=2e-6, max_tol=2e-3):
     """Equal up to fp32 summation order: hi.x + lo.x and (2 hi).x differ in the last bits of an
     fp32 sum, which now and then moves a later 16-bit rounding by one step (max ~1e-4 of the
     rms); a wiring mistake (wrong row, pitch or operand) moves every element by O(1)."""
     mx, mn = stats(a, b)
     print(f"[precision] {name}: max/rms={mx:.3e} mean/rms={mn:.3e}", flush=True)
-    assert torch.isfinite(a).all() and mx <= 2e-3 and mn <= mean_tol, f"{name}: max/rms={mx:.3e} mean/rms={mn:.3e}"
+    assert torch.isfinite(a).all() and mx <= max_tol and mn <= mean_tol, f"{name}: max/rms={mx:.3e} mean/rms={mn:.3e}"
 
 
 @pytest.mark.parametrize("ending", [False, True])
@@ -105,16 +107,17 @@ def test_pair_recycling_projection_is_fp32_accurate(gpu):
         assert pmn > 100 * mn
 
 
+@pytest.mark.parametrize("N", [256, 320])   # 256: the residuals as a second MFMA; 320: the mean correction
 @pytest.mark.parametrize("direction", [0, 1])
-def test_trimul_mean_correction_removes_coherent_error(gpu, direction):
+def test_trimul_mean_correction_removes_coherent_error(gpu, direction, N):
     """z rows share a strong channel pattern (so the normalized rows have a large mean over
     positions).  The error of the 16-bit weights then has a large coherent part: the same
-    offset at every position.  With the exact beta offsets and the mean correction, the
+    offset at every position.  With the exact beta offsets and the weights' residuals (multiplied
+    by as they are up to N = 256 on 256 CUs, else through the mean correction), the
     per-channel mean over positions of the update's error must drop well below the plain
     kernel's, and the update must stay within the parity bar.  (The corrected run also carries
     p_out as hi + lo, as the module does: the contraction output's LayerNorm has a mean over
     positions too.)"""
-    N = 256
     prefix = "tri_mul_out" if direction == 0 else "tri_mul_in"
     raw = _sub_w(25, prefix)
     g = torch.Generator().manual_seed(26)
@@ -139,9 +142,135 @@ def test_trimul_mean_correction_removes_coherent_error(gpu, direction):
     coh_plain = ((a.cpu() - want).mean(dim=(0, 1, 2)).abs().mean() / rms).item()
     coh_fixed = ((b.cpu() - want).mean(dim=(0, 1, 2)).abs().mean() / rms).item()
     print(f"[precision] trimul direction={direction}: coherent error plain {coh_plain:.3e}, "
-          f"mean-corrected {coh_fixed:.3e}", flush=True)
-    check(f"trimul mean-corrected direction={direction}", b, want)
+          f"corrected {coh_fixed:.3e} (N={N})", flush=True)
+    check(f"trimul corrected direction={direction} N={N}", b, want)
     assert coh_fixed < 0.35 * coh_plain
+
+
+def _sample_mean(z):
+    """The mean over the sampled positions of the rows of z [1, N, N, 128] normalized without affine part."""
+    ntiles = z.shape[1] ** 2 // 32
+    tiles = range(ntiles) if ntiles <= 1024 else [k * 2654435761 % ntiles for k in range(1024)]
+    rows = z.double().reshape(-1, 32, 128)[list(tiles)].reshape(-1, 128)
+    xhat = (rows - rows.mean(1, keepdim=True)) / (rows.var(1, unbiased=False, keepdim=True) + 1e-5).sqrt()
+    return xhat.mean(0)
+
+
+# Bounds where the two sides differ in the last fp32 bits ahead of several 16-bit roundings.  An fp32 sum
+# of 128 products moves by about 2^-22, which flips a rounding to 11 bits in 2^-10 to 2^-9 of the values,
+# by 2^-11 of their size.  Mean: 2^-20 a rounding, four of them on the way (4e-6); a query's logits see 32
+# q values, so 32 * 2^-9 * 2^-11 = 2^-15 for the attention.  Largest: one step of a value of 4 rms is
+# 2^-8 of the rms, and an output may see two.
+TM_STEPS = {"mean_tol": 4e-6, "max_tol": 2.0 ** -7}
+TA_STEPS = {"mean_tol": 2.0 ** -15, "max_tol": 2.0 ** -7}
+
+
+def _patterned(N, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(128, generator=g) + torch.randn((1, N, N, 128), generator=g), g
+
+
+@pytest.mark.parametrize("N", [64, 192, 256])   # one group of 64 positions per workgroup and several
+@pytest.mark.parametrize("direction", [0, 1])
+def test_trimul_residual_mfma_wiring(gpu, N, direction):
+    """p_in, g_in and g_out with residuals equal to the 16-bit weights (and p_out with zeros, which
+    selects the residual MFMA) equal the plain kernel on the doubled weights."""
+    w = _dev_w(_sub_w(51, "tri_mul_out" if direction == 0 else "tri_mul_in"), gpu)
+    z, g = _patterned(N, 52)
+    zd = z.to(gpu)
+    w["in_offsets"] = (0.3 * torch.randn(640, generator=g)).to(gpu)
+    w["p_out.weight.lo"] = torch.zeros_like(w["p_out.weight"])
+    keys = ("p_in.weight", "g_in.weight", "g_out.weight")
+    lo, doubled = dict(w), dict(w)
+    for k in keys:
+        lo[k + ".lo"] = w[k]
+        doubled[k] = 2 * w[k]
+    a, b = torch.empty_like(zd), torch.empty_like(zd)
+    ws = ops.workspace(ops.trimul_workspace_bytes(1, N), gpu)
+    ops.launch_trimul(zd, a, None, lo, direction, ws, accumulate=False)
+    ops.launch_trimul(zd, b, None, doubled, direction, ws, accumulate=False)
+    _same(a, b, f"trimul residual MFMA(=hi) vs doubled N={N} direction={direction}", **TM_STEPS)
+
+
+@pytest.mark.parametrize("N", [128, 320])   # the mean over all positions, over sampled ones
+@pytest.mark.parametrize("direction", [0, 1])
+def test_trimul_mean_correction_wiring(gpu, N, direction):
+    """Large residuals of p_in, g_in and g_out through the mean correction (no residual of p_out, so it
+    is taken at every N) equal their product with gamma * mu added to the offsets by the host."""
+    raw = _sub_w(53, "tri_mul_out" if direction == 0 else "tri_mul_in")
+    w = _dev_w(raw, gpu)
+    z, g = _patterned(N, 54)
+    zd = z.to(gpu)
+    mu = raw["norm_in.weight"].double() * _sample_mean(z)
+    off = 0.3 * torch.randn(640, generator=g)
+    lo, host = dict(w), dict(w)
+    lo["in_offsets"] = off.to(gpu)
+    add = []
+    for k in ("p_in.weight", "g_in.weight", "g_out.weight"):
+        r = (0.05 * torch.randn(raw[k].shape, generator=g)).to(w[k].dtype)
+        lo[k + ".lo"] = r.to(gpu)
+        add.append(r.double() @ mu)
+    host["in_offsets"] = (off.double() + torch.cat(add)).float().to(gpu)
+    a, b = torch.empty_like(zd), torch.empty_like(zd)
+    ws = ops.workspace(ops.trimul_workspace_bytes(1, N), gpu)
+    ops.launch_trimul(zd, a, None, lo, direction, ws, accumulate=False)
+    ops.launch_trimul(zd, b, None, host, direction, ws, accumulate=False)
+    _same(a, b, f"trimul mean correction vs offsets N={N} direction={direction}", **TM_STEPS)
+
+
+TA_KEYS = ("linear_q.weight", "linear_k.weight", "linear_v.weight", "linear.weight")
+
+
+def _triatt_pair(gpu, z, first, second, ending):
+    N = z.shape[1]
+    zd = z.to(gpu)
+    pm = torch.ones((1, N, N))
+    pm[:, :, N - 13:] = 0
+    ws = ops.workspace(ops.triatt_workspace_bytes(1, N), gpu)
+    out = []
+    for w in (first, second):
+        out.append(torch.empty_like(zd))
+        ops.launch_triatt(zd, out[-1], pm.to(gpu), w, ending, ws, accumulate=False, n_valid=N - 5)
+    return out
+
+
+@pytest.mark.parametrize("N", [64, 192, 256])
+@pytest.mark.parametrize("ending", [False, True])
+def test_triatt_residual_mfma_wiring(gpu, N, ending):
+    """q, k, v and the bias with residuals equal to the kernel's gamma-folded 16-bit weights (and those
+    of the gate and output zero, which selects the residual MFMA) equal the doubled weights."""
+    w = _dev_w(_sub_w(55, "tri_att_end" if ending else "tri_att_start"), gpu, "mha.")
+    z, g = _patterned(N, 56)
+    w["in_offsets"] = (0.3 * torch.randn(388, generator=g)).to(gpu)
+    for k in ("linear_g.weight", "linear_o.weight"):
+        w[k + ".lo"] = torch.zeros_like(w[k])
+    lo, doubled = dict(w), dict(w)
+    for k in TA_KEYS:
+        lo[k + ".lo"] = (w[k].float() * w["layer_norm.weight"]).to(w[k].dtype)
+        doubled[k] = 2 * w[k]
+    a, b = _triatt_pair(gpu, z, lo, doubled, ending)
+    _same(a, b, f"triatt residual MFMA(=hi) vs doubled N={N} ending={ending}", **TA_STEPS)
+
+
+@pytest.mark.parametrize("N", [128, 320])
+@pytest.mark.parametrize("ending", [False, True])
+def test_triatt_mean_correction_wiring(gpu, N, ending):
+    """Large residuals of q, k, v and the bias through the mean correction (none of the gate and output,
+    so it is taken at every N) equal their product with mu added to the offsets by the host."""
+    w = _dev_w(_sub_w(57, "tri_att_end" if ending else "tri_att_start"), gpu, "mha.")
+    z, g = _patterned(N, 58)
+    mu = _sample_mean(z)
+    off = 0.3 * torch.randn(388, generator=g)
+    lo, host = dict(w), dict(w)
+    lo["in_offsets"] = off.to(gpu)
+    add = []
+    for k in TA_KEYS:
+        r = (0.05 * torch.randn(w[k].shape, generator=g)).to(w[k].dtype)
+        lo[k + ".lo"] = r.to(gpu)
+        add.append(r.double() @ mu)
+    host["in_offsets"] = (off.double() + torch.cat(add)).float().to(gpu)
+    a, b = _triatt_pair(gpu, z, lo, host, ending)
+    _same(a, b, f"triatt mean correction vs offsets N={N} ending={ending}", **TA_STEPS)
 
 
 @pytest.mark.parametrize("N", [64, 128, 192, 256])
@@ -157,7 +286,7 @@ def test_pair_stats_sample_mean(gpu, N):
     g = torch.Generator().manual_seed(28)
     z = 2.0 * torch.randn(128, generator=g) + torch.randn((1, N, N, 128), generator=g)
     w = dict(_dev_w(raw, gpu))
-    w["in_offsets"] = torch.zeros(3 * 128, device=gpu)
+    w["in_offsets"] = torch.zeros(5 * 128, device=gpu)   # 256 rows of p_in, 256 of g_in, 128 of g_out
     for k in ("p_in.weight", "g_in.weight", "g_out.weight"):
         w[k + ".lo"] = ops.opw_lo(raw[k], gpu)
     zd = z.to(gpu).contiguous()
@@ -166,11 +295,7 @@ def test_pair_stats_sample_mean(gpu, N):
     torch.cuda.synchronize()
     start = 3 * 128 * N * N * 2 + 1024 * 4
     mu = ws[start:start + 64 * 128 * 4].cpu().view(torch.float32).view(64, 128).double().sum(0)
-    ntiles = N * N // 32
-    tiles = range(ntiles) if ntiles <= 1024 else [k * 2654435761 % ntiles for k in range(1024)]
-    rows = z.double().reshape(-1, 32, 128)[list(tiles)].reshape(-1, 128)
-    xhat = (rows - rows.mean(1, keepdim=True)) / (rows.var(1, unbiased=False, keepdim=True) + 1e-5).sqrt()
-    want = xhat.mean(0)
+    want = _sample_mean(z)
     err = (mu - want).abs().max().item()
     print(f"[precision] pair stats N={N}: |mu| max {want.abs().max().item():.3f}, max error {err:.2e}", flush=True)
     assert err < 1e-5
