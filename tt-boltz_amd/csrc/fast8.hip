@@ -778,8 +778,6 @@ Tm8Buffers tm8_buffers(void* ws, int B, int N) {
   return t;
 }
 
-// grid of a wave-tile loop: enough workgroups to fill the chip several times over
-
 }  // namespace
 
 // ---------------------------------------------------------------------------------

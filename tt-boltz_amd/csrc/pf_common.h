@@ -20,7 +20,7 @@
 // use this to feed an accumulator straight back in as the next MFMA's A/B operand:
 // accumulator regs 8*s .. 8*s+7 of a lane in half h hold rows
 //   16*s + 4*h + {0,1,2,3}  and  16*s + 8 + 4*h + {0,1,2,3}
-// so the partner operand is loaded with the same two 4-element runs (kperm_row()),
+// so the partner operand is loaded with the same two 4-element runs,
 // or the producer's rows are pre-permuted so the runs come out contiguous (perm16()).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -61,10 +61,6 @@ PF_DEV f32x16 zero16() {
 
 // Row of the 32x32 accumulator held by register r of a lane in half h.
 PF_DEV int acc_row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
-
-// k index carried by slot t (0..7) of a lane in half h for k-step s when the
-// operand comes from accumulator registers 8*s .. 8*s+7 (see header comment).
-PF_DEV int kperm_row(int s, int h, int t) { return 16 * s + 4 * h + (t < 4 ? t : t + 4); }
 
 // Involution on row indices swapping bits 2 and 3.  If a producer GEMM's weight row
 // rho holds output unit perm16(rho), accumulator regs 8*s+t of half h come out as
@@ -161,25 +157,6 @@ PF_DEV void ln_gamma_to_frag(const float (&x)[CC / 2], int h, const float* gamma
     }
   }
 }
-
-// (x - mean) * rstd of a CC-vector (load_row_frag order) as CC/16 MFMA fragments: the
-// LayerNorm without its affine part, for callers that fold gamma / beta into the weights.
-template <int CC>
-PF_DEV void ln_norm_to_frag(const float (&x)[CC / 2], float eps, opx8 (&f)[CC / 16]) {
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < CC / 2; ++i) s += x[i];
-  const float mean = xor32_sum(s) * (1.f / CC);
-  float v = 0.f;
-#pragma unroll
-  for (int i = 0; i < CC / 2; ++i) { const float d = x[i] - mean; v += d * d; }
-  const float rstd = rsqrtf(xor32_sum(v) * (1.f / CC) + eps);
-#pragma unroll
-  for (int s8 = 0; s8 < CC / 16; ++s8)
-#pragma unroll
-    for (int t = 0; t < 8; ++t) f[s8][t] = (op_t)((x[8 * s8 + t] - mean) * rstd);
-}
-PF_DEV void ln128_norm_to_frag(const float (&x)[64], float eps, opx8 (&f)[8]) { ln_norm_to_frag<128>(x, eps, f); }
 
 // LayerNorm of a CC-vector split over the two halves of a wave (CC/2 values per
 // lane, in load_row_frag order), written as CC/16 opx8 MFMA fragments.
@@ -596,7 +573,7 @@ namespace {
 //   pair_stats_kernel  mu of z (batch 0) from PS_TILES tiles of 32 consecutive positions spread
 //                      over the grid by Fibonacci hashing (every tile when there are fewer), as
 //                      PS_WG partial sums already divided by the sample size
-//   stats_mu           a workgroup sums the partials into mu (LDS) in its prologue
+//   stats_load / stats_reduce  a workgroup sums the partials into mu (LDS) in its prologue
 // ---------------------------------------------------------------------------------
 #ifndef PF_PS_TILES
 #define PF_PS_TILES 1024
@@ -680,27 +657,9 @@ __global__ __launch_bounds__(64 * PS_WAVES) void pair_stats_kernel(const float* 
   }
 }
 
-// mu[c] (LDS, 128 floats) = the sum of the PS_WG partials, with every thread of the workgroup
-// (blockDim.x a multiple of 128) summing a share into `scratch` (LDS, blockDim.x floats) first;
-// the caller synchronizes before reading mu.
-PF_DEV void stats_mu(const float* __restrict__ partials, float* mu, float* scratch) {
-  const int nq = blockDim.x / PS_C, c = threadIdx.x % PS_C, q = threadIdx.x / PS_C;
-  float sum = 0.f;
-#pragma unroll 4
-  for (int g = q; g < PS_WG; g += nq) sum += partials[g * PS_C + c];
-  scratch[threadIdx.x] = sum;
-  __syncthreads();
-  if (threadIdx.x < PS_C) {
-    float t = 0.f;
-    for (int j = 0; j < nq; ++j) t += scratch[j * PS_C + threadIdx.x];
-    mu[threadIdx.x] = t;
-  }
-}
-
 // Prologue helpers of the persistent pair kernels.  Every global load of a thread's share is
 // issued before the first use, so the set-up costs about one memory round trip instead of one
-// per (partly unrolled) loop step; the arithmetic and its order are those of stats_mu,
-// corrected_offset and a plain staging loop.
+// per (partly unrolled) loop step.
 template <int NT>
 constexpr int stats_per() { return PS_WG / (NT / PS_C); }
 // this thread's partials (channel threadIdx.x % 128, groups q, q + NT / 128, ...)
@@ -712,8 +671,7 @@ PF_DEV void stats_load(const float* __restrict__ partials, float (&v)[stats_per<
 #pragma unroll
   for (int i = 0; i < stats_per<NT>(); ++i) v[i] = partials[(q + i * nq) * PS_C + c];
 }
-// mu (LDS, 128 floats) from the loaded partials as stats_mu forms it; `scratch`: NT floats of
-// LDS.  Synchronizes once; the caller synchronizes again before reading mu.
+// mu (LDS, 128 floats) from the loaded partials; `scratch`: NT floats of LDS.  Synchronizes once; the caller synchronizes again before reading mu.
 template <int NT>
 PF_DEV void stats_reduce(const float (&v)[stats_per<NT>()], float* mu, float* scratch) {
   constexpr int nq = NT / PS_C;
@@ -727,32 +685,6 @@ PF_DEV void stats_reduce(const float (&v)[stats_per<NT>()], float* mu, float* sc
     for (int j = 0; j < nq; ++j) t += scratch[j * PS_C + threadIdx.x];
     mu[threadIdx.x] = t;
   }
-}
-// a 128-element op_t row in registers
-PF_DEV void load_row_x8(const op_t* __restrict__ row, opx8 (&v)[PS_C / 8]) {
-#pragma unroll
-  for (int c = 0; c < PS_C / 8; ++c) v[c] = ld_x8(row + 8 * c);
-}
-// corrected_offset with the residual row already in registers (has_lo false: no correction);
-// GAMMA false: no gamma factor (corrected_offset's gamma = nullptr: the product by 1 it takes is
-// exact).  The LDS reads of gamma and mu go in groups of four chunks, so they are not all hoisted
-// into registers at once.
-template <bool GAMMA>
-PF_DEV float corrected_offset_regs(float offb, const opx8 (&lo)[PS_C / 8], bool has_lo, const float* gamma,
-                                   const float* mu) {
-  float acc = offb;
-  if (has_lo) {
-#pragma unroll
-    for (int c = 0; c < PS_C / 8; ++c) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float l = (float)lo[c][e];
-        acc += (GAMMA ? l * gamma[8 * c + e] : l) * mu[8 * c + e];
-      }
-      if (c % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  return acc;
 }
 // [ROWS][COLS] op_t weights: this thread's 16-byte chunks (chunk threadIdx.x + NT i), loaded
 // all at once, then stored to LDS rows `pitch` elements apart (8-byte aligned rows: two 8-byte
@@ -780,22 +712,6 @@ PF_DEV void stage_store(op_t* dst, int pitch, const opx8 (&v)[stage_per<NT, ROWS
       *reinterpret_cast<opx4*>(d + 4) = opx4{v[i][4], v[i][5], v[i][6], v[i][7]};
     }
   }
-}
-
-// Offset of one output row: offb (the fp32 W . beta) plus, with the mean correction, the row of
-// the weight residual against gamma * mu (gamma, mu: 128 floats, LDS or global; gamma = nullptr
-// when the kernel folds gamma into its weights, whose residual then already carries it).
-PF_DEV float corrected_offset(float offb, const op_t* __restrict__ lo_row, const float* gamma, const float* mu) {
-  float acc = offb;
-  if (lo_row) {
-#pragma unroll 4
-    for (int c = 0; c < PS_C; c += 8) {
-      const opx8 l8 = ld_x8(lo_row + c);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc += (float)l8[e] * (gamma ? gamma[c + e] : 1.f) * mu[c + e];
-    }
-  }
-  return acc;
 }
 
 }  // namespace

@@ -23,7 +23,7 @@
 
 namespace {
 
-constexpr int C = 128, LDSW = 136, LDS3 = 40;
+constexpr int C = 128, LDSW = 136;
 PF_DEV opx8 lds_x8(const char* p) { return *reinterpret_cast<const opx8*>(p); }
 
 // Pair transition: a workgroup is TRW waves x 32 pairs; three workgroups share a CU.

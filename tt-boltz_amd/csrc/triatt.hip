@@ -30,7 +30,7 @@ namespace {
 
 // C = H * D: the attention width (q / k / v / o channels).  The pair width c_z (CC in the
 // projection kernels) is 128 in the trunk and 64 in the template stack.
-constexpr int C = 128, H = 4, D = 32, LDSW = 136;
+constexpr int C = 128, H = 4, D = 32;
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float RESCALE_SLACK = 8.f;   // log2 units: a rescale leaves queries whose P stay <= 2^8 as they are
 // Log2 units that every stored bias is raised by.  The softmax does not see it, but rows of logits
@@ -178,7 +178,8 @@ __global__ __launch_bounds__(64 * TAP_WAVES, 1) void ta_proj_kernel(
     w.turn(stg, lane);
   __builtin_amdgcn_sched_barrier(0);
   // (the residuals' own round trip runs beside the LayerNorm: with everything in flight at once
-  // the set-up spilled)
+  // the set-up spilled.  DL_MFMA, whose residuals stay in registers, keeps 5 registers of loop-
+  // invariant addresses in scratch: 24 bytes a lane, each read once a group)
   if constexpr (LO != DL_NONE) wl.load(mf.lo[kind] + r0, lane);
   if (wid < TAP_LN) ln.store(sx, eps, wid, lane);
   if (!exact) c0 = direct_wbeta<KS, f32x4>(w.v, sgb + CC, h);
@@ -394,15 +395,9 @@ constexpr float LSTEP_MIN = 16.f;
 // 16-byte bank groups.
 PF_DEV int swz8(int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); }
 PF_DEV int swz4(int r) { return (r >> 2) & 3; }
-PF_DEV opx8 lds_x8(const char* p) { return *reinterpret_cast<const opx8*>(p); }
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 PF_DEV uint32_t half_bits(op_t v) { return __builtin_bit_cast(uint16_t, v); }
 PF_DEV opx8 as_x8(const u32x4& v) { return __builtin_bit_cast(opx8, v); }
-// operand whose slots 0 and 1 are (lo, hi) in lanes 0..31 and zero elsewhere
-PF_DEV opx8 slots01(int h, uint32_t lo_hi) {
-  const u32x4 v = {h ? 0u : lo_hi, 0u, 0u, 0u};
-  return as_x8(v);
-}
 // LDS reads from absolute LDS byte addresses (the per-lane address registers already hold the
 // allocation base, so the loop's reads need no address arithmetic beyond the immediate offset)
 typedef __attribute__((address_space(3))) const char* lds_ptr;

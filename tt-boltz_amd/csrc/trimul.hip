@@ -24,32 +24,14 @@ namespace {
 
 constexpr int C = 128;        // c_z
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr int LDSW = 136;     // padded LDS row stride (elements) for [rows][128] tiles
-
-// A [32][128] op_t block moved by 256 threads: 512 chunks of 16 B, 2 per thread.
-struct Blk32 { opx8 v[2]; };
-PF_DEV void blk32_load(const op_t* __restrict__ src, int tid, Blk32& r) {
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int c = tid + 256 * q;
-    r.v[q] = ld_x8(src + (c >> 4) * C + (c & 15) * 8);
-  }
-}
-PF_DEV void blk32_store(op_t* lds, int tid, const Blk32& r) {
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int c = tid + 256 * q;
-    st_x8(lds + (c >> 4) * LDSW + (c & 15) * 8, r.v[q]);
-  }
-}
 
 // ---------------------------------------------------------------------------------
 // Input projection of large grids at c_z = 64 (the others: tm_proj_direct_kernel).  Persistent:
-// one workgroup (8 waves, two per SIMD) per CU keeps p_in and g_in ([2 CC][CC] each, op_t as given, so rounded once) resident in LDS, with the LayerNorm's
-// beta folded into fp32 offsets W beta added in the epilogue (gamma scales the normalized z
-// before its rounding to op_t).  Every wave walks tiles of 32
-// consecutive positions of one operand-plane row (orow, ocol0 .. ocol0+31) and loads the next
-// tile's z rows while it computes the current one.  The projection is formed as
+// one workgroup (8 waves, two per SIMD) per CU keeps p_in and g_in ([2 CC][CC] each, op_t as
+// given, so rounded once) resident in LDS, with the LayerNorm's beta folded into fp32 offsets
+// W beta added in the epilogue (gamma scales the normalized z before its rounding to op_t).
+// Every wave walks tiles of 32 consecutive positions of one operand-plane row (orow, ocol0 ..
+// ocol0+31) and loads the next tile's z rows while it computes the current one.  The projection is formed as
 // D[position][channel]; each 32x32 output block goes through a per-wave LDS stage so that it
 // leaves as 16-byte stores, four lanes per 64-byte plane-row segment (a full segment per
 // instruction writes faster than register-permuted 32-byte halves).  The channel-block loop is
@@ -58,25 +40,22 @@ PF_DEV void blk32_store(op_t* lds, int tid, const Blk32& r) {
 // ---------------------------------------------------------------------------------
 constexpr int TMP_WAVES = 8;
 constexpr int SPITCH = 40;     // output staging pitch (elements): one 32-position row + 16 B
-template <int CC>
-constexpr int tmp_waves() { return TMP_WAVES; }
-// CC = c_z (64 or 128).  LDS: gamma [CC] and the offsets W_p beta [2 CC], -log2(e) W_g beta
+// The persistent kernels' c_z.
+constexpr int C64 = 64;
+// LDS: gamma [CC] and the offsets W_p beta [2 CC], -log2(e) W_g beta
 // [2 CC] (fp32, first: small immediate offsets), then W_p, W_g [2 CC][CC + 8] op_t, the per-wave
 // output stages and the per-wave maxima.
-template <int CC>
-constexpr size_t tmp_lds() {
-  return 5 * CC * sizeof(float) + (size_t)2 * 2 * CC * (CC + 8) * sizeof(op_t) +
-         (size_t)TMP_WAVES * 32 * SPITCH * sizeof(op_t) + TMP_WAVES * sizeof(float);
-}
+constexpr size_t TMP_LDS = 5 * C64 * sizeof(float) + (size_t)2 * 2 * C64 * (C64 + 8) * sizeof(op_t) +
+                           (size_t)TMP_WAVES * 32 * SPITCH * sizeof(op_t) + TMP_WAVES * sizeof(float);
 
-template <int CC, bool MASK>
+template <bool MASK>
 __global__ __launch_bounds__(64 * TMP_WAVES, 1) void tm_proj_kernel(
     const float* __restrict__ z, const float* __restrict__ mask,
     const float* __restrict__ lnw, const float* __restrict__ lnb,
     const op_t* __restrict__ w_p, const op_t* __restrict__ w_g,
     op_t* __restrict__ opA, op_t* __restrict__ opB, float* __restrict__ amax_parts, int B, int N, int incoming,
     float eps) {
-  constexpr int LW = CC + 8, KS = CC / 16;
+  constexpr int CC = C64, LW = CC + 8, KS = CC / 16;
   extern __shared__ __attribute__((aligned(16))) op_t wlds[];
   float* gam = reinterpret_cast<float*>(wlds);
   float* cbias = gam + CC;   // [0, 2 CC): W_p beta, [2 CC, 4 CC): -log2(e) W_g beta
@@ -615,22 +594,19 @@ __global__ __launch_bounds__(64 * TMD_WAVES, 1) void tm_contract_dma_kernel(
 constexpr int TMO_WAVES = 8, XSP = 40;   // per-wave X stage: [CC channels][32 pairs + 8]
 // LDS: the offsets W_p beta_out [CC], -log2(e) W_g beta_in [CC] and gamma_out [CC], gamma_in [CC]
 // (fp32, first: small immediate offsets), then W_p, W_g [CC][CC + 4] op_t, then the per-wave X stages
-template <int CC>
-constexpr size_t tmo_lds() {
-  return 4 * CC * sizeof(float) + (size_t)2 * CC * (CC + 4) * sizeof(op_t) + (size_t)TMO_WAVES * CC * XSP * sizeof(op_t);
-}
+constexpr size_t TMO_LDS = 4 * C64 * sizeof(float) + (size_t)2 * C64 * (C64 + 4) * sizeof(op_t) +
+                           (size_t)TMO_WAVES * C64 * XSP * sizeof(op_t);
 
 // resid: 0 -> out = update; 1 -> out = z_in + update (out may alias z_in); 2 -> out += update
 // X is read back divided by the contraction's x_store_scale of the operand maxima in amax_parts
 // (contraction length N).
-template <typename XT, int CC>
 __global__ __launch_bounds__(64 * TMO_WAVES, 1) void tm_out_kernel(
-    const XT* __restrict__ X, const float* __restrict__ amax_parts, int nparts,
+    const op_t* __restrict__ X, const float* __restrict__ amax_parts, int nparts,
     const float* z_in, float* out,
     const float* __restrict__ lni_w, const float* __restrict__ lni_b,
     const float* __restrict__ lno_w, const float* __restrict__ lno_b,
     const op_t* __restrict__ w_pout, const op_t* __restrict__ w_gout, int B, int N, int resid, float eps) {
-  constexpr int LW = CC + 4, KS = CC / 16;
+  constexpr int CC = C64, LW = CC + 4, KS = CC / 16;
   extern __shared__ __attribute__((aligned(16))) op_t olds[];
   float* cbias = reinterpret_cast<float*>(olds);   // [0, CC): p, [CC, 2 CC): g
   float* gam_o = cbias + 2 * CC;
@@ -639,7 +615,7 @@ __global__ __launch_bounds__(64 * TMO_WAVES, 1) void tm_out_kernel(
   op_t* sWg = sWp + CC * LW;
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, m = lane & 31;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  XT* xs = reinterpret_cast<XT*>(sWg + CC * LW) + wid * CC * XSP;   // this wave's X stage
+  op_t* xs = sWg + CC * LW + wid * CC * XSP;   // this wave's X stage
   // weights -> LDS (rows are 8-byte aligned: two 8-byte stores per 16-byte load), gamma, and
   // the offsets W beta (one row per thread)
   constexpr int NT = 64 * TMO_WAVES;
@@ -684,12 +660,12 @@ __global__ __launch_bounds__(64 * TMO_WAVES, 1) void tm_out_kernel(
     {
       // X[b][ch][q0 .. q0+31]: 16-byte chunk c -> channel c >> 2, pairs 8*(c & 3) ..  (a wave's
       // LDS accesses complete in order)
-      const XT* src = X + (long)b * CC * NN + (p0 - (long)b * NN);
+      const op_t* src = X + (long)b * CC * NN + (p0 - (long)b * NN);
       float xv[CC / 2];
 #pragma unroll
       for (int k = 0; k < CC / 16; ++k) {
         const int c = lane + 64 * k, ch = c >> 2, col = (c & 3) * 8;
-        *reinterpret_cast<opx8*>(xs + ch * XSP + col) = *reinterpret_cast<const opx8*>(src + (long)ch * NN + col);
+        st_x8(xs + ch * XSP + col, ld_x8(src + (long)ch * NN + col));
       }
 #pragma unroll
       for (int q = 0; q < CC / 8; ++q)
@@ -945,16 +921,16 @@ int trimul_run_direct(const pf_trimul_args* a, op_t* opA, op_t* opB, op_t* X, fl
 
 // The persistent kernels (c_z = 64).
 int trimul_run_persistent64(const pf_trimul_args* a, op_t* opA, op_t* opB, op_t* X, float* amax_parts, int cus) {
-  constexpr int CC = 64;
+  constexpr int CC = C64;
   hipStream_t st = (hipStream_t)a->stream;
   const int B = a->B, N = a->N;
   const long positions = (long)B * N * N;
   const int grid_proj = (int)min((long)min(cus, TM_MAX_PARTS), (positions / 32 + TMP_WAVES - 1) / TMP_WAVES);
   const int grid_out = (int)min((long)cus, (positions / 32 + TMO_WAVES - 1) / TMO_WAVES);
   {
-    auto kern = a->pair_mask ? tm_proj_kernel<CC, true> : tm_proj_kernel<CC, false>;
-    if (const int rc = pf_reserve_lds((const void*)kern, tmp_lds<CC>(), "tm_proj_kernel")) return rc;
-    kern<<<grid_proj, 64 * tmp_waves<CC>(), tmp_lds<CC>(), st>>>(
+    auto kern = a->pair_mask ? tm_proj_kernel<true> : tm_proj_kernel<false>;
+    if (const int rc = pf_reserve_lds((const void*)kern, TMP_LDS, "tm_proj_kernel")) return rc;
+    kern<<<grid_proj, 64 * TMP_WAVES, TMP_LDS, st>>>(
         a->z_in, a->pair_mask, a->norm_in_w, a->norm_in_b, (const op_t*)a->p_in_w, (const op_t*)a->g_in_w, opA, opB,
         amax_parts, B, N, a->direction, a->eps);
     PF_CHECK_LAUNCH("tm_proj_kernel");
@@ -964,8 +940,8 @@ int trimul_run_persistent64(const pf_trimul_args* a, op_t* opA, op_t* opB, op_t*
   pf_kernel_mark(PF_TIMED_CONTRACT, st, 1);
   if (rc != PF_OK) return rc;
   const int resid = !a->accumulate ? 0 : (a->out == a->z_in ? 1 : 2);
-  if (const int rc2 = pf_reserve_lds((const void*)tm_out_kernel<op_t, CC>, tmo_lds<CC>(), "tm_out_kernel")) return rc2;
-  tm_out_kernel<op_t, CC><<<grid_out, 64 * TMO_WAVES, tmo_lds<CC>(), st>>>(
+  if (const int rc2 = pf_reserve_lds((const void*)tm_out_kernel, TMO_LDS, "tm_out_kernel")) return rc2;
+  tm_out_kernel<<<grid_out, 64 * TMO_WAVES, TMO_LDS, st>>>(
       X, amax_parts, grid_proj, a->z_in, a->out, a->norm_in_w, a->norm_in_b, a->norm_out_w, a->norm_out_b,
       (const op_t*)a->p_out_w, (const op_t*)a->g_out_w, B, N, resid, a->eps);
   PF_CHECK_LAUNCH("tm_out_kernel");
