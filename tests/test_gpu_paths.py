@@ -350,6 +350,20 @@ def test_transition_direct(gpu, rows, hidden, mode):
     assert torch.equal(out[rows:], keep)
 
 
+@pytest.mark.parametrize("N,mean_fix", [(320, False), (384, True)])
+def test_transition_residual_line(gpu, N, mean_fix):
+    """The module takes the fc3 residual as hi + lo up to 400 pairs per CU (102400 on 256 CUs) and
+    through the mean correction above."""
+    mod = pairformer.Transition(_sub_w(13, "transition_z"))
+    z = torch.randn((1, N, N, 128), generator=torch.Generator().manual_seed(N)).to(gpu)
+    want = torch.empty_like(z)
+    ws = ops.workspace(mod.workspace_bytes(N * N), gpu)
+    ops.launch_transition(z, want, mod.w, ws, False, fc3_mean_fix=mean_fix)
+    other = torch.empty_like(z)
+    ops.launch_transition(z, other, mod.w, ws, False, fc3_mean_fix=not mean_fix)
+    assert torch.equal(mod(z), want) and not torch.equal(want, other)
+
+
 @pytest.mark.parametrize("B,N", [(1, 64), (2, 96), (1, 352)])
 def test_transition_direct_pair_bias(gpu, B, N):
     """The pair bias of the updated rows from the same kernel against the bias kernel on them (odd

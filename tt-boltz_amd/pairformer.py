@@ -293,8 +293,9 @@ class TriangleAttention(Module):
 class Transition(Module):
     """``tenstorrent.py:856-946`` / ``boltz2.py:1188-1258``."""
 
-    #: pairs up to which the fc3 residual enters as a second MFMA instead of the mean correction
-    HILO_ROWS = 320 * 320
+    #: pairs per CU up to which the fc3 residual enters as a second MFMA instead of the mean correction
+    #: (N = 320 on 256 CUs)
+    HILO_ROWS_PER_CU = 400
 
     def __init__(self, state_dict, options: Optional[Options] = None, allow_fast: bool = True):
         super().__init__(state_dict, options)
@@ -304,6 +305,7 @@ class Transition(Module):
         # fast mode covers the Pairformer's pair transition (c_z = 128); the single-track
         # one and those outside the Pairformer (allow_fast=False) stay 16-bit
         self.fast = self.fast and allow_fast and self.C == C_Z
+        self.hilo_rows = self.HILO_ROWS_PER_CU * torch.cuda.get_device_properties(self.device).multi_processor_count
         if self.fast:
             self.w.update(ops.mx8_weights(self.weights, self.device, ops.TRANSITION_MX8_KEYS, self.variant))
         else:
@@ -338,10 +340,12 @@ class Transition(Module):
         if ws is None:
             nb = self.workspace_bytes(rows)
             ws = ops.workspace(nb, x.device) if nb else None
-        # the sampled mean is one batch element's: batch 1 only (otherwise hi + lo).  On small grids
-        # hi + lo is faster than the sampling pass (N = 128 30 vs 45 us, 320 87 vs 94, 384 114 vs 112)
+        # the sampled mean is one batch element's: batch 1 only (otherwise hi + lo).  hi + lo takes the
+        # whole residual and is also faster than the sampling pass and the register-weight kernel up to
+        # four groups of 64 pairs per CU (N = 128 23 vs 35 us, 256 50 vs 57); its exactness is kept
+        # where it costs up to a tenth (288 71 vs 70, 320 85 vs 77), not beyond (384 112 vs 95)
         mean_fix = (self.options.mean_correction and "fc3.weight.lo" in self.w and x.dim() == 4 and x.shape[0] == 1
-                    and rows > self.HILO_ROWS)
+                    and rows > self.hilo_rows)
         ops.launch_transition(x, out, self.w, ws, accumulate, self.options.eps, self.variant, pb, mean_fix)
         return out
 
