@@ -14,7 +14,7 @@ struct PadShape {
 
 // dst [B][n1p][M][n2p][C] = src[b, i, m, j, c] for i < N1 and j < N2, else 0; src null: 1.  One pass
 // that writes every element once (a fill and a strided copy write the valid part twice: z at
-// N = 413 45 us, this 28; at N = 1024, where nothing is padded, 288 us against 214), four units a
+// N = 413 41 us, this 28; at N = 1024, where nothing is padded, 285 us against 178), four units a
 // thread with their loads in flight, every store instruction of a wave contiguous.
 template <int VEC>
 __global__ __launch_bounds__(256) void pad_kernel(const float* __restrict__ src, float* __restrict__ dst, PadShape p) {

@@ -121,22 +121,22 @@ class Options:
     overlapped single track (it then starts beside the following ones).  The default 1 keeps it
     off the outgoing triangle multiplication, whose contraction it slows the most (N = 512:
     1.254 vs 1.263 ms per layer with 0; 1.269 with 2, 1.308 with 4).
-    ``weight_residuals``: the pair kernels whose weights fit twice in LDS (the triangle
-    attention's gate and output projection, the triangle multiplication's output projection,
-    the recycling projection; the pair transition's output projection when the mean correction
-    is off or the batch is larger than one) take each 16-bit weight together with its rounding
+    ``weight_residuals``: the triangle attention's gate and output projection, the triangle
+    multiplication's output projection, the recycling projection and the pair transition's output
+    projection (on small grids, or when the mean correction is off or the batch is larger than
+    one) take each 16-bit weight together with its rounding
     residual and multiply by both (default on).  A 16-bit weight's rounding error is the same at
     every position, so it adds up coherently through a deep stack; with the residual the
     weights are good to ~2^-22 of their size.
-    ``mean_correction``: the weights after a LayerNorm whose LDS does not hold them twice (the
-    triangle multiplication's p_in, g_in, g_out; the triangle attention's q, k, v and bias
-    projections) get the exact W . beta offsets plus the mean correction
+    ``mean_correction``: the other weights after a LayerNorm (the triangle multiplication's p_in,
+    g_in, g_out; the triangle attention's q, k, v and bias projections) get the exact W . beta offsets plus the mean correction
     (W - W16) . (gamma * mu), mu the mean over positions of the normalized input, estimated per
     call from sampled positions: the part of their rounding error that every position shares.
     The pair transition's fc3 then takes its residual the same way, (W - W16) . mean(h) over the
     hidden activations of sampled positions, instead of as the hi + lo product (default on;
-    c_z = 128, batch 1).  On small grids (N <= 256), with ``weight_residuals`` also on, the triangle
-    operators multiply by these residuals as well instead, which is exact and faster there."""
+    c_z = 128, batch 1).  On small grids (N <= 256; fc3 N <= 320, on 256 CUs), with
+    ``weight_residuals`` also on, the kernels multiply by these residuals as well instead, which is
+    exact and (but for fc3 above 256) faster there."""
 
     def __init__(self, eps: float = 1e-5, operand: str = ops.DEFAULT_VARIANT, overlap_single: bool = True,
                  single_delay: int = 1, weight_residuals: bool = True, mean_correction: bool = True):
