@@ -464,6 +464,7 @@ def summarize_probe(N: int, kt_dir: str, pmc_dirs) -> None:
     (``pmc_dirs``), each written with ``--output-format csv -o run``."""
     import collections
     import csv
+    from statistics import median
     mean = lambda xs: sum(xs) / len(xs) if xs else float("nan")
     dur = collections.defaultdict(list)
     for r in csv.DictReader(open(os.path.join(kt_dir, "run_kernel_trace.csv"))):
@@ -478,7 +479,7 @@ def summarize_probe(N: int, kt_dir: str, pmc_dirs) -> None:
     copy = cnt["copy (torch.mul, calibration)"]
     f_fac = COPY_BYTES / (mean(copy["FETCH_SIZE"]) * 1024)
     w_fac = COPY_BYTES / (mean(copy["WRITE_SIZE"]) * 1024)
-    copy_us = mean([d for d in dur["copy (torch.mul, calibration)"] if d > 20])
+    copy_us = median([d for d in dur["copy (torch.mul, calibration)"] if d > 20])
     P = N * N
     alg = {"tm_proj_direct_kernel": P * 128 * 4 + 2 * P * 128 * 2,
            "tm_contract_dma_kernel": 3 * P * 128 * 2,
@@ -495,7 +496,7 @@ def summarize_probe(N: int, kt_dir: str, pmc_dirs) -> None:
         fe = mean(c["FETCH_SIZE"]) * 1024 * f_fac if c.get("FETCH_SIZE") else float("nan")
         wr = mean(c["WRITE_SIZE"]) * 1024 * w_fac if c.get("WRITE_SIZE") else float("nan")
         gr = mean(c["GRBM_GUI_ACTIVE"])
-        us = mean(d)
+        us = median(d)   # (a kernel's first dispatch loads its code: up to milliseconds)
         rows.append(dict(kernel=k, us=us, fetch=fe, write=wr, gbs=(fe + wr) / (us * 1e3), alg=alg.get(k),
                          mfma=mean(c["SQ_INSTS_MFMA"]) if c.get("SQ_INSTS_MFMA") else 0.0,
                          busy=mean(c["SQ_VALU_MFMA_BUSY_CYCLES"]) / (128 * gr) if c.get("SQ_VALU_MFMA_BUSY_CYCLES")
@@ -508,10 +509,11 @@ def summarize_probe(N: int, kt_dir: str, pmc_dirs) -> None:
     lines = [f"# Kernel durations, bench.py --probe-traffic at N={N} (MI355X, one GPU)", f"# command: {cmd_kt}",
              "# workload: the triangle-attention core x5 and the trimul contraction x5 on their real operands,",
              "# a 256 MiB copy x3 (calibration), then 3 full PairformerLayers (serial schedule, single track included)",
-             f"# {'kernel':34s} {'calls':>6s} {'avg_us':>9s} {'total_ms':>9s}"]
-    for k, d in sorted(dur.items(), key=lambda kv: -sum(kv[1])):
+             "# (a kernel's first dispatch loads its code and can take several times the others: the medians count)",
+             f"# {'kernel':34s} {'calls':>6s} {'median_us':>9s} {'avg_us':>9s}"]
+    for k, d in sorted(dur.items(), key=lambda kv: -median(kv[1]) * len(kv[1])):
         if not k.startswith(("distribution", "__amd", "reduce")):
-            lines.append(f"  {k:34s} {len(d):6d} {mean(d):9.1f} {sum(d) / 1e3:9.3f}")
+            lines.append(f"  {k:34s} {len(d):6d} {median(d):9.1f} {mean(d):9.1f}")
     open(os.path.join(ROOT, "profiles", f"layer_n{N}_kernel_stats.txt"), "w").write("\n".join(lines) + "\n")
     md = [f"# Per-kernel counters, N = {N} (MI355X, one GPU)", "",
           f"Workload: `bench.py --probe-traffic --n {N}` (attention core x5, trimul contraction x5, a 256 MiB copy x3 "
@@ -519,7 +521,7 @@ def summarize_probe(N: int, kt_dir: str, pmc_dirs) -> None:
           "trace; the tables are made by `bench.py --summarize-probe`):", "", f"    {cmd_kt}"]
     md += [f"    rocprofv3 --pmc {c} --output-format csv -d <dir> -o run -- python3 bench.py --probe-traffic --n {N}"
            for c in PROBE_PMC_PASSES]
-    md += ["", "Values are means per dispatch over every dispatch of the kernel in the run.",
+    md += ["", "Values are means per dispatch over every dispatch of the kernel in the run, times medians.",
            f"HBM bytes: `FETCH_SIZE` x {f_fac:.3f} and `WRITE_SIZE` x {w_fac:.3f} (KiB): the factors that make the "
            f"plain copy kernel's counters read its known 256 MiB in / 256 MiB out (the copy itself ran at "
            f"{2 * COPY_BYTES / (copy_us * 1e3):.0f} GB/s).",
