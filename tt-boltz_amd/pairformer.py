@@ -129,8 +129,8 @@ class Options:
     every position, so it adds up coherently through a deep stack; with the residual the
     weights are good to ~2^-22 of their size.
     ``mean_correction``: the other weights after a LayerNorm (the triangle multiplication's p_in,
-    g_in, g_out; the triangle attention's q, k, v and bias projections) get the exact W . beta offsets plus the mean correction
-    (W - W16) . (gamma * mu), mu the mean over positions of the normalized input, estimated per
+    g_in, g_out; the triangle attention's q, k, v and bias projections) get the exact W . beta
+    offsets plus the mean correction (W - W16) . (gamma * mu), mu the mean over positions of the normalized input, estimated per
     call from sampled positions: the part of their rounding error that every position shares.
     The pair transition's fc3 then takes its residual the same way, (W - W16) . mean(h) over the
     hidden activations of sampled positions, instead of as the hi + lo product (default on;
