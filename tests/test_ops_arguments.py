@@ -200,3 +200,26 @@ def test_msa_inputs_broadcast_emb(size):
 def test_msa_inputs_refuse_other_emb(size):
     with pytest.raises(RuntimeError):
         _msa_inputs(torch.ones(size))
+
+
+# ------------------------------------------------------------------------------ size-1 dimensions
+def test_size_one_dimensions_may_differ_where_nothing_is_padded(lib):
+    """At N = 64 the kernels read the caller's memory as it is: an unbatched z or k_in, a mask with
+    dimensions of size 1 between."""
+    N = 64
+    z, k_in, mask = torch.randn((N, N, 128)), torch.randn((1, 1, N, 384)), torch.ones((1, 1, 1, N))
+    _apb(1, N, k_in, z, mask)
+    a, z_n = _apb_args_of(lib)
+    assert z_n == N and torch.equal(lib.tensors[a.z], z[None])
+    assert torch.equal(lib.tensors[a.k_in], k_in[0]) and torch.equal(lib.tensors[a.mask], mask[0, 0])
+    lib.calls.clear()
+    _apb(2, N, mask=torch.arange(2.0 * N).view(2, 1, N))
+    a, _ = _apb_args_of(lib)
+    assert torch.equal(lib.tensors[a.mask], torch.arange(2.0 * N).view(2, N))
+
+
+def test_size_one_dimensions_where_padding_refuses_them(lib):
+    for z, mask in ((torch.zeros((50, 50, 128)), None), (None, torch.ones((2, 1, 50)))):
+        with pytest.raises((RuntimeError, ValueError)):
+            _apb(1 if z is not None else 2, 50, z=z, mask=mask)
+    assert not lib.calls

@@ -133,12 +133,14 @@ def _pads_on_device(x: torch.Tensor, device: torch.device) -> bool:
             and x.stride(-1) == 1)
 
 
-def shaped(t: torch.Tensor, shape: tuple) -> torch.Tensor:
+def shaped(t: torch.Tensor, shape: tuple, units: bool = False) -> torch.Tensor:
     """``t`` in the call's own ``shape``, broadcast to it as an assignment to a slice of that shape
     would (a view), RuntimeError where it does not fit: the kernels read a whole tensor of that shape
-    from the pointer."""
+    from the pointer.  ``units``: dimensions of size 1 may stand elsewhere."""
     if t.shape == shape:
         return t
+    if units and [n for n in t.shape if n != 1] == [n for n in shape if n != 1]:
+        return t.reshape(shape)
     while t.dim() > len(shape) and t.shape[0] == 1:
         t = t[0]
     return t.expand(shape)
@@ -703,17 +705,19 @@ def attention_pair_bias(s: torch.Tensor, z: torch.Tensor, mask: Optional[torch.T
     n_pad = padded_len(N)
 
     def pad_tokens(t):   # [B, N, c_s] -> [B, n_pad, c_s] fp32; read-only, so no copy when N needs no padding
-        t = shaped(t, (B, N, c_s))
+        t = shaped(t, (B, N, c_s), n_pad == N)
         if n_pad == N:
             return t.to(torch.float32).contiguous()
         return padded(t.to(torch.float32), n_pad, dev, (1,))
     sp = pad_tokens(s)
     kp = sp if k_in is s else pad_tokens(k_in)   # both are only read
-    z = shaped(z, (B,) + tuple(z.shape[1:3]) + (C_Z,)).to(torch.float32)
+    if z.dim() != 4 and n_pad != N:
+        raise ValueError(f"attention_pair_bias expects z [B, N, N, {C_Z}], got {tuple(z.shape)}")
+    z = shaped(z, (B, *z.shape[1:3], C_Z) if z.dim() == 4 else (B, N, N, C_Z), n_pad == N).to(torch.float32)
     # read unpadded where it has the tokens of s, else through a padded copy
     zp, z_n = (z.contiguous(), N) if tuple(z.shape[1:3]) == (N, N) else (pad_pair(z, n_pad), n_pad)
     if mask is not None:
-        mask = shaped(mask, (B, N)).to(device=dev, dtype=torch.float32)
+        mask = shaped(mask, (B, N), n_pad == N).to(device=dev, dtype=torch.float32)
         mp = mask.contiguous() if n_pad == N else padded(mask, n_pad, dev, (1,))
     else:
         mp = torch.zeros((B, n_pad), dtype=torch.float32, device=dev)
